@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "lib")
 LIB = os.path.join(OUT, "libmci_amd.so")
-SOURCES = ["mci_kernels.hip", "mci_fast.hip", "mci_batch.hip", "mci_mlp.hip", "mci_lp.hip", "mci_noalloc.hip", "mci_em.hip", "mci_api.cpp",
+SOURCES = ["mci_kernels.hip", "mci_fast.hip", "mci_fast_group.hip", "mci_batch.hip", "mci_mlp.hip", "mci_lp.hip", "mci_noalloc.hip", "mci_em.hip", "mci_api.cpp",
            "mci_batch_api.cpp", "mci_lp_api.cpp", "mci_rtc.cpp"]
 ROOT = os.path.dirname(HERE)
 # headers the run-time build of the step kernels with the caller's device functors needs, under the
@@ -61,13 +61,17 @@ FLAGS = ["-std=c++17", "-O3", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=
          "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument"]
 # the learned move keeps the last layer's 128 outputs per lane across phases: matrix-core results in
 # ordinary VGPRs, so that they are not held twice (accumulation registers and VGPRs)
+# sources compiled in several parts at once, each with its number in a macro
+PARTS = {"mci_fast_group.hip": ("GROUP_PART", 7)}
 EXTRA = {"mci_lp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
-def _compile(src):
-    obj = os.path.join(OUT, os.path.splitext(os.path.basename(src))[0] + ".o")
+def _compile(src, part=None):
+    name = os.path.splitext(os.path.basename(src))[0]
+    obj = os.path.join(OUT, name + (".o" if part is None else f"_{part}.o"))
     lang = ["-x", "hip"] if src.endswith(".hip") else []
-    cmd = [HIPCC] + FLAGS + EXTRA.get(src, []) + lang + ["-c", os.path.join(CSRC, src), "-o", obj]
+    define = [] if part is None else [f"-D{PARTS[src][0]}={part}"]
+    cmd = [HIPCC] + FLAGS + EXTRA.get(src, []) + define + lang + ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")
@@ -76,9 +80,10 @@ def _compile(src):
 
 def build(verbose=False):
     os.makedirs(OUT, exist_ok=True)
-    srcs = SOURCES + [_embed()]
-    with cf.ThreadPoolExecutor(max_workers=len(srcs)) as ex:
-        objs = list(ex.map(_compile, srcs))
+    jobs = [(src, part) for src in SOURCES + [_embed()] for part in (range(PARTS[src][1]) if src in PARTS else [None])]
+    jobs.sort(key=lambda j: j[0] not in PARTS)  # the longest first
+    with cf.ThreadPoolExecutor(max_workers=min(len(jobs), 2 * (os.cpu_count() or 8))) as ex:
+        objs = list(ex.map(lambda j: _compile(*j), jobs))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs + ["-lhiprtc"]
     r = subprocess.run(cmd, capture_output=True, text=True)

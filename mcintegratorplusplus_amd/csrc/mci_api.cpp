@@ -384,6 +384,7 @@ hipError_t calibrate_indep_launch(const mci_ctx *c, const Chain &ch, int nfind, 
 mci_status mt_align_if_needed(mci_ctx *c)
 {
     if (c->rng != MCI_RNG_MT19937_64 || !c->mt_diverged) { return MCI_OK; }
+    if (fast_rotates_mt(c->movetype, c->ndim, c->W)) { return MCI_OK; }
     HIPCHK(launch_mt_align(c->mt.p, c->mtp.p, c->W, c->stream));
     c->mt_diverged = false;
     return MCI_OK;

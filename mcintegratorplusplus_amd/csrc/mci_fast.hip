@@ -23,77 +23,15 @@
 // acceptance uniform on a 2^-24 grid, block sums as Kahan-compensated FP32 pairs, flushed to
 // FP64 for the FP64 estimators.  Every FP32 operation is correctly rounded and exp is the
 // library's own bexp (mci_f32math.hpp), so the CPU oracle reproduces the chain bit for bit.
-#include "mci_f32math.hpp"
-#include "mci_fast.hpp"
-#include "mci_fast_plan.hpp"
-#include "mci_kernels.hpp"
+#include "mci_fast_dev.hpp"
+#include "mci_fast_group.hpp"
 
-#include <float.h>
 #include <type_traits>
 
 namespace mcid
 {
 namespace
 {
-constexpr int WAVE = 64;
-
-struct FastArgs
-{
-    int64_t W;
-    int ndim;
-    int64_t nsteps;
-    uint32_t key0, key1;
-    uint64_t *ctr;         // [W]
-    double *x64;           // [ndim][W] (FP64 state, also FP32 mode's persistent copy)
-    const double *a;       // [ndim] p_i = a_i x_i^2
-    double *steps;         // [W] (one type; rescaled in place by a launch with a pending factor)
-    int64_t *acc, *rej;    // [W]
-    int64_t blocksize;     // B (Simple: nsteps)
-    int64_t nblocks;
-    double *d_x2;          // X2 data [nblocks][ndim][W] or nullptr
-    double *d_x2sum;       // X2_SUM data [nblocks][1][W] or nullptr
-    double *d_exp;         // EXP_X2 data [nblocks][1][W] or nullptr
-    double x2sum_div;      // X2_SUM divisor
-    double exp_div;        // EXP_X2 divisor
-    int nvecs;
-    uint32_t lemire_thr;   // 2^32 mod nvecs
-    int ibits;             // index bits m in the shared word (nvecs = 2^m), -1: Lemire index
-    int vshift;            // 32 - m: the index is the shared word's bits [vshift, 32) (none when m = 0)
-    uint32_t ubits;        // max(m, 0): the acceptance uniform's bits start below the index
-    uint32_t umask;        // FP64: the shared word's n = 32 - ubits acceptance bits
-    float uexp;            // FP64: n, the screening exponent's offset
-    const CalibCtrl *pend; // shared calibration: pending step factor, loop finished (FP64 kernel only)
-    const double *dimsizes;
-    uint64_t *mt;          // reference streams: [312][W] mt19937_64 states (F_MT launches)
-    int32_t *mtp;          // [W] next state index
-    const uint8_t *active; // [W] or nullptr: walkers whose flag is 0 do nothing (the independent
-                           // decorrelation rounds of walkers that have finished theirs)
-    const int32_t *wmap;   // or nullptr: the walker each lane's columns belong to (its Philox stream),
-    const int32_t *wcount; // and the number of lanes in use, when the walkers are compacted
-};
-
-__device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1,
-                                       uint32_t &o0, uint32_t &o1, uint32_t &o2, uint32_t &o3)
-{
-#pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        if (r > 0) { k0 += 0x9E3779B9u; k1 += 0xBB67AE85u; }
-        const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
-        const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
-        const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
-        c1 = (uint32_t)p1;
-        c3 = (uint32_t)p0;
-        c0 = n0;
-        c2 = n2;
-    }
-    o0 = c0; o1 = c1; o2 = c2; o3 = c3;
-}
-
-// a or b by a lane's flag as arithmetic on the values: a select of two elements of a register array
-// can otherwise become a select of their addresses, which puts the array in scratch memory
-__device__ __forceinline__ uint32_t pick(bool on, uint32_t a, uint32_t b) { return b ^ ((a ^ b) & (0u - (uint32_t)on)); }
-
 // Lemire index on [0, range) from word w0 (SRRDVecMove.hpp:78 through uniform_int_distribution), for
 // a range whose index the shared word does not hold: low = (w0 * range) mod 2^32 < thr = 2^32 mod
 // range rejects and draws from the extra-word stream of step t.  thr is computed on the host; a wave
@@ -114,12 +52,6 @@ __device__ __forceinline__ int draw_lemire(uint32_t w0, uint32_t range, uint32_t
     }
     return (int)(prod >> 32);
 }
-
-// observable set of one launch (template flags: no per-step branches on them)
-// F_P2: the index is the shared word's top bits (a power-of-two range); F_FULL: Full accumulators (every
-// step's values stored)
-// F_MT: the reference streams (mt19937_64 per walker) instead of the native ones
-enum { F_X2 = 1, F_SUM = 2, F_EXP = 4, F_P2 = 8, F_FULL = 16, F_MT = 32 };
 
 // FP64 chain.  One wave runs alone on its SIMD at the benchmark size (65,536 walkers =
 // 1,024 waves), so a step costs about 4 cycles per instruction of any kind and 16 per
@@ -158,15 +90,6 @@ struct Run64
     double mult;  // steps of the block a value set now counts for (B - j)
     uint32_t na;  // accepted steps of the chunk
 };
-
-// canonical53 of the reference streams (generate_canonical<double, 53> on mt19937_64): w / 2^64,
-// clamped below 1 (as in mci_device.hpp)
-__device__ __forceinline__ double mt_canonical(uint64_t w)
-{
-    double r = (double)w / 18446744073709551616.0;
-    if (r >= 1.0) { r = 0x1.fffffffffffffp-1; }
-    return r;
-}
 
 // One step on coordinate v (LDS slot `slot`) from its value xo and block sum So, which the caller
 // read and which hold the values after the step on return.  Native streams: w0 is the step's
@@ -862,9 +785,7 @@ __global__ __launch_bounds__(WAVE) void k_fast64_all(FastArgs A)
 // wave-uniform d guard, so a step touches no LDS.  The arithmetic, the draws and the per-step sums
 // are those of k_fast64_all (bit-identical to the generic kernel).  Native streams: steps go in
 // pairs, one Philox block per two words of each of the two steps (the first step keeps words 2 and
-// 3 of every block for the second), so a pair computes ceil((d + 1) / 2) blocks.  Reference streams:
-// the walker's mt19937_64 outputs are made 32 at a time (their state words loaded a chunk ahead)
-// into a per-lane LDS ring of 64; a step reads its d + 1 outputs from the ring.
+// 3 of every block for the second), so a pair computes ceil((d + 1) / 2) blocks.
 // EX: d == DM exactly (every coordinate guard folds away, the step is straight-line code).
 template <int FL, int DM, bool EX>
 __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
@@ -873,9 +794,7 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
     constexpr bool HX2 = (FL & F_X2) != 0, HSUM = (FL & F_SUM) != 0, HEXP = (FL & F_EXP) != 0;
     constexpr bool ACC = (FL & 7) != 0 && !FULL;  // per-step block sums
     constexpr bool REC = HX2 && !FULL;             // per-coordinate block sums
-    constexpr bool MT = (FL & F_MT) != 0;
     constexpr int NB = DM / 2 + 1;                 // Philox blocks of a step pair at most
-    extern __shared__ double lds[];
     const int d = EX ? DM : A.ndim;
     const int lane = threadIdx.x;
     const int64_t w = (int64_t)blockIdx.x * WAVE + lane;
@@ -911,30 +830,26 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
     if (HEXP) { e = exp(-(q / A.exp_div)); }
     const double step = A.steps[w];
     const uint32_t wid = A.wmap ? (uint32_t)A.wmap[w] : (uint32_t)w;
-    [[maybe_unused]] uint64_t t = MT ? 0 : A.ctr[w];
+    uint64_t t = A.ctr[w];
     int64_t nacc = 0, inblk = 0, b = 0, s = 0;
 
     // the decision of a step from the proto sum Snew and |x'|^2 qn of its proposal (xn), then the
-    // observables after it; uw: the native shared word or the reference acceptance output
-    auto finish = [&](double Snew, double qn, uint64_t uw) {
+    // observables after it; uw: the shared word
+    auto finish = [&](double Snew, double qn, uint32_t uw) {
         const double ee = Sold - Snew;
-        const float U = MT ? (float)(uint32_t)(uw >> 32) : (float)(uint32_t)uw;
+        const float U = (float)uw;
         const float F = __builtin_amdgcn_exp2f(fmaf((float)ee, 0x1.715476p+0f, 32.0f));
-        const float Facc = MT ? fmaf(F, 0.9999f, -3.0f) : fmaf(F, 0.9999f, -2.0f);
-        const float Frej = MT ? fmaf(F, 1.0001f, 1.0f) : F * 1.0001f;
+        const float Facc = fmaf(F, 0.9999f, -2.0f);
+        const float Frej = F * 1.0001f;
         bool acc = U < Facc;
         const bool band = !acc && U <= Frej;
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(band) != 0, 0)) {
-            double u;
-            if (MT) { u = (mt_canonical(uw) * 1.0) + 0.0; }
-            else {
-                uint32_t l0, l1, l2, l3;
-                philox(0x30000000u, wid, (uint32_t)t, (uint32_t)(t >> 32), A.key0, A.key1, l0, l1, l2, l3);
-                u = (double)((((uint64_t)(uint32_t)uw << 32) | l0) >> 11) * 0x1p-53;
-            }
+            uint32_t l0, l1, l2, l3;
+            philox(0x30000000u, wid, (uint32_t)t, (uint32_t)(t >> 32), A.key0, A.key1, l0, l1, l2, l3);
+            const double u = (double)((((uint64_t)uw << 32) | l0) >> 11) * 0x1p-53;
             if (band) { acc = u <= exp(ee); }
         }
-        if (!MT) { ++t; }
+        ++t;
         nacc += acc ? 1 : 0;
         Sold = acc ? Snew : Sold;
         q = acc ? qn : q;
@@ -992,133 +907,62 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
         qn = qn + v * v;
     };
 
-    if constexpr (MT) {
-        constexpr int MT_C = 32, RING = 64;
-        uint64_t *ring = reinterpret_cast<uint64_t *>(lds);  // [RING][64]
-        const int kw = A.mtp[w];
-        // The walkers of a wave are usually at the same state position (every step of this kernel
-        // takes d + 1 outputs; seeding starts all at 0); then the position is wave-uniform and every
-        // state access is a uniform row pointer plus the lane (scalar address arithmetic).
-        const int kf = __builtin_amdgcn_readfirstlane(kw);
-        const bool uniform = __builtin_amdgcn_ballot_w64(kw != kf) == 0;
-        const int64_t wbase = (int64_t)blockIdx.x * WAVE;
-        auto run = [&](auto uni_c) {
-            constexpr bool UNI = decltype(uni_c)::value;
-            int k = UNI ? kf : kw;
-            auto at = [&](int kk) -> uint64_t * {
-                if constexpr (UNI) { return (A.mt + ((int64_t)kk * W + wbase)) + lane; }
-                else { return A.mt + ((int64_t)kk * W + w); }
-            };
-            uint64_t xk = *at(k);
-            uint64_t x1[MT_C], xm[MT_C];
-            int64_t need = A.nsteps * (int64_t)(d + 1);
-            auto issue = [&](int kk) {
+    // main word j of step t: word 2 (t mod 2) + (j mod 2) of block j / 2 of pair t / 2; the
+    // native proposal (2 w + 1 - 2^32) 2^-32 as one exact fused multiply-add
+    auto rnd = [](uint32_t v) { return fma((double)v, 0x1p-31, -(1.0 - 0x1p-32)); };
+    const int nb = (d + 2) >> 1;
+    uint32_t sw[2 * NB];  // the second step's words of a pair
+    // one step on its own (either parity)
+    auto single = [&]() {
+        const uint32_t par = (uint32_t)(t & 1u);
+        const uint64_t tp = t >> 1;
+        double Sn = 0.0, qn = 0.0;
+        uint32_t uw = 0;
 #pragma unroll
-                for (int j = 0; j < MT_C; ++j) {
-                    const int k1 = (kk + 1 == MT_N) ? 0 : kk + 1;
-                    const int km = (kk < MT_N - MT_M) ? kk + MT_M : kk + MT_M - MT_N;
-                    x1[j] = *at(k1);
-                    xm[j] = *at(km);
-                    kk = k1;
-                }
-            };
-            if (need > 0) { issue(k); }
-            int head = 0, tail = 0, avail = 0;
-            for (int64_t st = 0; st < A.nsteps; ++st) {
-                while (avail < d + 1) {
-                    // the next chunk: exactly the outputs still to be consumed, at most MT_C
-                    const int c = (int)(need < MT_C ? need : MT_C);
-#pragma unroll
-                    for (int j = 0; j < MT_C; ++j) {
-                        if (j < c) {
-                            const uint64_t nv = mt_twist(j == 0 ? xk : x1[j - 1], x1[j], xm[j]);
-                            *at(k) = nv;
-                            ring[((head + j) & (RING - 1)) * WAVE + lane] = mt_temper(nv);
-                            k = (k + 1 == MT_N) ? 0 : k + 1;
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < MT_C; ++j) {
-                        if (j == c - 1) { xk = x1[j]; }
-                    }
-                    head = (head + c) & (RING - 1);
-                    avail += c;
-                    need -= c;
-                    if (need > 0) { issue(k); }
-                }
-                double Sn = 0.0, qn = 0.0;
-#pragma unroll
-                for (int i = 0; i < DM; ++i) {
-                    if (i < d) { propose(i, (mt_canonical(ring[((tail + i) & (RING - 1)) * WAVE + lane]) * 2.0) + (-1.0), Sn, qn); }
-                }
-                const uint64_t uw = ring[((tail + d) & (RING - 1)) * WAVE + lane];
-                tail = (tail + d + 1) & (RING - 1);
-                avail -= d + 1;
-                finish(Sn, qn, uw);
+        for (int bi = 0; bi < NB; ++bi) {
+            if (bi < nb) {
+                uint32_t o0, o1, o2, o3;
+                philox((uint32_t)bi, wid, (uint32_t)tp, (uint32_t)(tp >> 32), A.key0, A.key1, o0, o1, o2, o3);
+                const uint32_t wa = par ? o2 : o0, wb = par ? o3 : o1;
+                if (bi == 0) { uw = wa; }
+                else { propose(2 * bi - 1, rnd(wa), Sn, qn); }
+                if (2 * bi < d) { propose(2 * bi, rnd(wb), Sn, qn); }
             }
-            A.mtp[w] = k;
-        };
-        if (uniform) { run(std::integral_constant<bool, true>{}); }
-        else { run(std::integral_constant<bool, false>{}); }
-    }
-    else {
-        // main word j of step t: word 2 (t mod 2) + (j mod 2) of block j / 2 of pair t / 2; the
-        // native proposal (2 w + 1 - 2^32) 2^-32 as one exact fused multiply-add
-        auto rnd = [](uint32_t v) { return fma((double)v, 0x1p-31, -(1.0 - 0x1p-32)); };
-        const int nb = (d + 2) >> 1;
-        uint32_t sw[2 * NB];  // the second step's words of a pair
-        // one step on its own (either parity)
-        auto single = [&]() {
-            const uint32_t par = (uint32_t)(t & 1u);
-            const uint64_t tp = t >> 1;
-            double Sn = 0.0, qn = 0.0;
-            uint32_t uw = 0;
-#pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                if (bi < nb) {
-                    uint32_t o0, o1, o2, o3;
-                    philox((uint32_t)bi, wid, (uint32_t)tp, (uint32_t)(tp >> 32), A.key0, A.key1, o0, o1, o2, o3);
-                    const uint32_t wa = par ? o2 : o0, wb = par ? o3 : o1;
-                    if (bi == 0) { uw = wa; }
-                    else { propose(2 * bi - 1, rnd(wa), Sn, qn); }
-                    if (2 * bi < d) { propose(2 * bi, rnd(wb), Sn, qn); }
-                }
-            }
-            finish(Sn, qn, uw);
-        };
-        if ((t & 1u) && s < A.nsteps) { single(); }
-        while (s + 2 <= A.nsteps) {
-            const uint64_t tp = t >> 1;
-            double Sn = 0.0, qn = 0.0;
-            uint32_t uw = 0;
-#pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                if (bi < nb) {
-                    uint32_t o0, o1, o2, o3;
-                    philox((uint32_t)bi, wid, (uint32_t)tp, (uint32_t)(tp >> 32), A.key0, A.key1, o0, o1, o2, o3);
-                    sw[2 * bi] = o2;
-                    sw[2 * bi + 1] = o3;
-                    if (bi == 0) { uw = o0; }
-                    else { propose(2 * bi - 1, rnd(o0), Sn, qn); }
-                    if (2 * bi < d) { propose(2 * bi, rnd(o1), Sn, qn); }
-                }
-            }
-            finish(Sn, qn, uw);
-            Sn = 0.0;
-            qn = 0.0;
-#pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                if (bi < nb) {
-                    if (bi == 0) { uw = sw[0]; }
-                    else { propose(2 * bi - 1, rnd(sw[2 * bi]), Sn, qn); }
-                    if (2 * bi < d) { propose(2 * bi, rnd(sw[2 * bi + 1]), Sn, qn); }
-                }
-            }
-            finish(Sn, qn, uw);
         }
-        if (s < A.nsteps) { single(); }
-        A.ctr[w] = t;
+        finish(Sn, qn, uw);
+    };
+    if ((t & 1u) && s < A.nsteps) { single(); }
+    while (s + 2 <= A.nsteps) {
+        const uint64_t tp = t >> 1;
+        double Sn = 0.0, qn = 0.0;
+        uint32_t uw = 0;
+#pragma unroll
+        for (int bi = 0; bi < NB; ++bi) {
+            if (bi < nb) {
+                uint32_t o0, o1, o2, o3;
+                philox((uint32_t)bi, wid, (uint32_t)tp, (uint32_t)(tp >> 32), A.key0, A.key1, o0, o1, o2, o3);
+                sw[2 * bi] = o2;
+                sw[2 * bi + 1] = o3;
+                if (bi == 0) { uw = o0; }
+                else { propose(2 * bi - 1, rnd(o0), Sn, qn); }
+                if (2 * bi < d) { propose(2 * bi, rnd(o1), Sn, qn); }
+            }
+        }
+        finish(Sn, qn, uw);
+        Sn = 0.0;
+        qn = 0.0;
+#pragma unroll
+        for (int bi = 0; bi < NB; ++bi) {
+            if (bi < nb) {
+                if (bi == 0) { uw = sw[0]; }
+                else { propose(2 * bi - 1, rnd(sw[2 * bi]), Sn, qn); }
+                if (2 * bi < d) { propose(2 * bi, rnd(sw[2 * bi + 1]), Sn, qn); }
+            }
+        }
+        finish(Sn, qn, uw);
     }
+    if (s < A.nsteps) { single(); }
+    A.ctr[w] = t;
 #pragma unroll
     for (int i = 0; i < DM; ++i) {
         if (i < d) { A.x64[(int64_t)i * W + w] = x[i]; }
@@ -1434,12 +1278,12 @@ size_t lds_bytes(int prec, int ndim, bool x2)
     return sizeof(float) * ((size_t)(x2 ? 3 : 1) * ndim * WAVE + ndim);
 }
 
-// the all-coordinate kernels: registers up to ALL_DM coordinates (LDS: the reference streams' ring);
-// beyond, positions (X2 blocks: records), proposals, a_i and the ring in LDS
+// the one-lane all-coordinate kernels: k_fast64_allr holds up to ALL_DM coordinates in registers (no
+// LDS); k_fast64_all positions (X2 blocks: records), proposals, a_i, and the reference streams' ring or
+// the native streams' kept words
 constexpr int ALL_DM = 16;
 size_t lds_bytes_all(int ndim, bool x2, bool mt)
 {
-    if (ndim <= ALL_DM) { return mt ? sizeof(uint64_t) * 64 * WAVE : 0; }
     return sizeof(double) * ((size_t)(x2 ? 2 : 1) * ndim * WAVE + (size_t)ndim * WAVE + ndim) +
            (mt ? sizeof(uint64_t) * 16 * WAVE : sizeof(uint32_t) * (size_t)(ndim + 2) * WAVE);
 }
@@ -1463,17 +1307,23 @@ void launch_fl(int prec, dim3 grid, size_t sh, hipStream_t s, const FastArgs &A)
     else if constexpr ((FL & (F_FULL | F_MT)) == 0) { hipLaunchKernelGGL(k_fast32<FL>, grid, dim3(WAVE), sh, s, A); }
 }
 
+// All-coordinate launches that no group of lanes takes (group_shape): native streams with up to 16
+// coordinates and enough walkers to fill the card with one lane each; k_fast64_all takes what is left,
+// the widest walkers of the reference streams and rows of x_i^2 beyond 4 GiB.
 template <int FL>
 void launch_all(dim3 grid, size_t sh, hipStream_t s, const FastArgs &A)
 {
     if constexpr ((FL & F_MT) == 0) {
         if (A.ndim == ALL_DM) {
-            hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, true>), grid, dim3(WAVE), sh, s, A);
+            hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, true>), grid, dim3(WAVE), 0, s, A);
+            return;
+        }
+        if (A.ndim < ALL_DM) {
+            hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, false>), grid, dim3(WAVE), 0, s, A);
             return;
         }
     }
-    if (A.ndim <= ALL_DM) { hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, false>), grid, dim3(WAVE), sh, s, A); }
-    else { hipLaunchKernelGGL(k_fast64_all<FL>, grid, dim3(WAVE), sh, s, A); }
+    hipLaunchKernelGGL(k_fast64_all<FL>, grid, dim3(WAVE), sh, s, A);
 }
 } // namespace
 
@@ -1575,6 +1425,11 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         if (prec != MCI_PREC_FP64 || (mt && (!c.mt || !c.mtp))) { return MCI_E_INVALID_ARGUMENT; }
         if (mt) { fl |= F_MT; }
         const size_t sha = lds_bytes_all(c.ndim, (fl & F_X2) != 0 && !(fl & F_FULL), mt);
+        int L = 0, S = 0;
+        if (group_shape(mt, c.ndim, c.W, L, S)) {
+            if (!launch_group(fl, L, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
+            return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
+        }
         switch (fl) {
         case 0: launch_all<0>(grid, sha, s, A); break;
         case 1: launch_all<1>(grid, sha, s, A); break;
@@ -1667,6 +1522,12 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     default: return MCI_E_INVALID_ARGUMENT;
     }
     return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
+}
+
+bool fast_rotates_mt(int movetype, int ndim, int64_t W)
+{
+    int L, S;
+    return movetype == MCI_MOVE_ALL && group_shape(true, ndim, W, L, S);
 }
 
 void fast_release(FastState &fs) { (void)fs; }

@@ -1,0 +1,81 @@
+// mci_fast_group.hpp — launch interface of the all-coordinate kernel with a walker on a group of
+// lanes (mci_fast_group.hip).
+#pragma once
+
+#include <cstdint>
+
+#include <hip/hip_runtime.h>
+
+namespace mcid
+{
+struct FastArgs;
+
+// (lanes a walker, slots a lane) of the forms that are built.  Native streams: L S >= d + 1 words;
+// reference streams: L S >= d coordinates.
+#define GROUP_SHAPES(X)                                                                                  \
+    X(2, 2) X(2, 4) X(2, 6) X(2, 10) X(2, 18) X(4, 2) X(4, 4) X(4, 6) X(4, 10) X(4, 14) X(4, 18) X(8, 10) X(8, 16)
+#define GROUP_SHAPES_MT(X) X(4, 1) X(4, 2) X(4, 3) X(4, 4) X(4, 6) X(4, 8) X(4, 12) X(4, 16)
+
+// The form for W walkers in d dimensions; false: none (the walker runs on one lane).
+//  Reference streams: groups of four, up to 64 coordinates (elements 156 apart then share a lane).
+//  Native streams: one wave per SIMD (1,024 in all) is the fewest that use the whole card, and a step
+//  is shorter the more lanes share it, so the largest group that still gives at most one wave per
+//  SIMD (d = 16, 16,384 walkers x 10,240 steps: one lane 7.9 ms, two 5.4, four 4.2), beyond that the
+//  smallest that holds the walker in registers (d = 16, 65,536 walkers: one lane 8.0 ms, two 9.9, four
+//  13.5; d = 35: two 5.0, four 5.3 for 2,560 steps): the ordered sum and the decision are then the
+//  fewest.  Eight lanes measured the same as four for 1,000 walkers at d = 16, so they serve only the
+//  widest walkers.
+inline bool group_shape(bool mt, int d, int64_t W, int &L, int &S)
+{
+    if (W * (int64_t)d >= (int64_t)1 << 29) { return false; }  // a row of x_i^2 stays below 4 GiB
+    constexpr int64_t FULL = 65536;                            // lanes of one wave per SIMD
+    const int need = mt ? d : d + 1;
+    const int lanes[] = {4, 2, 8};
+    int bestL = 0, bestS = 0;
+    auto smallest = [&](int l) {
+        int s = 0;
+#define SHAPE(a, b)                                                                                      \
+    if (a == l && a * b >= need && (s == 0 || b < s)) { s = b; }
+        if (mt) { GROUP_SHAPES_MT(SHAPE) }
+        else { GROUP_SHAPES(SHAPE) }
+#undef SHAPE
+        return s;
+    };
+    if (mt) {
+        L = 4;
+        S = smallest(4);
+        return S != 0;
+    }
+    for (int l : lanes) {
+        const int s = smallest(l);
+        if (s == 0) { continue; }
+        if (l < 8 && W * l <= FULL) {
+            L = l;
+            S = s;
+            return true;
+        }
+        if (bestL == 0 || l < bestL) {
+            bestL = l;
+            bestS = s;
+        }
+    }
+    L = bestL;
+    S = bestS;
+    return bestL != 0 && d > 16;  // up to 16 coordinates one lane holds the walker
+}
+
+// one launch of kernel form fl (the F_* flags of mci_fast_dev.hpp); false: there is no such form
+bool launch_group_0(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_1(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_2(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_3(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_4(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_5(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_6(int fl, int L, int S, const FastArgs &A, hipStream_t s);
+inline bool launch_group(int fl, int L, int S, const FastArgs &A, hipStream_t s)
+{
+    return launch_group_0(fl, L, S, A, s) || launch_group_1(fl, L, S, A, s) || launch_group_2(fl, L, S, A, s) ||
+           launch_group_3(fl, L, S, A, s) || launch_group_4(fl, L, S, A, s) || launch_group_5(fl, L, S, A, s) ||
+           launch_group_6(fl, L, S, A, s);
+}
+} // namespace mcid

@@ -1,0 +1,46 @@
+"""The all-coordinate kernel with a walker on a group of lanes against the generic kernel, at the edges
+of its forms: the smallest and largest dimensions of each (lanes, slots), walker counts that leave a
+ragged last wave or call for two, four or eight lanes, odd step counts (a step pair cut, generator
+outputs left over), and launches that continue the streams.  Every number is bit-identical."""
+import numpy as np
+import pytest
+
+from mcitest import (ESTIM_MJ, ESTIM_NOOP, KERNELS_GENERIC, OBS_EXP_X2, OBS_X2, OBS_X2_SUM, PDF_GAUSS_DIAG, PDF_GAUSS_ISO, RNG_MT,
+                     RNG_PHILOX, chain_setup)
+
+pytestmark = pytest.mark.gpu
+
+# native streams: two lanes for 17,000 walkers (where one does not hold the walker, or the card is not
+# full), four for few, eight beyond 71 coordinates
+NATIVE = [(1, 33), (3, 70), (4, 70), (7, 70), (8, 16), (15, 64), (16, 5), (23, 70), (24, 70), (36, 70), (39, 70), (40, 70), (55, 70),
+          (56, 70), (71, 33), (72, 33), (79, 9), (80, 9), (88, 20), (2, 17000), (9, 17000), (11, 17000), (16, 17000), (17, 17000),
+          (18, 33000), (35, 17000), (40, 17000)]
+REFERENCE = [(1, 1), (2, 21), (4, 70), (5, 70), (8, 33), (9, 70), (12, 16), (13, 70), (16, 70), (17, 70), (24, 21), (25, 21), (32, 33),
+             (33, 21), (48, 21), (49, 21), (51, 21), (63, 21), (64, 33), (65, 5)]
+ALL_OBS = [OBS_X2, OBS_X2_SUM, OBS_EXP_X2]
+
+
+@pytest.mark.parametrize("rng,d,W", [(RNG_PHILOX, *c) for c in NATIVE] + [(RNG_MT, *c) for c in REFERENCE])
+def test_walker_on_a_group_of_lanes(rng, d, W):
+    print("lane groups", rng, d, W, flush=True)
+    blocksize = (3, 1, 0)[d % 3]
+    obs = [[OBS_X2], [OBS_X2_SUM], ALL_OBS, [OBS_X2, OBS_X2_SUM], [OBS_EXP_X2], [OBS_X2, OBS_EXP_X2]][d % 6]
+    est = ESTIM_NOOP if blocksize == 0 else ESTIM_MJ
+    sig = np.random.default_rng(d).uniform(0.5, 2.0, d)
+    pdf = (PDF_GAUSS_ISO, []) if d % 4 == 1 else (PDF_GAUSS_DIAG, 0.5 / sig ** 2)
+    cfg = dict(ndim=d, seed=77 + d, ndecorr=37, move=(0, 0, 1, None), pdfs=[pdf],
+               obs=[(k, [], blocksize, 1, 0, est) for k in obs])
+    n1 = 64 * max(blocksize, 1) if blocksize else 151
+    out = {}
+    for path in ("groups", "generic"):
+        c = chain_setup("mci", cfg, nwalkers=W)
+        c.setRng(rng)
+        c.setCoupling(1)
+        if path == "generic":
+            c.setKernelPath(KERNELS_GENERIC)
+        first = c.integrate(n1)
+        data = [c.observableData(i, d if k == OBS_X2 else 1) for i, k in enumerate(obs)]
+        second = c.integrate(16 * max(blocksize, 1), False, True)
+        out[path] = (*first, *second, c.getX(), c.getWalkerSteps(), *c.walkerAcceptance(), *c.walkerResults(), *data)
+    for k, (f, g) in enumerate(zip(out["groups"], out["generic"])):
+        assert np.array_equal(f, g), k

@@ -148,7 +148,7 @@ struct mci_ctx
     DBuf<uint64_t> cmp_mt, cmp_ctr;
     DBuf<int32_t> cmp_mtp, cmp_list, cmp_count;
     int calib_indep_hint = 0; // iterations the last such calibration took: the next one's first batch
-    std::vector<DBuf<double>> accdata, scratch;
+    std::vector<DBuf<double>> accdata, scratch, tracesum;
     std::vector<double> h_wavg, h_werr;
     int nobsdim_last = 0;
     std::vector<int64_t> nstore_last; // rows of each observable's data after the last integrate
@@ -1639,7 +1639,7 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
     if (nmc > 0) {
         // ---- accumulators (MCIntegrator.cpp:54-57), allocated before any work so that a
         //      configuration the kernels cannot run fails before calibration ----
-        if (c->accdata.size() < c->obs.size()) { c->accdata.resize(c->obs.size()); c->scratch.resize(c->obs.size()); }
+        if (c->accdata.size() < c->obs.size()) { c->accdata.resize(c->obs.size()); c->scratch.resize(c->obs.size()); c->tracesum.resize(c->obs.size()); }
         int voff = 0;
         for (size_t i = 0; i < c->obs.size(); ++i) {
             const ObsHost &o = c->obs[i];
@@ -1669,6 +1669,14 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
             for (const ObsDev &d : od) {
                 if (d.acc == ACC_SIMPLE) { return fail(MCI_E_INVALID_ARGUMENT, "FP32 precision accumulates at most 2^31 - 1 steps per block (Simple accumulator: per run)"); }
             }
+        }
+    }
+    // the estimators that need a trace's mean first take its sum from the sampling launch
+    if (fast_main && c->obsfile.empty() && c->wlkfile.empty() && fast_sums_traces(c->movetype, c->rng, c->ndim, W)) {
+        for (size_t i = 0; i < od.size(); ++i) {
+            if (od[i].acc != ACC_FULL || !needs_scratch(c->obs[i].estim, od[i].nstore)) { continue; }
+            HIPCHK(c->tracesum[i].ensure((size_t)od[i].nobs * W));
+            od[i].sum = c->tracesum[i].p;
         }
     }
     // ---- file output of the main sampling (MCIntegrator.cpp:61-65, 495-542): the generic kernel
@@ -1752,6 +1760,7 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
         j.nobs = od[i].nobs;
         j.off = od[i].voff;
         j.estim = c->obs[i].estim;
+        j.sum = od[i].sum;
         j.scale = vol;
         j.active = nullptr;
         j.avg = c->wavg.p;

@@ -48,6 +48,7 @@ struct ObsDev
     double p0;        // first parameter (divisor, constant or index)
     int64_t nstore;   // rows of data: 1 (simple), NAccu (full), nblocks (block)
     double *data;     // [nstore][nobs][W]
+    double *sum;      // Full accumulators on the specialised kernels: [nobs][W] sums of the traces, or nullptr
 };
 
 // Everything a kernel needs to advance W walkers; passed by value.

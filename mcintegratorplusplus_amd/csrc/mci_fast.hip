@@ -862,11 +862,22 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
             if (HX2) {
 #pragma unroll
                 for (int i = 0; i < DM; ++i) {
-                    if (i < d) { A.d_x2[(s * d + i) * W + w] = x[i] * x[i]; }
+                    if (i < d) {
+                        const double v = x[i] * x[i];
+                        sm[i] = sm[i] + v;
+                        A.d_x2[(s * d + i) * W + w] = v;
+                    }
                 }
             }
-            if (HSUM) { A.d_x2sum[s * W + w] = q / A.x2sum_div; }
-            if (HEXP) { A.d_exp[s * W + w] = e; }
+            if (HSUM) {
+                const double v = q / A.x2sum_div;
+                Sr = Sr + v;
+                A.d_x2sum[s * W + w] = v;
+            }
+            if (HEXP) {
+                Se = Se + e;
+                A.d_exp[s * W + w] = e;
+            }
         }
         if (ACC) {
             if (REC) {
@@ -965,8 +976,13 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
     A.ctr[w] = t;
 #pragma unroll
     for (int i = 0; i < DM; ++i) {
-        if (i < d) { A.x64[(int64_t)i * W + w] = x[i]; }
+        if (i < d) {
+            A.x64[(int64_t)i * W + w] = x[i];
+            if (FULL && HX2 && A.s_x2) { A.s_x2[(int64_t)i * W + w] = sm[i]; }
+        }
     }
+    if (FULL && HSUM && A.s_x2sum) { A.s_x2sum[w] = Sr; }
+    if (FULL && HEXP && A.s_exp) { A.s_exp[w] = Se; }
     A.acc[w] = nacc;
     A.rej[w] = A.nsteps - nacc;
 }
@@ -1406,6 +1422,7 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     A.blocksize = 1;
     A.nblocks = 0;
     A.d_x2 = A.d_x2sum = A.d_exp = nullptr;
+    A.s_x2 = A.s_x2sum = A.s_exp = nullptr;
     A.x2sum_div = 1.0;
     A.exp_div = (double)c.ndim;
     int fl = 0;
@@ -1414,9 +1431,9 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         if (o.acc == ACC_FULL) { fl |= F_FULL; }
         A.blocksize = (o.acc == ACC_SIMPLE) ? nsteps : (int64_t)o.blocksize;
         A.nblocks = o.nstore;
-        if (o.kind == MCI_OBS_X2) { A.d_x2 = o.data; fl |= F_X2; }
-        if (o.kind == MCI_OBS_X2_SUM) { A.d_x2sum = o.data; A.x2sum_div = o.p0; fl |= F_SUM; }
-        if (o.kind == MCI_OBS_EXP_X2) { A.d_exp = o.data; A.exp_div = o.p0; fl |= F_EXP; }
+        if (o.kind == MCI_OBS_X2) { A.d_x2 = o.data; A.s_x2 = o.sum; fl |= F_X2; }
+        if (o.kind == MCI_OBS_X2_SUM) { A.d_x2sum = o.data; A.s_x2sum = o.sum; A.x2sum_div = o.p0; fl |= F_SUM; }
+        if (o.kind == MCI_OBS_EXP_X2) { A.d_exp = o.data; A.s_exp = o.sum; A.exp_div = o.p0; fl |= F_EXP; }
     }
     if (!A.a && c.movetype != MCI_MOVE_ALL) { return MCI_E_INVALID_ARGUMENT; } // single-coordinate moves: explicit weights
     if (prec != MCI_PREC_FP64 && A.blocksize > INT32_MAX) { return MCI_E_INVALID_ARGUMENT; }
@@ -1522,6 +1539,12 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     default: return MCI_E_INVALID_ARGUMENT;
     }
     return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
+}
+
+bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
+{
+    int L, S;
+    return movetype == MCI_MOVE_ALL && (group_shape(rng == MCI_RNG_MT19937_64, ndim, W, L, S) || (rng == MCI_RNG_PHILOX && ndim <= ALL_DM));
 }
 
 bool fast_rotates_mt(int movetype, int ndim, int64_t W)

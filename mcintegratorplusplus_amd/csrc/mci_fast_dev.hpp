@@ -29,6 +29,7 @@ struct FastArgs
     double *d_x2;          // X2 data [nblocks][ndim][W] or nullptr
     double *d_x2sum;       // X2_SUM data [nblocks][1][W] or nullptr
     double *d_exp;         // EXP_X2 data [nblocks][1][W] or nullptr
+    double *s_x2, *s_x2sum, *s_exp;  // Full accumulators: the sums of the traces, [ndim][W], [W], [W], or nullptr
     double x2sum_div;      // X2_SUM divisor
     double exp_div;        // EXP_X2 divisor
     int nvecs;

@@ -257,15 +257,20 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
             if (HX2) {
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
-                    if (ok[s]) { put(rx, offx[s], x[s] * x[s]); }
+                    const double v = x[s] * x[s];
+                    sm[s] = sm[s] + v;
+                    if (ok[s]) { put(rx, offx[s], v); }
                 }
                 rx += rowx;
             }
             if (HSUM) {
-                if (g == 0) { put(rs, off, q / A.x2sum_div); }
+                const double v = q / A.x2sum_div;
+                Sr = Sr + v;
+                if (g == 0) { put(rs, off, v); }
                 rs += w8;
             }
             if (HEXP) {
+                Se = Se + e;
                 if (g == 0) { put(re, off, e); }
                 re += w8;
             }
@@ -438,9 +443,14 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        if (ok[s]) { A.x64[(int64_t)(c0 + s) * W + w] = x[s]; }
+        if (ok[s]) {
+            A.x64[(int64_t)(c0 + s) * W + w] = x[s];
+            if (FULL && HX2 && A.s_x2) { A.s_x2[(int64_t)(c0 + s) * W + w] = sm[s]; }
+        }
     }
     if (g == 0) {
+        if (FULL && HSUM && A.s_x2sum) { A.s_x2sum[w] = Sr; }
+        if (FULL && HEXP && A.s_exp) { A.s_exp[w] = Se; }
         A.acc[w] = nacc;
         A.rej[w] = A.nsteps - nacc;
     }

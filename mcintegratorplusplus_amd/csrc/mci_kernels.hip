@@ -288,6 +288,7 @@ struct FcState
 
 // finishes the estimate with k blocks (running sums a, e of its k block means: the tail of
 // uncorr()) and passes it to the plateau search; k is uniform
+template <bool START>
 __device__ inline void fc_push(FcState &st, int64_t k, double aa, double ee);
 
 __device__ inline void fc_emit(FcState &st, int64_t k, double a, double e, bool onedim)
@@ -297,10 +298,12 @@ __device__ inline void fc_emit(FcState &st, int64_t k, double a, double e, bool 
     double ee = e * norm - aa * aa;
     if (ee > 1.e-300) { ee = onedim ? sqrt(ee / ((double)k - 1.)) : sqrt(ee * c_fc_rk1[k - 6]); }
     else { ee = 0.; }
-    fc_push(st, k, aa, ee);
+    fc_push<true>(st, k, aa, ee);
 }
 
-// the estimate with k blocks (average aa, error ee) into the window and the plateau search
+// the estimate with k blocks (average aa, error ee) into the window and the plateau search, which starts
+// at k = 14 (START) or has been given a value no difference is below
+template <bool START>
 __device__ inline void fc_push(FcState &st, int64_t k, double aa, double ee)
 {
 #pragma unroll
@@ -317,7 +320,7 @@ __device__ inline void fc_push(FcState &st, int64_t k, double aa, double ee)
         const double fa = fabs(acd);
         const double sa = 0.2 * (st.wa[2] + st.wa[3] + st.wa[4] + st.wa[5] + st.wa[6]);
         const double se = 0.2 * (st.we[2] + st.we[3] + st.we[4] + st.we[5] + st.we[6]);
-        if (k == 14 || fa < st.best) {
+        if ((START && k == 14) || fa < st.best) {
             st.best = fa;
             st.bav = sa;
             st.ber = se;
@@ -433,22 +436,27 @@ __device__ inline void fcblocker_reg(const Col &x, double &avg, double &err)
 
 // The same for longer series, streaming each value past running block sums.  Every block count k
 // keeps its own running block sum and every value is added to each of them (independent chains);
-// the block ends come from a table built per workgroup in LDS: for each position, the mask of the
-// block counts that close a block there and the mask of those that close their last block there.
-// Each block count tests its bit (groups of eight without a close are skipped together), so the
-// sums stay in registers and no per-value bookkeeping runs on the scalar unit.  Per block count the operations and their order
-// are those of OneDim/MultiDimBlockEstimator: each block summed from 0 in index order, its mean
+// the block ends come from a table built per workgroup in LDS: for each position, the block counts that
+// close a block there and those that close their last one.  Per block count the operations and their
+// order are those of OneDim/MultiDimBlockEstimator: each block summed from 0 in index order, its mean
 // added to the running sums of means and of their squares.  After a block count's last block its
-// running sum takes the rest of the series, which no close reads.  The 45 block counts take three
-// passes over the series (15 each: their three running sums each fit the registers); each pass
-// hands its finished estimates to the windowed plateau search in increasing k.  The values reach LDS in batches of eight through a two-batch ring per lane, the
-// loads two batches ahead; each value and its masks are read one position ahead.
+// running sum takes the rest of the series, which no close reads.
+//
+// A workgroup is three waves over the same 64 series, each with fifteen of the 45 block counts, whose
+// running sums fit its registers; the values come from memory once, through tiles in LDS that the
+// three waves load in turn.  The plateau search of each wave continues the window of the one before;
+// its smallest differences are then compared in the order of the block counts.  The additions bound
+// it: 1,048,576 series x 800 values hold 45 x 800 additions each, 1.3 ms at the card's FP64 rate (the
+// 6.7 GB once: 1.3 ms).
+// One wave with three passes over the series (20 GB) took 4.4 ms; this takes 2.7 ms (and one walker 75 us
+// instead of 256).
 constexpr int64_t FC_STREAM_MAX = 2048;
-constexpr int FC_STREAM_TPB = 256;
-constexpr int FC_SB = 16;
+constexpr int FC_WAVES = 3, FC_STREAM_TPB = 64 * FC_WAVES;
+constexpr int FC_NQ = FC_NB / FC_WAVES;             // block counts of a wave
+constexpr int FC_ROWS = 8, FC_TILE = FC_WAVES * FC_ROWS;  // positions a wave loads, positions of a tile
 __host__ __device__ inline size_t fc_stream_lds(int64_t n)
 {
-    return 16 * (size_t)n + 48 * 8 + (FC_STREAM_TPB / 64) * (2 * FC_SB) * 64 * 8;
+    return sizeof(double) * (2 * FC_TILE * 64 + 48) + sizeof(uint32_t) * FC_WAVES * (size_t)(n + FC_TILE);
 }
 
 template <bool ONEDIM>
@@ -463,125 +471,160 @@ __device__ inline void fc_finish(int k, double &a, double &e)
     e = ee;
 }
 
-__device__ inline uint64_t uniform64(uint64_t v)
+__device__ inline double uniform_value(double v)
 {
-    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)u), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-// rows i0 .. i0+FC_SB-1 of a series (indices past the end clamped to its last value)
-__device__ inline void fc_load_batch(const double *xp, int64_t stride, int n, int i0, double (&v)[FC_SB])
+// block counts k = Q0+6 .. Q0+FC_NQ+5 of this wave over the whole series; every wave of the workgroup
+// calls its own.  marks[i]: bit q: block count Q0+q+6 closes a block at position i; bit 16+q: its last
+template <bool ONEDIM, int Q0>
+__device__ inline void fc_stream_wave(const double *xp, int64_t stride, int n, const uint32_t *marks, const double *nrm, double *tile,
+                                      FcState &st)
 {
-    if (i0 + FC_SB <= n) {
-        const double *q = xp + (int64_t)i0 * stride;
-#pragma unroll
-        for (int t = 0; t < FC_SB; ++t) {
-            v[t] = *q;
-            q += stride;
-        }
-    }
-    else {
-#pragma unroll
-        for (int t = 0; t < FC_SB; ++t) { v[t] = xp[(int64_t)((i0 + t < n) ? i0 + t : n - 1) * stride]; }
-    }
-}
-
-// block counts k = Q0+6 .. Q1+5 over the whole series
-template <bool ONEDIM, int Q0, int Q1>
-__device__ inline void fc_stream_pass(const double *xp, int64_t stride, int n, const uint64_t *cmask, const uint64_t *fmask,
-                                      const double *nrm, double *ring, FcState &st)
-{
-    constexpr int NQ = Q1 - Q0;
-    constexpr uint64_t RANGE = ((1ull << NQ) - 1) << Q0;
-    double s[NQ], a[NQ], e[NQ];
+    constexpr int NQ = FC_NQ, WV = Q0 / FC_NQ;
+    const int lane = threadIdx.x & 63;
+    double s[NQ], a[NQ], e[NQ], r[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         s[q] = 0.0;
         a[q] = 0.;
         e[q] = 0.;
+        r[q] = uniform_value(nrm[Q0 + q]);
     }
-    double v[FC_SB];
-    fc_load_batch(xp, stride, n, 0, v);
+    // this wave's rows of the tile that starts at position i0 (past the end: the last value)
+    double v[FC_ROWS];
+    auto load = [&](int i0) {
+        const int i1 = i0 + WV * FC_ROWS;
+        if (i1 + FC_ROWS <= n) {
+            const double *p = xp + (int64_t)i1 * stride;
 #pragma unroll
-    for (int t = 0; t < FC_SB; ++t) { ring[t * 64] = v[t]; }
-    fc_load_batch(xp, stride, n, FC_SB, v);
-    double x = ring[0];
-    uint64_t cm = cmask[0], fm = fmask[0];
-    for (int i0 = 0; i0 < n; i0 += FC_SB) {
-        // batch j + 1 into the ring's other half, batch j + 2's loads in flight
-        const int half = ((i0 / FC_SB + 1) & 1) * FC_SB;
+            for (int t = 0; t < FC_ROWS; ++t) { v[t] = p[t * stride]; }
+        }
+        else {
 #pragma unroll
-        for (int t = 0; t < FC_SB; ++t) { ring[(half + t) * 64] = v[t]; }
-        fc_load_batch(xp, stride, n, i0 + 2 * FC_SB, v);
-        const int iend = (i0 + FC_SB < n) ? i0 + FC_SB : n;
+            for (int t = 0; t < FC_ROWS; ++t) { v[t] = xp[(int64_t)(i1 + t < n ? i1 + t : n - 1) * stride]; }
+        }
+    };
+    auto keep = [&](double *buf) {
+#pragma unroll
+        for (int t = 0; t < FC_ROWS; ++t) { buf[(WV * FC_ROWS + t) * 64 + lane] = v[t]; }
+    };
+    double *cur = tile, *nxt = tile + FC_TILE * 64;
+    load(0);
+    keep(cur);
+    load(FC_TILE);
+    __syncthreads();
+    for (int i0 = 0; i0 < n; i0 += FC_TILE) {
+        keep(nxt);                              // the next tile, while this one is summed
+        load(i0 + 2 * FC_TILE);
+        const int m = (n - i0 < FC_TILE) ? n - i0 : FC_TILE;
+        const uint32_t mk = marks[i0 + (lane < FC_TILE ? lane : 0)];  // lane t: the marks of position i0 + t
+        double x = cur[lane];
 #pragma unroll 1
-        for (int i = i0; i < iend; ++i) {
+        for (int t = 0; t < m; ++t) {
             const double xc = x;
-            const uint64_t cc = cm, ff = fm;
-            if (i + 1 < n) {
-                x = ring[((i + 1) & (2 * FC_SB - 1)) * 64];
-                cm = cmask[i + 1];
-                fm = fmask[i + 1];
-            }
+            x = cur[((t + 1 < m) ? t + 1 : t) * 64 + lane];
+            const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)mk, t);
 #pragma unroll
             for (int q = 0; q < NQ; ++q) { s[q] = s[q] + xc; }
-            const uint64_t c = uniform64(cc) & RANGE;
-            if (c == 0) { continue; }
-            const uint64_t f = uniform64(ff);
-            // each block count that closes here updates its own registers (no dispatch, no merge);
-            // groups of eight block counts with no close skipped at once
+            if ((c & 0xFFFFu) == 0u) { continue; }
+            // each block count that closes here updates its own registers (no dispatch, no merge); groups
+            // of five without a close are skipped at once
 #pragma unroll
-            for (int g = Q0; g < Q1; g += 8) {
-                if ((c >> g) & 0xFFull) {
+            for (int g = 0; g < NQ; g += 5) {
+                if ((c >> g) & 0x1Fu) {
 #pragma unroll
-                    for (int q = g; q < g + 8 && q < Q1; ++q) {
+                    for (int q = g; q < g + 5; ++q) {
                         if ((c >> q) & 1u) {
-                            const double m = s[q - Q0] * nrm[q];
-                            a[q - Q0] = a[q - Q0] + m;
-                            e[q - Q0] = e[q - Q0] + m * m;
-                            s[q - Q0] = 0.0;
-                            if ((f >> q) & 1u) { fc_finish<ONEDIM>(q + 6, a[q - Q0], e[q - Q0]); }
+                            const double mean = s[q] * r[q];
+                            a[q] = a[q] + mean;
+                            e[q] = e[q] + mean * mean;
+                            s[q] = 0.0;
+                            if ((c >> (16 + q)) & 1u) { fc_finish<ONEDIM>(Q0 + q + 6, a[q], e[q]); }
                         }
                     }
                 }
             }
         }
+        double *sw = cur;
+        cur = nxt;
+        nxt = sw;
+        __syncthreads();
+    }
+    // the last eight estimates to the next wave's window, then this wave's into its own
+    double *win = tile + WV * 16 * 64;
+    if (WV + 1 < FC_WAVES) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            win[(2 * t) * 64 + lane] = a[NQ - 8 + t];
+            win[(2 * t + 1) * 64 + lane] = e[NQ - 8 + t];
+        }
+    }
+    __syncthreads();
+    if (WV > 0) {
+        const double *before = tile + (WV - 1) * 16 * 64;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            st.wa[1 + t] = before[(2 * t) * 64 + lane];
+            st.we[1 + t] = before[(2 * t + 1) * 64 + lane];
+        }
+        st.best = __builtin_huge_val();
     }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) { fc_push(st, Q0 + q + 6, a[q], e[q]); }
+    for (int q = 0; q < NQ; ++q) { fc_push<WV == 0>(st, Q0 + q + 6, a[q], e[q]); }
+    double *bests = tile + 2 * 16 * 64;  // [FC_WAVES - 1][3][64]
+    if (WV > 0) {
+        bests[((WV - 1) * 3) * 64 + lane] = st.best;
+        bests[((WV - 1) * 3 + 1) * 64 + lane] = st.bav;
+        bests[((WV - 1) * 3 + 2) * 64 + lane] = st.ber;
+    }
+    __syncthreads();
+    if (WV == 0) {
+#pragma unroll
+        for (int t = 0; t < FC_WAVES - 1; ++t) {
+            const double b = bests[(t * 3) * 64 + lane];
+            if (b < st.best) {
+                st.best = b;
+                st.bav = bests[(t * 3 + 1) * 64 + lane];
+                st.ber = bests[(t * 3 + 2) * 64 + lane];
+            }
+        }
+    }
 }
 
 template <bool ONEDIM>
 __global__ __launch_bounds__(FC_STREAM_TPB) void k_fc_stream(EstimJob j)
 {
     extern __shared__ double fs_sh[];
-    const int n = (int)j.n;
-    uint64_t *cmask = reinterpret_cast<uint64_t *>(fs_sh);
-    uint64_t *fmask = cmask + n;
-    double *nrm = reinterpret_cast<double *>(fmask + n);
-    double *ring = nrm + 48 + (threadIdx.x >> 6) * (2 * FC_SB * 64) + (threadIdx.x & 63);  // [16][64] per wave
-    for (int i = threadIdx.x; i < n; i += FC_STREAM_TPB) {
-        cmask[i] = 0;
-        fmask[i] = 0;
-    }
+    static_assert((2 * 16 + (FC_WAVES - 1) * 3) * 64 <= 2 * FC_TILE * 64, "the windows and minima fit the tiles");
+    const int n = (int)j.n, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double *tile = fs_sh;                       // [2][FC_TILE][64]
+    double *nrm = tile + 2 * FC_TILE * 64;      // [48]
+    uint32_t *marks = reinterpret_cast<uint32_t *>(nrm + 48);  // [FC_WAVES][n + FC_TILE]
+    const int rows = n + FC_TILE;
+    const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
+    bool live = tid < j.W * j.nobs;
+    const int64_t w = live ? tid % j.W : 0;
+    const int comp = live ? (int)(tid / j.W) : 0;
+    if (j.wcount && w >= *j.wcount) { live = false; }
+    const int64_t wo = (live && j.wmap) ? j.wmap[w] : w;  // the walker of this column
+    if (live && j.active && !j.active[wo]) { live = false; }
+    if (__builtin_amdgcn_ballot_w64(live) == 0) { return; }  // the same in the three waves
+    for (int i = threadIdx.x; i < FC_WAVES * rows; i += FC_STREAM_TPB) { marks[i] = 0u; }
     if (threadIdx.x < FC_NB) { nrm[threadIdx.x] = 1. / (double)(n / ((int)threadIdx.x + 6)); }
     __syncthreads();
     for (int r = threadIdx.x; r < FC_NB * 50; r += FC_STREAM_TPB) {
         const int q = r / 50, b = r % 50, k = q + 6;
         if (b < k) {
-            const int pos = (b + 1) * (n / k) - 1;
-            atomicOr((unsigned long long *)&cmask[pos], 1ull << q);
-            if (b == k - 1) { atomicOr((unsigned long long *)&fmask[pos], 1ull << q); }
+            const int pos = (b + 1) * (n / k) - 1, sh = q % FC_NQ;
+            atomicOr(&marks[(q / FC_NQ) * rows + pos], (1u << sh) | (b == k - 1 ? 1u << (16 + sh) : 0u));
         }
     }
     __syncthreads();
-    const int64_t tid = (int64_t)blockIdx.x * FC_STREAM_TPB + threadIdx.x;
-    if (tid >= j.W * j.nobs) { return; }
-    const int64_t w = tid % j.W;
-    const int comp = (int)(tid / j.W);
-    if (j.wcount && w >= *j.wcount) { return; }
-    const int64_t wo = j.wmap ? j.wmap[w] : w;  // the walker of this column
-    if (j.active && !j.active[wo]) { return; }
-    const double *xp = j.data + (int64_t)comp * j.W + w;
+    const double *xp = j.data + (live ? (int64_t)comp * j.W + w : 0);  // a lane without a series reads the first
     const int64_t stride = (int64_t)j.nobs * j.W;
     FcState st;
 #pragma unroll
@@ -589,11 +632,13 @@ __global__ __launch_bounds__(FC_STREAM_TPB) void k_fc_stream(EstimJob j)
     st.best = 0.;
     st.bav = 0.;
     st.ber = 0.;
-    fc_stream_pass<ONEDIM, 0, 15>(xp, stride, n, cmask, fmask, nrm, ring, st);
-    fc_stream_pass<ONEDIM, 15, 30>(xp, stride, n, cmask, fmask, nrm, ring, st);
-    fc_stream_pass<ONEDIM, 30, FC_NB>(xp, stride, n, cmask, fmask, nrm, ring, st);
-    j.avg[(int64_t)(j.off + comp) * j.W + wo] = st.bav * j.scale;
-    j.err[(int64_t)(j.off + comp) * j.W + wo] = st.ber * j.scale;
+    if (wv == 0) { fc_stream_wave<ONEDIM, 0>(xp, stride, n, marks, nrm, tile, st); }
+    else if (wv == 1) { fc_stream_wave<ONEDIM, FC_NQ>(xp, stride, n, marks + rows, nrm, tile, st); }
+    else { fc_stream_wave<ONEDIM, 2 * FC_NQ>(xp, stride, n, marks + 2 * rows, nrm, tile, st); }
+    if (wv == 0 && live) {
+        j.avg[(int64_t)(j.off + comp) * j.W + wo] = st.bav * j.scale;
+        j.err[(int64_t)(j.off + comp) * j.W + wo] = st.ber * j.scale;
+    }
 }
 
 // a thread's series staged in LDS, one column per lane of a 64-thread workgroup, rows allocated to a
@@ -637,7 +682,7 @@ __constant__ double c_chi2_q95[64] = {
 // The first MJ_LB blocking levels of a block of 2^MJ_LB values, in registers: each level's terms
 // added to its sums in index order (FIRST: the series' first block, whose first value has no
 // predecessor), then the block halved in place; v[0] ends as the block's value at level MJ_LB.
-constexpr int MJ_LB = 4, MJ_BS = 1 << MJ_LB;
+constexpr int MJ_BS = 1 << MJ_LB;
 template <bool FIRST>
 __device__ inline void mj_block_levels(double (&v)[MJ_BS], double mean, double (&g0)[MJ_LB], double (&g1)[MJ_LB], double (&pv)[MJ_LB])
 {
@@ -670,19 +715,24 @@ __device__ inline void mj_load_block(const Col &x, int64_t i0, double (&v)[MJ_BS
 // The blocking transform runs in place on this thread's column of the scratch copy `y`.
 // A level whose variance is exactly zero contributes M = 0 (the reference reads out of
 // bounds there).
-__device__ inline void mjblocker(int64_t n, const Col &x, double *y, int64_t ystride, double &avg, double &err)
+// sum: the series' sum in index order if whoever wrote the series has it (a pass over the data less), or
+// nullptr.
+__device__ inline void mjblocker(int64_t n, const Col &x, const double *sum, double *y, int64_t ystride, double &avg, double &err)
 {
     int npow = 0;
     while (((int64_t)1 << npow) < n) { ++npow; }
     double mean = 0.0;
-    int64_t i = 0;
-    for (; i + MJ_BS <= n; i += MJ_BS) {  // batches of loads, the sum in index order
-        double v[MJ_BS];
-        mj_load_block(x, i, v);
+    if (sum) { mean = *sum; }
+    else {
+        int64_t i = 0;
+        for (; i + MJ_BS <= n; i += MJ_BS) {  // batches of loads, the sum in index order
+            double v[MJ_BS];
+            mj_load_block(x, i, v);
 #pragma unroll
-        for (int t = 0; t < MJ_BS; ++t) { mean = mean + v[t]; }
+            for (int t = 0; t < MJ_BS; ++t) { mean = mean + v[t]; }
+        }
+        for (; i < n; ++i) { mean = mean + x[i]; }
     }
-    for (; i < n; ++i) { mean = mean + x[i]; }
     mean = mean / (double)n;
     double var[64], gam[64];
     int64_t nred = n;
@@ -952,7 +1002,7 @@ __global__ __launch_bounds__(256) void k_estimate(EstimJob j)
         }
         fcblocker(j.n, LdsCol{col, rows}, onedim, a, e);
     }
-    if (E == MCI_ESTIM_MJBLOCKER) { mjblocker(j.n, x, j.scratch + (int64_t)comp * j.W + w, (int64_t)j.nobs * j.W, a, e); }
+    if (E == MCI_ESTIM_MJBLOCKER) { mjblocker(j.n, x, j.sum ? j.sum + (int64_t)comp * j.W + w : nullptr, j.scratch + (int64_t)comp * j.W + w, (int64_t)j.nobs * j.W, a, e); }
     if (E == EST_MJ_SMALL) { mjblocker_small(j.n, x, est_sh + threadIdx.x, (int64_t)blockDim.x, a, e); }
     if (E == EST_MJ_REG) { mjblocker_reg<P>(x, a, e); }
     j.avg[(int64_t)(j.off + comp) * j.W + wo] = a * j.scale;
@@ -1195,19 +1245,8 @@ hipError_t launch_estimate(const EstimJob &j, hipStream_t s)
         hipLaunchKernelGGL(k_estimate<EST_FC_LDS>, g, dim3(64), sizeof(double) * 64 * (size_t)fc_rows(j.n), s, j);
     }
     else if ((j.estim == MCI_ESTIM_CORRELATED || j.estim == MCI_ESTIM_FCBLOCKER) && j.n <= FC_STREAM_MAX) {
-        const dim3 gs = grid1(j.W * j.nobs, FC_STREAM_TPB);
-        const size_t lds = fc_stream_lds(j.n);
-        if (lds > 65536) {
-            // the largest table once per process (the first such call; later calls, under a graph
-            // capture too, make no runtime call besides the launch)
-            static const hipError_t attr = [] {
-                const int mx = (int)fc_stream_lds(FC_STREAM_MAX);
-                hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fc_stream<true>), hipFuncAttributeMaxDynamicSharedMemorySize, mx);
-                if (e == hipSuccess) { e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fc_stream<false>), hipFuncAttributeMaxDynamicSharedMemorySize, mx); }
-                return e;
-            }();
-            if (attr != hipSuccess) { return attr; }
-        }
+        const dim3 gs = grid1(j.W * j.nobs, 64);
+        const size_t lds = fc_stream_lds(j.n);  // at most 49 KiB
         if (j.nobs == 1) { hipLaunchKernelGGL(k_fc_stream<true>, gs, dim3(FC_STREAM_TPB), lds, s, j); }
         else { hipLaunchKernelGGL(k_fc_stream<false>, gs, dim3(FC_STREAM_TPB), lds, s, j); }
     }

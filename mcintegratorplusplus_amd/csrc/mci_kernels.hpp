@@ -17,11 +17,17 @@ struct CalibCtrl
     unsigned arrive;  // k_calib_round's arrival counter (zeroed with the rest at each calibration)
 };
 
-// one estimator pass over one observable's accumulator data [n][nobs][W]
-// rows of the general MJBlocker's working copy for a series of n values: the blocked levels,
-// n/2 values at most (the data itself is level 0)
-inline int64_t mj_scratch_rows(int64_t n) { return n / 2 > 0 ? n / 2 : 1; }
+// levels of the general MJBlocker that stay in registers for a long series of 2^P values
+constexpr int MJ_LB = 4;
+// rows of the general MJBlocker's working copy for a series of n values: the values of level MJ_LB
+// where the levels before it stay in registers, else those of level 1 (the data itself is level 0)
+inline int64_t mj_scratch_rows(int64_t n)
+{
+    if (n >= (int64_t)2 << MJ_LB && (n & (n - 1)) == 0) { return n >> MJ_LB; }
+    return n / 2 > 0 ? n / 2 : 1;
+}
 
+// one estimator pass over one observable's accumulator data [n][nobs][W]
 struct EstimJob
 {
     const double *data;
@@ -34,6 +40,9 @@ struct EstimJob
     // or nullptr: the data's columns hold a compacted set of walkers -- column i < *wcount belongs to
     // walker wmap[i], whose results go to column wmap[i]; the other columns are not read
     const int32_t *wmap = nullptr, *wcount = nullptr;
+    // or nullptr: every series' sum in index order, [nobs][W] (the general MJBlocker's mean without a
+    // pass over the data)
+    const double *sum = nullptr;
 };
 
 #ifndef MCI_RTC_USER // the host's launch interface (not part of the run-time build of the step kernels)

@@ -1444,7 +1444,7 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         const size_t sha = lds_bytes_all(c.ndim, (fl & F_X2) != 0 && !(fl & F_FULL), mt);
         int L = 0, S = 0;
         if (group_shape(mt, c.ndim, c.W, L, S)) {
-            if (!launch_group(fl, L, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
+            if (!launch_group(fl, false, L, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
             return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
         }
         switch (fl) {
@@ -1483,11 +1483,16 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
     }
     const size_t sh = lds_bytes(prec, c.ndim, (fl & F_X2) != 0 && !(fl & F_FULL));
-    if (A.ibits >= 0) { fl |= F_P2; }
     if (mt) {
         if (prec != MCI_PREC_FP64 || (c.nvecs & (c.nvecs - 1)) != 0 || !c.mt || !c.mtp) { return MCI_E_INVALID_ARGUMENT; }
         fl |= F_MT;
+        int S = 0;
+        if (group_slots_vec(c.ndim, c.W, S)) {
+            if (!launch_group(fl, true, 4, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
+            return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
+        }
     }
+    if (A.ibits >= 0) { fl |= F_P2; }
     switch (fl) {
     case 0: launch_fl<0>(prec, grid, sh, s, A); break;
     case 1: launch_fl<1>(prec, grid, sh, s, A); break;
@@ -1544,13 +1549,15 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
 bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
 {
     int L, S;
-    return movetype == MCI_MOVE_ALL && (group_shape(rng == MCI_RNG_MT19937_64, ndim, W, L, S) || (rng == MCI_RNG_PHILOX && ndim <= ALL_DM));
+    const bool mt = rng == MCI_RNG_MT19937_64;
+    if (movetype == MCI_MOVE_ALL) { return group_shape(mt, ndim, W, L, S) || (!mt && ndim <= ALL_DM); }
+    return mt && group_slots_vec(ndim, W, S);
 }
 
 bool fast_rotates_mt(int movetype, int ndim, int64_t W)
 {
     int L, S;
-    return movetype == MCI_MOVE_ALL && group_shape(true, ndim, W, L, S);
+    return movetype == MCI_MOVE_ALL ? group_shape(true, ndim, W, L, S) : group_slots_vec(ndim, W, S);
 }
 
 void fast_release(FastState &fs) { (void)fs; }

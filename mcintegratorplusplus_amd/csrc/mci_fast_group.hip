@@ -1,9 +1,9 @@
-// mci_fast_group.hip — the all-coordinate Metropolis kernel with a walker's coordinates spread over a
-// group of lanes (SRRDAllMove with one step size, MoveType::All, the reference's default move; FP64,
-// one diagonal Gaussian or exp(-|x|^2), unbounded domain, both random streams, observables as in
-// mci_fast.hip).
+// mci_fast_group.hip — Metropolis kernels with a walker's coordinates spread over a group of lanes (FP64,
+// one diagonal Gaussian or exp(-|x|^2), unbounded domain, observables as in mci_fast.hip): all-coordinate
+// moves on both random streams (SRRDAllMove with one step size, MoveType::All, the reference's default
+// move), and single-coordinate moves on the reference streams (k_fast64_vec4, below).
 //
-// A step proposes every coordinate, x'_i = x_i + step r_i, sums the protos (x'_i x'_i) a_i in coordinate
+// k_fast64_grp: a step proposes every coordinate, x'_i = x_i + step r_i, sums the protos (x'_i x'_i) a_i in coordinate
 // order and tests u <= exp(sum p - sum p'), with the screen of k_fast64.  Every operation and its order
 // are those of the generic kernel, so every number is bit-identical to it.
 //
@@ -18,12 +18,12 @@
 
 #include "mci_fast_dev.hpp"
 
+#include <type_traits>
+
 namespace mcid
 {
 namespace
 {
-constexpr int GROUP_SEG = 6;  // reference streams: parts in which a round of the generator's elements is made
-
 // ---- within a group of L adjacent lanes ----
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
@@ -124,6 +124,122 @@ __device__ __forceinline__ double mt_symmetric(U64 w)
 {
     const double v = fma((double)apart(w.hi), 0x1p32, (double)w.lo);
     return fma(fmin(v, 0x1.fffffffffffffp+63), 0x1p-63, -1.0);
+}
+
+// The generators of a wave's walkers in their groups' registers (groups of four lanes): element 4 i + g is
+// register i of lane g, so that elements 156 apart share a lane.
+constexpr int MT_NR = MT_N / 4;              // registers
+constexpr int MT_SEG = 6;                    // parts in which a round of the elements is made
+constexpr int MT_RS = MT_NR / MT_SEG;        // registers and
+constexpr int MT_CH = MT_N / MT_SEG;         // elements of a part
+constexpr int MT_RP = WAVE / 4 + 2;          // an LDS row: one output of each walker, padded so that a walker's
+                                             // lanes reading rows some way apart use different banks
+static_assert(MT_NR % MT_SEG == 0 && MT_N == 2 * MT_M && MT_M % 4 == 0, "");
+
+// the state rotated so that its next index is 0 (the same generator)
+__device__ __forceinline__ void mt_load(const FastArgs &A, int64_t w, int g, U64 (&m)[MT_NR])
+{
+    const int p0 = A.mtp[w];
+#pragma unroll
+    for (int i = 0; i < MT_NR; ++i) {
+        const int k = i * 4 + g + p0;
+        m[i] = halves(A.mt[(int64_t)(k < MT_N ? k : k - MT_N) * A.W + w]);
+    }
+}
+
+// part q (a constant once unrolled) of a round: its elements by the lazy twist of mci_device.hpp's
+// mt_next, their outputs to MT_CH rows from `row` (this walker's place in the first)
+__device__ __forceinline__ void mt_part(U64 (&m)[MT_NR], int q, int g, uint64_t *row)
+{
+#pragma unroll
+    for (int j = 0; j < MT_RS; ++j) {
+        const int i = q * MT_RS + j;
+        const uint32_t here = dpp<quad(1, 2, 3, 3)>(m[i].lo), next = dpp<quad(0, 0, 0, 0)>(m[(i + 1) % MT_NR].lo);
+        m[i] = mt_twist32(m[i], g == 3 ? next : here, m[(i + MT_NR / 2) % MT_NR]);
+        row[(j * 4 + g) * MT_RP] = whole(mt_temper32(m[i]));
+    }
+}
+
+// The state back to memory, kt the next element of the round and `over` outputs made but not taken:
+// their elements go back to their values before the twist, the last first.  new = far ^ (y >> 1) ^ (odd
+// y ? A : 0) gives y (A's top bit is set), which holds the element's high 33 bits and the next element's
+// low 31.
+__device__ __forceinline__ void mt_store(const FastArgs &A, int64_t w, int g, const U64 (&m)[MT_NR], int kt, int over)
+{
+#pragma unroll
+    for (int i = 0; i < MT_NR; ++i) { A.mt[(int64_t)(i * 4 + g) * A.W + w] = whole(m[i]); }
+    __threadfence_block();
+    auto at = [&](int k) -> uint64_t & { return A.mt[(int64_t)k * A.W + w]; };
+    auto before = [&](int k) -> uint64_t {
+        const uint64_t v = at(k) ^ at(k < MT_M ? k + MT_M : k - MT_M);
+        const uint64_t odd = v >> 63;
+        return ((v ^ (odd ? 0xb5026f5aa96619e9ULL : 0ULL)) << 1) | odd;
+    };
+    for (int r = 0; r < over; r += 4) {
+        if (r + g < over) {
+            int k = kt - 1 - r - g;
+            if (k < 0) { k += MT_N; }
+            const uint64_t y = before(k), yp = before(k > 0 ? k - 1 : MT_N - 1);
+            at(k) = (y & 0xffffffff80000000ULL) | (yp & 0x7fffffffULL);
+        }
+    }
+    if (g == 0) {
+        const int k = kt - over;
+        A.mtp[w] = k < 0 ? k + MT_N : k % MT_N;
+    }
+}
+
+// Runs nsteps steps of `per` outputs each: step(row) takes them from consecutive rows (MT_RP apart) from
+// `row`.  A part's outputs go to rows LEFT .. LEFT + MT_CH - 1, after the up to per - 1 that are left over,
+// which move to the rows before LEFT, so that a step's outputs are always consecutive.
+template <int LEFT, class F>
+__device__ __forceinline__ void mt_run(const FastArgs &A, int64_t w, int g, uint64_t *mine, int per, F step)
+{
+    U64 m[MT_NR];
+    mt_load(A, w, g, m);
+    int kc = LEFT, avail = 0, kt = 0;  // row of the next output, outputs waiting, next element
+    for (int64_t done = 0; done < A.nsteps;) {
+        const int64_t stretch = A.nsteps - done < FAST_MAX_CHUNK ? A.nsteps - done : FAST_MAX_CHUNK;
+        int left = (int)stretch;
+        done += stretch;
+        while (left > 0) {
+#pragma unroll
+            for (int q = 0; q < MT_SEG; ++q) {
+                if (left > 0) {
+                    if constexpr (LEFT == 4) {
+                        if (g < avail) { mine[(LEFT - avail + g) * MT_RP] = mine[(kc + g) * MT_RP]; }
+                    }
+                    else {
+                        for (int r = g; r < avail; r += 4) { mine[(LEFT - avail + r) * MT_RP] = mine[(kc + r) * MT_RP]; }
+                    }
+                    kc = LEFT - avail;
+                    mt_part(m, q, g, mine + LEFT * MT_RP);
+                    wave_order();
+                    avail += MT_CH;
+                    kt = (q + 1) * MT_CH;
+                    while (avail >= per && left > 0) {
+                        const uint64_t *row = mine + kc * MT_RP;
+                        kc += per;
+                        avail -= per;
+                        --left;
+                        step(row);
+                    }
+                    wave_order();
+                }
+            }
+        }
+    }
+    mt_store(A, w, g, m, kt, avail);
+}
+
+// q / div, the division (a dozen FP64 instructions) left out where it changes nothing: by 1, the default
+__device__ __forceinline__ double over_div(double q, double div)
+{
+    if (div != 1.0) {
+        asm volatile("");  // a branch, not a select of the finished division
+        q = q / div;
+    }
+    return q;
 }
 
 // One walker on L lanes, S slots a lane.
@@ -264,7 +380,7 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
                 rx += rowx;
             }
             if (HSUM) {
-                const double v = q / A.x2sum_div;
+                const double v = over_div(q, A.x2sum_div);
                 Sr = Sr + v;
                 if (g == 0) { put(rs, off, v); }
                 rs += w8;
@@ -280,7 +396,7 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
 #pragma unroll
                 for (int s = 0; s < S; ++s) { sm[s] = sm[s] + x[s] * x[s]; }
             }
-            if (HSUM) { Sr = Sr + q / A.x2sum_div; }
+            if (HSUM) { Sr = Sr + over_div(q, A.x2sum_div); }
             if (HEXP) { Se = Se + e; }
             if (++inblk == B) {
                 const double norm = 1. / (double)B;
@@ -309,91 +425,16 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
     };
 
     if constexpr (MT) {
-        // The walker's generator in its lanes' registers, rotated so that its next index is 0 (the same
-        // generator): element 4 i + g in register i of lane g.  Element k + 156 then lies in the same lane.
-        constexpr int NR = MT_N / L, SEG = GROUP_SEG, RS = NR / SEG, CH = MT_N / SEG;
-        static_assert(L == 4 && NR % SEG == 0, "elements 156 apart share a lane");
-        const int p0 = A.mtp[w];
-        U64 m[NR];
+        static_assert(L == 4, "the generator's elements lie on four lanes");
+        mt_run<L * S>(A, w, g, st + wl, d + 1, [&](const uint64_t *row) {
+            U64 o[S];
+            const U64 uo = halves(row[d * MT_RP]);
 #pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            const int k = i * L + g + p0;
-            m[i] = halves(A.mt[(int64_t)(k < MT_N ? k : k - MT_N) * W + w]);
-        }
-        // The outputs wait in LDS rows of one output of each walker.  A segment's CH outputs go to rows
-        // LEFT .. LEFT + CH - 1, after the up to d that are left over, which move to the rows before LEFT,
-        // so that a step's outputs are always consecutive rows.  Rows are padded so that a read of rows S
-        // apart by a walker's lanes falls into different banks.
-        constexpr int LEFT = L * S, RP = WL + 2;
-        int kc = LEFT, avail = 0, kt = 0;  // row of the next output, outputs waiting, next element
-        int left = 0;                       // steps to do of this stretch
-        uint64_t *mine = st + wl;
-        auto steps = [&]() {
-            while (avail > d && left > 0) {
-                U64 o[S];
-                const uint64_t *row = mine + kc * RP;
-                const U64 uo = halves(row[d * RP]);
+            for (int s = 0; s < S; ++s) { o[s] = halves(row[(g * S + s) * MT_RP]); }
 #pragma unroll
-                for (int s = 0; s < S; ++s) { o[s] = halves(row[(g * S + s) * RP]); }
-                kc += d + 1;
-                avail -= d + 1;
-                --left;
-#pragma unroll
-                for (int s = 0; s < S; ++s) { propose(s, mt_symmetric(o[s])); }
-                finish(uo);
-            }
-        };
-        for (int64_t done = 0; done < A.nsteps;) {
-            const int64_t stretch = A.nsteps - done < FAST_MAX_CHUNK ? A.nsteps - done : FAST_MAX_CHUNK;
-            left = (int)stretch;
-            done += stretch;
-            while (left > 0) {
-#pragma unroll
-                for (int q = 0; q < SEG; ++q) {
-                    if (left > 0) {
-                        for (int r = g; r < avail; r += L) { mine[(LEFT - avail + r) * RP] = mine[(kc + r) * RP]; }
-                        kc = LEFT - avail;
-                        // the next CH outputs (the lazy twist of mci_device.hpp's mt_next), tempered
-#pragma unroll
-                        for (int j = 0; j < RS; ++j) {
-                            const int i = q * RS + j;
-                            const uint32_t here = dpp<quad(1, 2, 3, 3)>(m[i].lo), next = dpp<quad(0, 0, 0, 0)>(m[(i + 1) % NR].lo);
-                            m[i] = mt_twist32(m[i], g == L - 1 ? next : here, m[(i + NR / 2) % NR]);
-                            mine[(LEFT + j * L + g) * RP] = whole(mt_temper32(m[i]));
-                        }
-                        wave_order();
-                        avail += CH;
-                        kt = (q + 1) * CH;
-                        steps();
-                        wave_order();
-                    }
-                }
-            }
-        }
-        // Outputs made but not taken: their elements go back to their values before the twist, the last
-        // first.  new = far ^ (y >> 1) ^ (odd y ? A : 0) gives y (A's top bit is set), which holds the
-        // element's high 33 bits and the next element's low 31.
-#pragma unroll
-        for (int i = 0; i < NR; ++i) { A.mt[(int64_t)(i * L + g) * W + w] = whole(m[i]); }
-        __threadfence_block();
-        auto at = [&](int k) -> uint64_t & { return A.mt[(int64_t)k * W + w]; };
-        auto before = [&](int k) -> uint64_t {
-            const uint64_t v = at(k) ^ at(k < MT_M ? k + MT_M : k - MT_M);
-            const uint64_t odd = v >> 63;
-            return ((v ^ (odd ? 0xb5026f5aa96619e9ULL : 0ULL)) << 1) | odd;
-        };
-        for (int r = 0; r < avail; r += L) {
-            if (r + g < avail) {
-                int k = kt - 1 - r - g;
-                if (k < 0) { k += MT_N; }
-                const uint64_t y = before(k), yp = before(k > 0 ? k - 1 : MT_N - 1);
-                at(k) = (y & 0xffffffff80000000ULL) | (yp & 0x7fffffffULL);
-            }
-        }
-        if (g == 0) {
-            const int k = kt - avail;
-            A.mtp[w] = k < 0 ? k + MT_N : k % MT_N;
-        }
+            for (int s = 0; s < S; ++s) { propose(s, mt_symmetric(o[s])); }
+            finish(uo);
+        });
     }
     else {
         constexpr int NB = S / 2;  // the lane's Philox blocks of a step pair
@@ -456,12 +497,216 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
     }
 }
 
+// Single-coordinate moves (SRRDVecMove, veclen 1, one step size) on the reference streams, a walker on
+// four lanes of S coordinates each (d = 2^m: 4 S, or fewer with S = 1).  A step takes three outputs: the
+// coordinate (the top m bits), the proposal and the acceptance uniform; the lane that owns the coordinate
+// decides, with k_fast64's screen and arithmetic, and every lane adds its coordinates' values to their
+// per-step sums, so every number is bit-identical to the generic kernel.
+//
+// On one lane a walker (k_fast64) the sums read and wrote the walker's 16-byte records in LDS every step
+// and the outputs moved 72 bytes of generator state in HBM: 14.3 ms for 65,536 walkers x 10,240 steps at
+// d = 16 (48.9 GB at 3.4 TB/s).  Here both stay in registers: 8.9 ms, bound by instruction issue.
+template <int FL, int S>
+__global__ __launch_bounds__(WAVE, S <= 4 ? 2 : 1) void k_fast64_vec4(FastArgs A)
+{
+    constexpr bool FULL = (FL & F_FULL) != 0;
+    constexpr bool HX2 = (FL & F_X2) != 0, HSUM = (FL & F_SUM) != 0, HEXP = (FL & F_EXP) != 0;
+    constexpr bool ACC = (FL & 7) != 0 && !FULL, QN = HSUM || HEXP;
+    constexpr int L = 4, WL = WAVE / L;
+    extern __shared__ uint64_t st[];
+    const int d = A.ndim;
+    const int lane = threadIdx.x, g = lane & (L - 1), wl = lane / L;
+    const int64_t W = A.W, B = A.blocksize;
+    const int64_t w = (int64_t)blockIdx.x * WL + wl;
+    const bool live = w < W && (!A.wcount || w < *A.wcount);
+    double step = live ? A.steps[w] : 0.0;
+    if (A.pend) {
+        if (A.pend->apply && live) {
+            step = step * A.pend->fact;
+            for (int i = 0; i < d; ++i) {
+                if (step > 0.5 * A.dimsizes[i]) { step = 0.5 * A.dimsizes[i]; }
+            }
+            if (step < (double)FLT_MIN) { step = (double)FLT_MIN; }
+            if (g == 0) { A.steps[w] = step; }
+        }
+        if (A.pend->done) { return; }
+    }
+    if (!live || (A.active && !A.active[w])) { return; }
+    const int c0 = g * S;
+    const bool mine = c0 < d;  // a lane holds S coordinates or (d < 4) none
+    double x[S], q2[S], sm[S];
+    float cs[S];               // the screen's -a_i log2 e
+    uint32_t offx[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        x[s] = 0.0;
+        sm[s] = 0.0;
+        cs[s] = 0.0f;
+        if (mine) {
+            x[s] = A.x64[(int64_t)(c0 + s) * W + w];
+            cs[s] = (float)(-A.a[c0 + s] * 0x1.71547652b82fep+0);
+        }
+        q2[s] = x[s] * x[s];
+        offx[s] = (uint32_t)((mine ? c0 + s : 0) * W * 8) + (uint32_t)w * 8u;
+    }
+    const uint32_t keep = apart(g == 0 ? 0u : 0xFFFFFFFFu);
+    auto ordered = [&](const double (&v)[S]) -> double {  // as in k_fast64_grp
+        double c = 0.0;
+#pragma unroll
+        for (int ph = 0; ph < L; ++ph) {
+            if (ph > 0) { c = from_prev<L>(c, keep); }
+#pragma unroll
+            for (int s = 0; s < S; ++s) { c = c + v[s]; }
+        }
+        return from_last<L>(c, g);
+    };
+    double e = 0.0, Sr = 0.0, Se = 0.0;
+    if (HEXP) { e = exp(-(ordered(q2) / A.exp_div)); }
+    int64_t nacc = 0, inblk = 0;
+    int na = 0;  // accepted steps of the block or, without sums, of the run so far (below 2^31 by the flush)
+    char *rx = reinterpret_cast<char *>(A.d_x2), *rs = reinterpret_cast<char *>(A.d_x2sum), *re = reinterpret_cast<char *>(A.d_exp);
+    const int64_t w8 = W * 8, rowx = w8 * d;
+    const uint32_t off = (uint32_t)w * 8u;
+    auto put = [](char *row, uint32_t o, double v) { *reinterpret_cast<double *>(row + o) = v; };
+    const uint32_t ibits = (uint32_t)A.ibits, vshift = (uint32_t)A.vshift;
+    int flush = 1 << 30;
+    mt_run<4>(A, w, g, st + wl, 3, [&](const uint64_t *row) {
+        const U64 oi = halves(row[0]), op = halves(row[MT_RP]), uw = halves(row[2 * MT_RP]);
+        const uint32_t v = __builtin_amdgcn_ubfe(apart(oi.hi), vshift, ibits);
+        const int slot = (int)(v & (S - 1));
+        const bool own = v / S == (uint32_t)g;
+        double xo = x[0];
+        float cv = cs[0];
+#pragma unroll
+        for (int s = 1; s < S; ++s) {
+            xo = slot == s ? x[s] : xo;
+            cv = slot == s ? cs[s] : cv;
+        }
+        const double xn = xo + step * mt_symmetric(op);
+        const double xn2 = xn * xn, xo2 = xo * xo;
+        const float U = (float)apart(uw.hi);
+        const float F = __builtin_amdgcn_exp2f(fmaf((float)(xn2 - xo2), cv, 32.0f));
+        const float Facc = fmaf(F, 0.9999f, -3.0f), Frej = fmaf(F, 1.0001f, 1.0f);
+        bool acc = U < Facc;
+        if (__builtin_expect((__builtin_amdgcn_ballot_w64(U <= Frej) & ~__builtin_amdgcn_ballot_w64(acc) & __builtin_amdgcn_ballot_w64(own)) != 0, 0)) {
+            if (own && !acc && U <= Frej) {
+                const double av = A.a[v];
+                const double ex = xn2 * av - xo2 * av;
+                acc = (mt_canonical(whole(uw)) * 1.0) + 0.0 <= exp(-ex);
+            }
+        }
+        acc = acc && own;
+        na += acc ? 1 : 0;
+        const int to = acc ? slot : -1;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            x[s] = to == s ? xn : x[s];
+            q2[s] = to == s ? xn2 : q2[s];
+        }
+        if (--flush == 0) {
+            nacc += na;
+            na = 0;
+            flush = 1 << 30;
+        }
+        if (!(ACC || FULL)) { return; }
+        double q = 0.0;
+        if (QN) { q = ordered(q2); }
+        if (HEXP) {
+            uint32_t any = acc ? 1u : 0u;  // some lane of the group moved
+            any |= dpp<quad(1, 0, 3, 2)>(any);
+            any |= dpp<quad(2, 3, 0, 1)>(any);
+            if (any) { e = exp(-(q / A.exp_div)); }
+        }
+        if (HX2) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                sm[s] = sm[s] + q2[s];
+                if (FULL && mine) { put(rx, offx[s], q2[s]); }
+            }
+            if (FULL) { rx += rowx; }
+        }
+        if (HSUM) {
+            const double t = over_div(q, A.x2sum_div);
+            Sr = Sr + t;
+            if (FULL) {
+                if (g == 0) { put(rs, off, t); }
+                rs += w8;
+            }
+        }
+        if (HEXP) {
+            Se = Se + e;
+            if (FULL) {
+                if (g == 0) { put(re, off, e); }
+                re += w8;
+            }
+        }
+        if (ACC && ++inblk == B) {
+            const double norm = 1. / (double)B;
+            if (HX2) {
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    if (mine) { put(rx, offx[s], sm[s] * norm); }
+                    sm[s] = 0.0;
+                }
+                rx += rowx;
+            }
+            if (HSUM) {
+                if (g == 0) { put(rs, off, Sr * norm); }
+                rs += w8;
+            }
+            if (HEXP) {
+                if (g == 0) { put(re, off, Se * norm); }
+                re += w8;
+            }
+            Sr = 0.0;
+            Se = 0.0;
+            inblk = 0;
+        }
+    });
+    nacc += na;
+    // the walker's accepted steps: the sum over its lanes
+    auto plus = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        const uint64_t u = (uint64_t)nacc;
+        nacc += (int64_t)(((uint64_t)dpp<C>((uint32_t)(u >> 32)) << 32) | dpp<C>((uint32_t)u));
+    };
+    plus(std::integral_constant<int, quad(1, 0, 3, 2)>{});
+    plus(std::integral_constant<int, quad(2, 3, 0, 1)>{});
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        if (mine) {
+            A.x64[(int64_t)(c0 + s) * W + w] = x[s];
+            if (FULL && HX2 && A.s_x2) { A.s_x2[(int64_t)(c0 + s) * W + w] = sm[s]; }
+        }
+    }
+    if (g == 0) {
+        if (FULL && HSUM && A.s_x2sum) { A.s_x2sum[w] = Sr; }
+        if (FULL && HEXP && A.s_exp) { A.s_exp[w] = Se; }
+        A.acc[w] = nacc;
+        A.rej[w] = A.nsteps - nacc;
+    }
+}
+
+template <int FL>
+bool go_vec(int S, hipStream_t s, const FastArgs &A)
+{
+    const size_t sh = sizeof(uint64_t) * (4 + MT_CH) * MT_RP;
+    const dim3 grid((unsigned)((A.W + WAVE / 4 - 1) / (WAVE / 4)));
+    switch (S) {
+#define SLOTS(n)                                                                                         \
+    case n: hipLaunchKernelGGL((k_fast64_vec4<FL, n>), grid, dim3(WAVE), sh, s, A); return true;
+        SLOTS(1) SLOTS(2) SLOTS(4) SLOTS(8) SLOTS(16)
+#undef SLOTS
+    }
+    return false;
+}
+
 template <int FL, int L, int S>
 void go(hipStream_t s, const FastArgs &A)
 {
     constexpr int WL = WAVE / L;
     constexpr bool MT = (FL & F_MT) != 0;
-    const size_t sh = MT ? sizeof(uint64_t) * (L * S + MT_N / GROUP_SEG) * (WL + 2) : 0;
+    const size_t sh = MT ? sizeof(uint64_t) * (L * S + MT_CH) * MT_RP : 0;
     const dim3 grid((unsigned)((A.W + WL - 1) / WL));
     if constexpr (MT && (S & (S - 1)) == 0) {
         if (A.ndim == L * S) {
@@ -490,12 +735,12 @@ bool go_shape(int L, int S, hipStream_t s, const FastArgs &A)
 // this file is compiled once for each part of the forms (the build defines GROUP_PART)
 #define GROUP_NAME2(n) launch_group_##n
 #define GROUP_NAME(n) GROUP_NAME2(n)
-bool GROUP_NAME(GROUP_PART)(int fl, int L, int S, const FastArgs &A, hipStream_t s)
+bool GROUP_NAME(GROUP_PART)(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s)
 {
     switch (fl) {
 #define FORM(f)                                                                                          \
-    case f: return go_shape<f>(L, S, s, A);                                                             \
-    case f + F_MT: return go_shape<f + F_MT>(L, S, s, A);
+    case f: return !vec && go_shape<f>(L, S, s, A);                                                     \
+    case f + F_MT: return vec ? go_vec<f + F_MT>(S, s, A) : go_shape<f + F_MT>(L, S, s, A);
 #if GROUP_PART == 0
         FORM(0) FORM(1)
 #elif GROUP_PART == 1

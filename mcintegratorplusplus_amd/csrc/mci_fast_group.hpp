@@ -1,5 +1,5 @@
-// mci_fast_group.hpp — launch interface of the all-coordinate kernel with a walker on a group of
-// lanes (mci_fast_group.hip).
+// mci_fast_group.hpp — launch interface of the kernels with a walker on a group of lanes
+// (mci_fast_group.hip).
 #pragma once
 
 #include <cstdint>
@@ -64,18 +64,27 @@ inline bool group_shape(bool mt, int d, int64_t W, int &L, int &S)
     return bestL != 0 && d > 16;  // up to 16 coordinates one lane holds the walker
 }
 
-// one launch of kernel form fl (the F_* flags of mci_fast_dev.hpp); false: there is no such form
-bool launch_group_0(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_1(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_2(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_3(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_4(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_5(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-bool launch_group_6(int fl, int L, int S, const FastArgs &A, hipStream_t s);
-inline bool launch_group(int fl, int L, int S, const FastArgs &A, hipStream_t s)
+// The slots a lane for single-coordinate moves over d = 2^m coordinates on the reference streams (groups of
+// four lanes, up to 64 coordinates); false: the walker runs on one lane
+inline bool group_slots_vec(int d, int64_t W, int &S)
 {
-    return launch_group_0(fl, L, S, A, s) || launch_group_1(fl, L, S, A, s) || launch_group_2(fl, L, S, A, s) ||
-           launch_group_3(fl, L, S, A, s) || launch_group_4(fl, L, S, A, s) || launch_group_5(fl, L, S, A, s) ||
-           launch_group_6(fl, L, S, A, s);
+    S = d > 4 ? d / 4 : 1;
+    return d <= 64 && (d & (d - 1)) == 0 && W * (int64_t)d < (int64_t)1 << 29;
+}
+
+// one launch of kernel form fl (the F_* flags of mci_fast_dev.hpp, without F_P2; vec: single-coordinate
+// moves); false: there is no such form
+bool launch_group_0(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_1(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_2(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_3(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_4(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_5(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+bool launch_group_6(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);
+inline bool launch_group(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s)
+{
+    return launch_group_0(fl, vec, L, S, A, s) || launch_group_1(fl, vec, L, S, A, s) || launch_group_2(fl, vec, L, S, A, s) ||
+           launch_group_3(fl, vec, L, S, A, s) || launch_group_4(fl, vec, L, S, A, s) || launch_group_5(fl, vec, L, S, A, s) ||
+           launch_group_6(fl, vec, L, S, A, s);
 }
 } // namespace mcid

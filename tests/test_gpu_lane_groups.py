@@ -1,5 +1,5 @@
-"""The all-coordinate kernel with a walker on a group of lanes against the generic kernel, at the edges
-of its forms: the smallest and largest dimensions of each (lanes, slots), walker counts that leave a
+"""The kernels with a walker on a group of lanes (all-coordinate moves; single-coordinate moves on the
+reference streams) against the generic kernel, at the edges of their forms: the smallest and largest dimensions of each (lanes, slots), walker counts that leave a
 ragged last wave or call for two, four or eight lanes, odd step counts (a step pair cut, generator
 outputs left over), and launches that continue the streams.  Every number is bit-identical."""
 import numpy as np
@@ -17,18 +17,29 @@ NATIVE = [(1, 33), (3, 70), (4, 70), (7, 70), (8, 16), (15, 64), (16, 5), (23, 7
           (18, 33000), (35, 17000), (40, 17000)]
 REFERENCE = [(1, 1), (2, 21), (4, 70), (5, 70), (8, 33), (9, 70), (12, 16), (13, 70), (16, 70), (17, 70), (24, 21), (25, 21), (32, 33),
              (33, 21), (48, 21), (49, 21), (51, 21), (63, 21), (64, 33), (65, 5)]
+SINGLE = [(1, 5), (2, 21), (4, 70), (8, 33), (16, 70), (32, 16), (64, 21), (128, 5)]  # 128: one lane a walker
 ALL_OBS = [OBS_X2, OBS_X2_SUM, OBS_EXP_X2]
 
 
 @pytest.mark.parametrize("rng,d,W", [(RNG_PHILOX, *c) for c in NATIVE] + [(RNG_MT, *c) for c in REFERENCE])
 def test_walker_on_a_group_of_lanes(rng, d, W):
-    print("lane groups", rng, d, W, flush=True)
-    blocksize = (3, 1, 0)[d % 3]
     obs = [[OBS_X2], [OBS_X2_SUM], ALL_OBS, [OBS_X2, OBS_X2_SUM], [OBS_EXP_X2], [OBS_X2, OBS_EXP_X2]][d % 6]
+    check(rng, d, W, 0, (3, 1, 0)[d % 3], obs)
+
+
+@pytest.mark.parametrize("obs", [[OBS_X2], ALL_OBS], ids=["x2", "all"])
+@pytest.mark.parametrize("blocksize", [0, 1, 3])
+@pytest.mark.parametrize("d,W", SINGLE)
+def test_single_coordinate_moves_on_a_group_of_lanes(d, W, blocksize, obs):
+    check(RNG_MT, d, W, 1, blocksize, obs)
+
+
+def check(rng, d, W, veclen, blocksize, obs):
+    print("lane groups", rng, d, W, veclen, blocksize, obs, flush=True)
     est = ESTIM_NOOP if blocksize == 0 else ESTIM_MJ
     sig = np.random.default_rng(d).uniform(0.5, 2.0, d)
-    pdf = (PDF_GAUSS_ISO, []) if d % 4 == 1 else (PDF_GAUSS_DIAG, 0.5 / sig ** 2)
-    cfg = dict(ndim=d, seed=77 + d, ndecorr=37, move=(0, 0, 1, None), pdfs=[pdf],
+    pdf = (PDF_GAUSS_ISO, []) if d % 4 == 1 and veclen == 0 else (PDF_GAUSS_DIAG, 0.5 / sig ** 2)
+    cfg = dict(ndim=d, seed=77 + d, ndecorr=37, move=(0, veclen, 1, None), pdfs=[pdf],
                obs=[(k, [], blocksize, 1, 0, est) for k in obs])
     n1 = 64 * max(blocksize, 1) if blocksize else 151
     out = {}

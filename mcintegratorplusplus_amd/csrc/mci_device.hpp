@@ -105,6 +105,28 @@ struct Chain
 
 __device__ __forceinline__ double &at(double *p, int64_t W, int i, int64_t w) { return p[(int64_t)i * W + w]; }
 
+// A walker's state as its kernel holds it: the wave's LDS columns, or the chain's columns in HBM
+struct Views
+{
+    MciVec xo, xn;  // xold, xnew [ndim]
+    MciVec po, pn;  // pold, pnew [nproto]
+    MciVec ov;      // last observable values [nobsdim]
+    MciVec sums;    // LDS kernels: running block sums [nobsdim]
+    int *cnt;       // LDS kernels: per observable, steps since its last evaluation, then evaluations in its
+    int cs;         // block ([2 nobs], elements cs apart)
+};
+
+// element i of parameters that nothing writes while a kernel runs: constant memory, so that an index the
+// wave shares is one scalar load (a vector load each of the means, weights and bounds a step reads, each
+// waited for, took most of the step)
+__device__ __forceinline__ double param(const double *p, int i)
+{
+    return reinterpret_cast<const __attribute__((address_space(4))) double *>(reinterpret_cast<uintptr_t>(p))[i];
+}
+
+__device__ __forceinline__ MciVec column(double *p, int64_t W, int64_t w) { return MciVec{p + w, W}; }
+__device__ __forceinline__ MciVec rows_from(const MciVec &v, int i) { return MciVec{v.p + (int64_t)i * v.s, v.s}; }
+
 // --------------------------------------------------------------------------
 // random streams
 // --------------------------------------------------------------------------
@@ -112,12 +134,17 @@ struct Lane
 {
     int64_t w;
     int32_t mtp;       // MT: next index
+    uint64_t m0, m1, mm; // MT: elements mtp, mtp + 1, mtp + 156 (mod 312)
     uint64_t t;        // Philox: step counter
     uint32_t k, kx;    // Philox: word index within the step, extra-word index
+    uint32_t b0[4], bk[4];  // Philox: block 0 of step pair b0t, block bkn of step pair bkt
+    uint64_t b0t, bkt;
+    uint32_t bkn;
     int nchanged;      // changed coordinates [cfirst, cfirst + nchanged) (== ndim: all)
     int cfirst;
     bool accepted;
     int64_t acc, rej;
+    double st0;        // the step size of type 0
     double sv[2];      // saved normals of the move's distribution (nsv)
     int sf;            // their availability bits (nsf)
 };
@@ -142,18 +169,29 @@ __device__ __forceinline__ uint64_t mt_temper(uint64_t z)
     return z;
 }
 
-__device__ __forceinline__ uint64_t mt_next(const Chain &c, Lane &L)
+// the elements the next output is made from (Lane::m0, m1, mm), read an output ahead: their latency would
+// otherwise be part of every draw
+template <class C>
+__device__ __forceinline__ void mt_ahead(const C &c, Lane &L)
 {
     const int64_t W = c.W;
     const int k = L.mtp;
     const int k1 = (k + 1 == MT_N) ? 0 : k + 1;
     const int km = (k < MT_N - MT_M) ? k + MT_M : k + MT_M - MT_N;
-    const uint64_t xk = c.mt[(int64_t)k * W + L.w];
-    const uint64_t xk1 = c.mt[(int64_t)k1 * W + L.w];
-    const uint64_t xkm = c.mt[(int64_t)km * W + L.w];
-    const uint64_t nv = mt_twist(xk, xk1, xkm);
+    L.m1 = c.mt[(int64_t)k1 * W + L.w];
+    L.mm = c.mt[(int64_t)km * W + L.w];
+}
+
+template <class C>
+__device__ __forceinline__ uint64_t mt_next(const C &c, Lane &L)
+{
+    const int64_t W = c.W;
+    const int k = L.mtp;
+    const uint64_t nv = mt_twist(L.m0, L.m1, L.mm);
     c.mt[(int64_t)k * W + L.w] = nv;
-    L.mtp = k1;
+    L.mtp = (k + 1 == MT_N) ? 0 : k + 1;
+    L.m0 = L.m1;
+    mt_ahead(c, L);
     return mt_temper(nv);
 }
 
@@ -182,16 +220,39 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 // (draw_accept); the move's draws start at word 1.  Side streams keyed by the step itself: Lemire
 // rejections (block 0x20000000 + kx / 4, word kx mod 4) and the acceptance uniform's low word
 // (block 0x30000000, word 0).
-__device__ __forceinline__ uint32_t ph_block_word(const Chain &c, const Lane &L, uint32_t blk, uint64_t ct, uint32_t word)
+template <class C>
+__device__ __forceinline__ uint32_t ph_block_word(const C &c, const Lane &L, uint32_t blk, uint64_t ct, uint32_t word)
 {
     uint32_t o[4];
     philox4x32_10(blk, (uint32_t)L.w, (uint32_t)ct, (uint32_t)(ct >> 32), c.key0, c.key1, o);
     return o[word];
 }
 
-__device__ __forceinline__ uint32_t ph_word(const Chain &c, const Lane &L, uint32_t k)
+// main word k of the step; a block's words serve until the next block is needed, and block 0 (the shared
+// word and the first draw of both steps of a pair) for the whole pair
+template <class C>
+__device__ __forceinline__ uint32_t ph_word(const C &c, Lane &L, uint32_t k)
 {
-    return ph_block_word(c, L, k >> 1, L.t >> 1, 2u * (uint32_t)(L.t & 1u) + (k & 1u));
+    const uint64_t pair = L.t >> 1;
+    const uint32_t j = k >> 1;
+    uint32_t w0, w1, w2, w3;
+    if (j == 0) {
+        if (L.b0t != pair) {
+            philox4x32_10(0u, (uint32_t)L.w, (uint32_t)pair, (uint32_t)(pair >> 32), c.key0, c.key1, L.b0);
+            L.b0t = pair;
+        }
+        w0 = L.b0[0]; w1 = L.b0[1]; w2 = L.b0[2]; w3 = L.b0[3];
+    }
+    else {
+        if (L.bkt != pair || L.bkn != j) {
+            philox4x32_10(j, (uint32_t)L.w, (uint32_t)pair, (uint32_t)(pair >> 32), c.key0, c.key1, L.bk);
+            L.bkt = pair;
+            L.bkn = j;
+        }
+        w0 = L.bk[0]; w1 = L.bk[1]; w2 = L.bk[2]; w3 = L.bk[3];
+    }
+    const uint32_t a = (k & 1u) ? w1 : w0, b = (k & 1u) ? w3 : w2;
+    return (L.t & 1u) ? b : a;
 }
 
 __device__ __forceinline__ void step_begin(Lane &L) { L.k = 1; L.kx = 0; }
@@ -206,7 +267,8 @@ __device__ __forceinline__ double canonical53(uint64_t w)
 }
 
 // symmetric uniform on (-1,1) (TrialMoveInterface.hpp:120-124): (u*(b-a)) + a
-__device__ __forceinline__ double draw_sym(const Chain &c, Lane &L)
+template <class C>
+__device__ __forceinline__ double draw_sym(const C &c, Lane &L)
 {
     if (c.rng == MCI_RNG_MT19937_64) {
         const double u = canonical53(mt_next(c, L));
@@ -217,7 +279,8 @@ __device__ __forceinline__ double draw_sym(const Chain &c, Lane &L)
 }
 
 // uniform on [0,1) (MCIntegrator.cpp:343 acceptance draw; :365 random moves)
-__device__ __forceinline__ double draw_unit(const Chain &c, Lane &L)
+template <class C>
+__device__ __forceinline__ double draw_unit(const C &c, Lane &L)
 {
     if (c.rng == MCI_RNG_MT19937_64) {
         const double u = canonical53(mt_next(c, L));
@@ -232,12 +295,17 @@ __device__ __forceinline__ double draw_unit(const Chain &c, Lane &L)
 // move over 2^m vectors (c.ibits = m <= 11) the shared word's top m bits are the move's index and
 // u = ((shared word : side-stream word) << m) >> 11, times 2^-53 (the m zero bits shifted in fall
 // below the 53 kept); otherwise m = 0.
-__device__ __forceinline__ double draw_accept(const Chain &c, Lane &L)
+// accept(r): u <= r.  The shared word fixes all but 32 of the uniform's bits, so the side stream's word is
+// drawn only where r lies between the smallest and the largest u with them.
+__device__ __forceinline__ bool draw_accept(const Chain &c, Lane &L, double r)
 {
-    if (c.rng == MCI_RNG_MT19937_64) { return draw_unit(c, L); }
+    if (c.rng == MCI_RNG_MT19937_64) { return draw_unit(c, L) <= r; }
     const uint32_t m = c.ibits > 0 ? (uint32_t)c.ibits : 0u;
-    const uint64_t hi = ph_word(c, L, 0), lo = ph_block_word(c, L, 0x30000000u, L.t, 0);
-    return (double)((((hi << 32) | lo) << m) >> 11) * 0x1p-53;
+    const uint64_t hi = (uint64_t)ph_word(c, L, 0) << 32;
+    auto u = [&](uint64_t lo) { return (double)(((hi | lo) << m) >> 11) * 0x1p-53; };
+    if (r < u(0u)) { return false; }
+    if (r >= u(0xFFFFFFFFu)) { return true; }
+    return u(ph_block_word(c, L, 0x30000000u, L.t, 0)) <= r;
 }
 
 // uniform integer on [0, n) (SRRDVecMove.hpp:78): Lemire's method as in libstdc++
@@ -282,7 +350,8 @@ __device__ __forceinline__ int draw_index(const Chain &c, Lane &L, int n)
 // the value (SymmetrizedPRRD, TrialMoveInterface.hpp:80-98).  With the reference stream the
 // draws are the reference's up to the last place of the device's log, tan, pow and exp.
 // --------------------------------------------------------------------------
-__device__ inline double nd_draw(const Chain &c, Lane &L, int s)
+template <class C>
+__device__ inline double nd_draw(const C &c, Lane &L, int s)
 {
     double ret;
     if (L.sf & (1 << s)) {
@@ -304,7 +373,8 @@ __device__ inline double nd_draw(const Chain &c, Lane &L, int s)
     return ret * 1.0 + 0.0;
 }
 
-__device__ inline double gamma_draw(const Chain &c, Lane &L, int s, double alpha, double beta)
+template <class C>
+__device__ inline double gamma_draw(const C &c, Lane &L, int s, double alpha, double beta)
 {
     const double malpha = alpha < 1.0 ? alpha + 1.0 : alpha;
     const double a1 = malpha - 1.0 / 3.0;
@@ -323,11 +393,21 @@ __device__ inline double gamma_draw(const Chain &c, Lane &L, int s, double alpha
     return pow(u, 1.0 / alpha) * a1 * v * beta;
 }
 
-__device__ inline double srrd_draw(const Chain &c, Lane &L)
+// what a draw needs of the chain
+struct Streams
+{
+    int rng, srrd;
+    uint32_t key0, key1;
+    uint64_t *mt;
+    int64_t W;
+};
+
+// the distributions other than the uniform one, in a function of their own: inlined at every draw they
+// made the step kernels larger than the instruction cache
+__device__ __noinline__ double srrd_draw_other(const Streams c, Lane &L)
 {
     double val;
     switch (c.srrd) {
-    case MCI_SRRD_UNIFORM: return draw_sym(c, L);
     case MCI_SRRD_GAUSSIAN: return nd_draw(c, L, 0);
     case MCI_SRRD_STUDENT: {
         const double z = nd_draw(c, L, 0);
@@ -354,107 +434,115 @@ __device__ inline double srrd_draw(const Chain &c, Lane &L)
     return ((draw_unit(c, L) - 0.0) < 0.5 * (1.0 - 0.0)) ? val : -val;
 }
 
+__device__ __forceinline__ double srrd_draw(const Chain &c, Lane &L)
+{
+    if (c.srrd == MCI_SRRD_UNIFORM) { return draw_sym(c, L); }
+    Lane other = L;  // a copy, so that L itself stays in registers
+    const double v = srrd_draw_other(Streams{c.rng, c.srrd, c.key0, c.key1, c.mt, c.W}, other);
+    L = other;
+    return v;
+}
+
 // --------------------------------------------------------------------------
 // sampling functions (device functors; arithmetic of include/mci_amd.h)
 // --------------------------------------------------------------------------
-__device__ __forceinline__ double pdf_a(const PdfDev &p, int i) { return p.a ? p.a[i] : 1.0; }
+__device__ __forceinline__ double pdf_a(const PdfDev &p, int i) { return p.a ? param(p.a, i) : 1.0; }
 
-__device__ inline double gmm_logp(const Chain &c, const PdfDev &p, const double *pv, int64_t W, int64_t w)
+__device__ __forceinline__ double gmm_logp(const PdfDev &p, const MciVec &q)
 {
     double m = -__builtin_huge_val();
     for (int k = 0; k < p.K; ++k) {
-        const double t = p.gc[k] - p.gb[k] * pv[(int64_t)k * W + w];
+        const double t = param(p.gc, k) - param(p.gb, k) * q[k];
         if (t > m) { m = t; }
     }
     double s = 0.0;
-    for (int k = 0; k < p.K; ++k) { s = s + exp((p.gc[k] - p.gb[k] * pv[(int64_t)k * W + w]) - m); }
+    for (int k = 0; k < p.K; ++k) { s = s + exp((param(p.gc, k) - param(p.gb, k) * q[k]) - m); }
     return m + log(s);
 }
 
-// protoFunction(x) -> proto values (written to pv + p.off rows)
-__device__ inline void pdf_proto(const Chain &c, const PdfDev &p, const double *x, double *pv, int64_t w)
+// protoFunction(x) -> proto values q
+__device__ __forceinline__ void pdf_proto(const Chain &c, const PdfDev &p, const MciVec &x, const MciVec &q)
 {
-    const int64_t W = c.W;
-    double *q = pv + (int64_t)p.off * W;
     switch (p.kind) {
     case MCI_PDF_GAUSS_ISO: {
-        double s = x[w] * x[w];
-        for (int i = 1; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; s = s + v * v; }
-        q[w] = s;
+        double s = x[0] * x[0];
+#pragma unroll 4
+        for (int i = 1; i < c.ndim; ++i) { const double v = x[i]; s = s + v * v; }
+        q[0] = s;
         break;
     }
     case MCI_PDF_GAUSS_DIAG:
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; q[(int64_t)i * W + w] = (v * v) * pdf_a(p, i); }
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; q[i] = (v * v) * pdf_a(p, i); }
         break;
     case MCI_PDF_EXP_DIAG:
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; q[(int64_t)i * W + w] = fabs(v) * pdf_a(p, i); }
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; q[i] = fabs(v) * pdf_a(p, i); }
         break;
     case MCI_PDF_GMM_ISO:
         for (int k = 0; k < p.K; ++k) {
             double s = 0.0;
-            for (int i = 0; i < c.ndim; ++i) { const double d = x[(int64_t)i * W + w] - p.gmu[k * c.ndim + i]; s = s + d * d; }
-            q[(int64_t)k * W + w] = s;
+#pragma unroll 4
+            for (int i = 0; i < c.ndim; ++i) { const double d = x[i] - param(p.gmu, k * c.ndim + i); s = s + d * d; }
+            q[k] = s;
         }
-        q[(int64_t)p.K * W + w] = gmm_logp(c, p, q, W, w);
+        q[p.K] = gmm_logp(p, q);
         break;
 #ifdef MCI_RTC_USER
     case MCI_PDF_DEVICE: // the caller's protoFunction (built at run time with the functor's source)
-        mci_user_pdf_proto(p.uid, c.ndim, MciVec{const_cast<double *>(x) + w, W}, p.a, MciVec{q + w, W});
+        mci_user_pdf_proto(p.uid, c.ndim, x, p.a, q);
         break;
 #endif
     }
 }
 
-__device__ inline double pdf_acceptance(const Chain &c, const PdfDev &p, const double *pold, const double *pnew, int64_t w)
+__device__ __forceinline__ double pdf_acceptance(const PdfDev &p, const MciVec &po, const MciVec &pn)
 {
-    const int64_t W = c.W;
-    const double *po = pold + (int64_t)p.off * W;
-    const double *pn = pnew + (int64_t)p.off * W;
     switch (p.kind) {
     case MCI_PDF_GAUSS_ISO:
-        return exp(-pn[w] + po[w]);
+        return exp(-pn[0] + po[0]);
     case MCI_PDF_GAUSS_DIAG:
     case MCI_PDF_EXP_DIAG: {
         double e = 0.0;
-        for (int i = 0; i < p.nproto; ++i) { e = e + po[(int64_t)i * W + w]; }
+#pragma unroll 4
+        for (int i = 0; i < p.nproto; ++i) { e = e + po[i]; }
         double s = 0.0;
-        for (int i = 0; i < p.nproto; ++i) { s = s + pn[(int64_t)i * W + w]; }
+#pragma unroll 4
+        for (int i = 0; i < p.nproto; ++i) { s = s + pn[i]; }
         e = e - s;
         return exp(e);
     }
     case MCI_PDF_GMM_ISO:
-        return exp(pn[(int64_t)p.K * W + w] - po[(int64_t)p.K * W + w]);
+        return exp(pn[p.K] - po[p.K]);
 #ifdef MCI_RTC_USER
     case MCI_PDF_DEVICE: // the caller's acceptanceFunction
-        return mci_user_pdf_acceptance(p.uid, p.nproto, MciVec{const_cast<double *>(po) + w, W}, MciVec{const_cast<double *>(pn) + w, W}, p.a);
+        return mci_user_pdf_acceptance(p.uid, p.nproto, po, pn, p.a);
 #endif
     }
     return 0.0;
 }
 
-// SamplingFunctionInterface::computeAcceptance (+ the updatedAcceptance of each kind)
-__device__ inline double pdf_compute_acceptance(const Chain &c, const PdfDev &p, const Lane &L, double *pold, double *pnew)
+// SamplingFunctionInterface::computeAcceptance (+ the updatedAcceptance of each kind) from positions xo, xn
+// and the chain's proto values pold, pnew
+__device__ __forceinline__ double pdf_compute_acceptance(const Chain &c, const PdfDev &p, const Lane &L, const MciVec &xo, const MciVec &xn,
+                                                         const MciVec &pold, const MciVec &pnew)
 {
-    const int64_t W = c.W, w = L.w;
+    const MciVec po = rows_from(pold, p.off), pn = rows_from(pnew, p.off);
 #ifdef MCI_RTC_USER
     // the caller's updatedAcceptance when it defines one (else its protoFunction and
     // acceptanceFunction, the interface's default), for the changed coordinates
     if (p.kind == MCI_PDF_DEVICE && L.nchanged < c.ndim) {
-        double *po = pold + (int64_t)p.off * W + w, *pn = pnew + (int64_t)p.off * W + w;
-        return mci_user_pdf_updated(p.uid, c.ndim, p.nproto, MciVec{c.xnew + w, W}, MciChanged{L.cfirst, L.nchanged}, MciVec{po, W},
-                                    MciVec{pn, W}, p.a);
+        return mci_user_pdf_updated(p.uid, c.ndim, p.nproto, xn, MciChanged{L.cfirst, L.nchanged}, po, pn, p.a);
     }
 #endif
     if (L.nchanged < c.ndim) {
-        double *po = pold + (int64_t)p.off * W;
-        double *pn = pnew + (int64_t)p.off * W;
         if (p.kind == MCI_PDF_GAUSS_DIAG || p.kind == MCI_PDF_EXP_DIAG) {
             double e = 0.0;
             for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
-                const double v = c.xnew[(int64_t)j * W + w];
+                const double v = xn[j];
                 const double f = (p.kind == MCI_PDF_GAUSS_DIAG) ? (v * v) * pdf_a(p, j) : fabs(v) * pdf_a(p, j);
-                pn[(int64_t)j * W + w] = f;
-                e = e + (f - po[(int64_t)j * W + w]);
+                pn[j] = f;
+                e = e + (f - po[j]);
             }
             return exp(-e);
         }
@@ -462,36 +550,35 @@ __device__ inline double pdf_compute_acceptance(const Chain &c, const PdfDev &p,
             for (int k = 0; k < p.K; ++k) {
                 double dr = 0.0;
                 for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
-                    const double mu = p.gmu[k * c.ndim + j];
-                    const double dn = c.xnew[(int64_t)j * W + w] - mu, dd = c.xold[(int64_t)j * W + w] - mu;
+                    const double mu = param(p.gmu, k * c.ndim + j);
+                    const double dn = xn[j] - mu, dd = xo[j] - mu;
                     dr = dr + (dn * dn - dd * dd);
                 }
-                pn[(int64_t)k * W + w] = po[(int64_t)k * W + w] + dr;
+                pn[k] = po[k] + dr;
             }
-            pn[(int64_t)p.K * W + w] = gmm_logp(c, p, pn, W, w);
-            return exp(pn[(int64_t)p.K * W + w] - po[(int64_t)p.K * W + w]);
+            pn[p.K] = gmm_logp(p, pn);
+            return exp(pn[p.K] - po[p.K]);
         }
     }
-    pdf_proto(c, p, c.xnew, pnew, w);
-    return pdf_acceptance(c, p, pold, pnew, w);
+    pdf_proto(c, p, xn, pn);
+    return pdf_acceptance(p, po, pn);
 }
 
 // samplingFunction(proto values) of each kind (exp of minus the proto sum, or of the mixture's log p)
-__device__ inline double pdf_value(const Chain &c, const PdfDev &p, const double *pv, int64_t w)
+__device__ __forceinline__ double pdf_value(const PdfDev &p, const MciVec &pv)
 {
-    const int64_t W = c.W;
-    const double *q = pv + (int64_t)p.off * W;
+    const MciVec q = rows_from(pv, p.off);
     switch (p.kind) {
-    case MCI_PDF_GAUSS_ISO: return exp(-q[w]);
+    case MCI_PDF_GAUSS_ISO: return exp(-q[0]);
     case MCI_PDF_GAUSS_DIAG:
     case MCI_PDF_EXP_DIAG: {
         double s = 0.0;
-        for (int i = 0; i < p.nproto; ++i) { s = s + q[(int64_t)i * W + w]; }
+        for (int i = 0; i < p.nproto; ++i) { s = s + q[i]; }
         return exp(-s);
     }
-    case MCI_PDF_GMM_ISO: return exp(q[(int64_t)p.K * W + w]);
+    case MCI_PDF_GMM_ISO: return exp(q[p.K]);
 #ifdef MCI_RTC_USER
-    case MCI_PDF_DEVICE: return mci_user_pdf_sampling(p.uid, p.nproto, MciVec{const_cast<double *>(q) + w, W}, p.a);
+    case MCI_PDF_DEVICE: return mci_user_pdf_sampling(p.uid, p.nproto, q, p.a);
 #endif
     }
     return 0.0;
@@ -505,7 +592,9 @@ __device__ inline double pdf_value(const Chain &c, const PdfDev &p, const double
 // reduced with fmod so every loop is bounded; non-finite coordinates are left unchanged.
 __device__ __forceinline__ void wrap(const Chain &c, int i, double &x)
 {
-    const double lo = c.lb[i], hi = c.ub[i], len = hi - lo;
+    const double lo = param(c.lb, i), hi = param(c.ub, i);
+    if (x >= lo && x <= hi) { return; }
+    const double len = hi - lo;
     if (!isfinite(x)) { return; }
     if (x < lo - 64.0 * len || x > hi + 64.0 * len) {
         double r = fmod(x - lo, len);
@@ -521,16 +610,35 @@ __device__ __forceinline__ void wrap(const Chain &c, int i, double &x)
 // the Metropolis step
 // --------------------------------------------------------------------------
 // SRRDAllMove / SRRDVecMove trial moves (uniform SRRD)
-__device__ inline double srrd_move(const Chain &c, Lane &L, bool outer)
+__device__ __forceinline__ double srrd_move(const Chain &c, Lane &L, const MciVec &xn, bool outer)
 {
     const int64_t W = c.W, w = L.w;
+    if (c.movetype == MCI_MOVE_ALL && c.ntypes == 1 && c.srrd == MCI_SRRD_UNIFORM && c.rng == MCI_RNG_PHILOX && L.k == 1) {
+        // the step's first draws, word i + 1 for coordinate i: a block is two coordinates (drawn one by
+        // one, the choice of block, word and distribution cost more branches than the blocks themselves)
+        auto sym = [](uint32_t v) { return (double)(2 * (int64_t)v + 1 - 4294967296LL) * 0x1p-32; };
+        const double st = L.st0;
+        xn[0] = xn[0] + st * sym(ph_word(c, L, 1));
+        const uint64_t pair = L.t >> 1;
+        const bool odd = (L.t & 1u) != 0;
+        for (int i = 1; i < c.ndim; i += 2) {
+            uint32_t o[4];
+            philox4x32_10((uint32_t)(i + 1) >> 1, (uint32_t)w, (uint32_t)pair, (uint32_t)(pair >> 32), c.key0, c.key1, o);
+            xn[i] = xn[i] + st * sym(odd ? o[2] : o[0]);
+            if (i + 1 < c.ndim) { xn[i + 1] = xn[i + 1] + st * sym(odd ? o[3] : o[1]); }
+        }
+        L.k += (uint32_t)c.ndim;
+        L.nchanged = c.ndim;
+        L.cfirst = 0;
+        return 1.;
+    }
     if (c.movetype == MCI_MOVE_ALL) {
         int xidx = 0;
         for (int t = 0; t < c.ntypes; ++t) {
-            const double st = c.steps[(int64_t)t * W + w];
+            const double st = t == 0 ? L.st0 : c.steps[(int64_t)t * W + w];
             while (xidx < c.typeEnds[t]) {
-                double &xn = c.xnew[(int64_t)xidx * W + w];
-                xn = xn + st * srrd_draw(c, L);
+                double &v = xn[xidx];
+                v = v + st * srrd_draw(c, L);
                 ++xidx;
             }
         }
@@ -547,10 +655,11 @@ __device__ inline double srrd_move(const Chain &c, Lane &L, bool outer)
         if (xidx < c.typeEnds[t]) { break; }
         ++t;
     }
-    const double st = c.steps[(int64_t)t * W + w];
+    double st = L.st0;
+    if (t > 0) { st = c.steps[(int64_t)t * W + w]; }
     for (int i = 0; i < c.veclen; ++i) {
-        double &xn = c.xnew[(int64_t)(xidx + i) * W + w];
-        xn = xn + st * srrd_draw(c, L);
+        double &v = xn[xidx + i];
+        v = v + st * srrd_draw(c, L);
     }
     L.nchanged = c.veclen;
     L.cfirst = xidx;
@@ -559,29 +668,28 @@ __device__ inline double srrd_move(const Chain &c, Lane &L, bool outer)
 
 // the state the reference's callback sees (MCIntegrator.cpp:265, 346-347, 373): walker 0's committed
 // position and its counters, recorded for the host to replay the calls in order
-__device__ inline void cb_record(const Chain &c, const Lane &L)
+__device__ __forceinline__ void cb_record(const Chain &c, const Lane &L, const Views &V)
 {
     if (c.cb_buf == nullptr || L.w != 0) { return; }
     const int64_t n = c.cb_n[0];
     if (n < c.cb_cap) {
         double *r = c.cb_buf + n * (c.ndim + 2);
-        for (int i = 0; i < c.ndim; ++i) { r[i] = c.xold[(int64_t)i * c.W]; }
+        for (int i = 0; i < c.ndim; ++i) { r[i] = V.xo[i]; }
         r[c.ndim] = (double)L.acc;
         r[c.ndim + 1] = (double)L.rej;
     }
     c.cb_n[0] = n + 1;
 }
 
-// log q(y) of the independence mixture at column w of y [ndim][W]: the log-sum-exp over components of
+// log q(y) of the independence mixture at y: the log-sum-exp over components of
 // lc_k - |(y - mu_k) / sigma_k|^2 / 2
-__device__ inline double lm_logq(const Chain &c, const double *y, int64_t w)
+__device__ inline double lm_logq(const Chain &c, const MciVec &y)
 {
-    const int64_t W = c.W;
     double e[8], mx = -__builtin_huge_val();
     for (int k = 0; k < c.lm_K; ++k) {
         double s = 0.0;
         for (int j = 0; j < c.ndim; ++j) {
-            const double z = (y[(int64_t)j * W + w] - c.lm_mu[k * c.ndim + j]) * c.lm_isig[k * c.ndim + j];
+            const double z = (y[j] - c.lm_mu[k * c.ndim + j]) * c.lm_isig[k * c.ndim + j];
             s = s + z * z;
         }
         e[k] = c.lm_lc[k] - 0.5 * s;
@@ -597,9 +705,8 @@ __device__ inline double lm_logq(const Chain &c, const double *y, int64_t w)
 // sigma_k z for every coordinate; the move's acceptance factor q(x) / q(x') (the reference's
 // trial-move hook, TrialMoveInterface.hpp:63-69, MCIntegrator.cpp:343), so that the chain keeps the
 // target exact whatever the mixture is.
-__device__ inline double lm_move(const Chain &c, Lane &L)
+__device__ inline double lm_move(const Chain &c, Lane &L, const Views &V)
 {
-    const int64_t W = c.W, w = L.w;
     const double uc = draw_unit(c, L);
     int k = c.lm_K - 1;
     for (int kk = 0; kk < c.lm_K - 1; ++kk) {
@@ -613,22 +720,22 @@ __device__ inline double lm_move(const Chain &c, Lane &L)
             r2 = x * x + y * y;
         } while (r2 > 1.0 || r2 == 0.0);
         const double mult = sqrt(-2 * log(r2) / r2);
-        c.xnew[(int64_t)j * W + w] = c.lm_mu[k * c.ndim + j] + c.lm_sig[k * c.ndim + j] * (y * mult);
-        if (j + 1 < c.ndim) { c.xnew[(int64_t)(j + 1) * W + w] = c.lm_mu[k * c.ndim + j + 1] + c.lm_sig[k * c.ndim + j + 1] * (x * mult); }
+        V.xn[j] = c.lm_mu[k * c.ndim + j] + c.lm_sig[k * c.ndim + j] * (y * mult);
+        if (j + 1 < c.ndim) { V.xn[j + 1] = c.lm_mu[k * c.ndim + j + 1] + c.lm_sig[k * c.ndim + j + 1] * (x * mult); }
     }
     L.nchanged = c.ndim;
     L.cfirst = 0;
-    return exp(lm_logq(c, c.xold, w) - lm_logq(c, c.xnew, w));
+    return exp(lm_logq(c, V.xo) - lm_logq(c, V.xn));
 }
 
 // MultiStepMove::trialMove (MultiStepMove.cpp:6-47): ms_nsteps Metropolis steps of the contained
 // move under the move's own sampling functions (none: every step accepted), from xold; xnew ends at
 // the last position, xold is restored, every coordinate counts as changed, and the factor
 // oldPDF / newPDF of the own sampling functions is the move's acceptance factor
-__device__ inline double trial_move(const Chain &c, Lane &L)
+__device__ __forceinline__ double trial_move(const Chain &c, Lane &L, const Views &V)
 {
     // a mixed move: first the uniform that picks the independence move with probability lm_pmix
-    if (c.lm_on && draw_unit(c, L) < c.lm_pmix) { return lm_move(c, L); }
+    if (c.lm_on && draw_unit(c, L) < c.lm_pmix) { return lm_move(c, L, V); }
 #ifdef MCI_RTC_USER
     if (c.movetype == MCI_MOVE_DEVICE) {
         // the caller's trialMove: it moves xnew (which holds xold), names the changed coordinates
@@ -636,86 +743,101 @@ __device__ inline double trial_move(const Chain &c, Lane &L)
         const int64_t W = c.W, w = L.w;
         MciRng rng{&c, &L};
         MciMoved mv{0, c.ndim};
-        const double f = mci_user_move(c.ndim, MciVec{c.xnew + w, W}, mv, MciVec{c.mv_pold + w, W}, MciVec{c.mv_pnew + w, W},
+        const double f = mci_user_move(c.ndim, V.xn, mv, MciVec{c.mv_pold + w, W}, MciVec{c.mv_pnew + w, W},
                                        MciVec{c.steps + w, W}, rng, c.mv_par);
         L.cfirst = mv.first;
         L.nchanged = mv.n;
         return f;
     }
 #endif
-    if (!c.ms_on) { return srrd_move(c, L, true); }
+    if (!c.ms_on) { return srrd_move(c, L, V.xn, true); }
     const int64_t W = c.W, w = L.w;
-    for (int i = 0; i < c.ndim; ++i) { c.ms_x0[(int64_t)i * W + w] = c.xold[(int64_t)i * W + w]; }
-    for (int p = 0; p < c.ms_npdf; ++p) { pdf_proto(c, c.ms_pdf[p], c.xold, c.ms_pold, w); }
-    for (int i = 0; i < c.ms_nproto; ++i) { c.ms_pnew[(int64_t)i * W + w] = c.ms_pold[(int64_t)i * W + w]; }
+    const MciVec x0 = column(c.ms_x0, W, w), mo = column(c.ms_pold, W, w), mn = column(c.ms_pnew, W, w);
+    for (int i = 0; i < c.ndim; ++i) { x0[i] = V.xo[i]; }
+    for (int p = 0; p < c.ms_npdf; ++p) { pdf_proto(c, c.ms_pdf[p], V.xo, rows_from(mo, c.ms_pdf[p].off)); }
+    for (int i = 0; i < c.ms_nproto; ++i) { mn[i] = mo[i]; }
     double oldPDF = 1.;
-    for (int p = 0; p < c.ms_npdf; ++p) { oldPDF *= pdf_value(c, c.ms_pdf[p], c.ms_pold, w); }
+    for (int p = 0; p < c.ms_npdf; ++p) { oldPDF *= pdf_value(c.ms_pdf[p], mo); }
     for (int s = 0; s < c.ms_nsteps; ++s) {
-        const double moveAcc = srrd_move(c, L, false);
+        const double moveAcc = srrd_move(c, L, V.xn, false);
         double pdfAcc = 1.;
-        for (int p = 0; p < c.ms_npdf; ++p) { pdfAcc *= pdf_compute_acceptance(c, c.ms_pdf[p], L, c.ms_pold, c.ms_pnew); }
+        for (int p = 0; p < c.ms_npdf; ++p) { pdfAcc *= pdf_compute_acceptance(c, c.ms_pdf[p], L, V.xo, V.xn, mo, mn); }
         const bool acc = (draw_unit(c, L) <= pdfAcc * moveAcc);
-        double *pf = acc ? c.ms_pnew : c.ms_pold, *pt = acc ? c.ms_pold : c.ms_pnew;
-        double *xf = acc ? c.xnew : c.xold, *xt = acc ? c.xold : c.xnew;
-        for (int i = 0; i < c.ms_nproto; ++i) { pt[(int64_t)i * W + w] = pf[(int64_t)i * W + w]; }
-        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) { xt[(int64_t)j * W + w] = xf[(int64_t)j * W + w]; }
+        for (int i = 0; i < c.ms_nproto; ++i) {
+            const double v = acc ? mn[i] : mo[i];
+            mo[i] = v;
+            mn[i] = v;
+        }
+        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
+            const double v = acc ? V.xn[j] : V.xo[j];
+            V.xo[j] = v;
+            V.xn[j] = v;
+        }
     }
     double newPDF = 1.;
-    for (int p = 0; p < c.ms_npdf; ++p) { newPDF *= pdf_value(c, c.ms_pdf[p], c.ms_pold, w); }
-    for (int i = 0; i < c.ndim; ++i) { c.xold[(int64_t)i * W + w] = c.ms_x0[(int64_t)i * W + w]; }
+    for (int p = 0; p < c.ms_npdf; ++p) { newPDF *= pdf_value(c.ms_pdf[p], mo); }
+    for (int i = 0; i < c.ndim; ++i) { V.xo[i] = x0[i]; }
     L.nchanged = c.ndim;
     L.cfirst = 0;
     return oldPDF / newPDF;
 }
 
 // MCI::initializeSampling (MCIntegrator.cpp:252-271)
-__device__ inline void init_sampling(const Chain &c, Lane &L)
+__device__ __forceinline__ void init_sampling(const Chain &c, Lane &L, const Views &V)
 {
-    const int64_t W = c.W, w = L.w;
     L.acc = 0;
     L.rej = 0;
-    for (int i = 0; i < c.ndim; ++i) { c.xnew[(int64_t)i * W + w] = c.xold[(int64_t)i * W + w]; }
+#pragma unroll 4
+    for (int i = 0; i < c.ndim; ++i) { V.xn[i] = V.xo[i]; }
     L.nchanged = c.ndim;
     L.cfirst = 0;
     L.accepted = true;
-    for (int p = 0; p < c.npdf; ++p) { pdf_proto(c, c.pdf[p], c.xold, c.pold, w); }
-    for (int i = 0; i < c.nproto; ++i) { c.pnew[(int64_t)i * W + w] = c.pold[(int64_t)i * W + w]; }
+    for (int p = 0; p < c.npdf; ++p) { pdf_proto(c, c.pdf[p], V.xo, rows_from(V.po, c.pdf[p].off)); }
+#pragma unroll 4
+    for (int i = 0; i < c.nproto; ++i) { V.pn[i] = V.po[i]; }
 #ifdef MCI_RTC_USER
     if (c.movetype == MCI_MOVE_DEVICE && c.mv_nproto > 0) { // the trial move's initializeProtoValues
-        mci_user_move_proto(c.ndim, MciVec{c.xold + w, W}, c.mv_par, MciVec{c.mv_pold + w, W});
+        const int64_t W = c.W, w = L.w;
+        mci_user_move_proto(c.ndim, V.xo, c.mv_par, MciVec{c.mv_pold + w, W});
         for (int i = 0; i < c.mv_nproto; ++i) { c.mv_pnew[(int64_t)i * W + w] = c.mv_pold[(int64_t)i * W + w]; }
     }
 #endif
-    cb_record(c, L);
+    cb_record(c, L, V);
 }
 
 // MCI::doStepMRT2 (MCIntegrator.cpp:326-360)
-__device__ inline void step_mrt2(const Chain &c, Lane &L)
+__device__ __forceinline__ void step_mrt2(const Chain &c, Lane &L, const Views &V)
 {
-    const int64_t W = c.W, w = L.w;
     step_begin(L);
-    const double moveAcc = trial_move(c, L);
+    const double moveAcc = trial_move(c, L, V);
     if (c.periodic) {
-        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) { wrap(c, j, c.xnew[(int64_t)j * W + w]); }
+        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) { wrap(c, j, V.xn[j]); }
     }
     double pdfAcc = 1.;
-    for (int p = 0; p < c.npdf; ++p) { pdfAcc = pdfAcc * pdf_compute_acceptance(c, c.pdf[p], L, c.pold, c.pnew); }
-    const double u = draw_accept(c, L);
-    L.accepted = (u <= pdfAcc * moveAcc);
+    for (int p = 0; p < c.npdf; ++p) { pdfAcc = pdfAcc * pdf_compute_acceptance(c, c.pdf[p], L, V.xo, V.xn, V.po, V.pn); }
+    L.accepted = draw_accept(c, L, pdfAcc * moveAcc);
     if (L.accepted) { ++L.acc; } else { ++L.rej; }
-    cb_record(c, L);
+    cb_record(c, L, V);
     step_end(c, L);
     // commit or roll back the coordinates and proto values that can differ
-    if (L.accepted) {
-        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) { c.xold[(int64_t)j * W + w] = c.xnew[(int64_t)j * W + w]; }
-        for (int i = 0; i < c.nproto; ++i) { c.pold[(int64_t)i * W + w] = c.pnew[(int64_t)i * W + w]; }
+    const bool acc = L.accepted;
+#pragma unroll 4
+    for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
+        const double o = V.xo[j], n = V.xn[j];
+        const double v = acc ? n : o;
+        V.xo[j] = v;
+        V.xn[j] = v;
     }
-    else {
-        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) { c.xnew[(int64_t)j * W + w] = c.xold[(int64_t)j * W + w]; }
-        for (int i = 0; i < c.nproto; ++i) { c.pnew[(int64_t)i * W + w] = c.pold[(int64_t)i * W + w]; }
+#pragma unroll 4
+    for (int i = 0; i < c.nproto; ++i) {
+        const double o = V.po[i], n = V.pn[i];
+        const double v = acc ? n : o;
+        V.po[i] = v;
+        V.pn[i] = v;
     }
 #ifdef MCI_RTC_USER
     if (c.movetype == MCI_MOVE_DEVICE) { // the trial move's newToOld / oldToNew
+        const int64_t W = c.W, w = L.w;
         double *mf = L.accepted ? c.mv_pnew : c.mv_pold, *mt = L.accepted ? c.mv_pold : c.mv_pnew;
         for (int i = 0; i < c.mv_nproto; ++i) { mt[(int64_t)i * W + w] = mf[(int64_t)i * W + w]; }
     }
@@ -723,97 +845,101 @@ __device__ inline void step_mrt2(const Chain &c, Lane &L)
 }
 
 // MCI::doStepRandom (MCIntegrator.cpp:362-376): no sampling function
-__device__ inline void step_random(const Chain &c, Lane &L)
+__device__ __forceinline__ void step_random(const Chain &c, Lane &L, const Views &V)
 {
-    const int64_t W = c.W, w = L.w;
     step_begin(L);
-    for (int i = 0; i < c.ndim; ++i) { c.xnew[(int64_t)i * W + w] = draw_unit(c, L); }
+    for (int i = 0; i < c.ndim; ++i) { V.xn[i] = draw_unit(c, L); }
     step_end(c, L);
     for (int i = 0; i < c.ndim; ++i) {
-        double &x = c.xnew[(int64_t)i * W + w];
-        if (c.periodic) { x = c.lb[i] + x * (c.ub[i] - c.lb[i]); }
+        double &x = V.xn[i];
+        if (c.periodic) { x = param(c.lb, i) + x * (param(c.ub, i) - param(c.lb, i)); }
         else { x = -(double)3.402823466e+38f + x * ((double)3.402823466e+38f + (double)3.402823466e+38f); }
     }
     L.nchanged = c.ndim;
     L.cfirst = 0;
     L.accepted = true;
     ++L.acc;
-    cb_record(c, L);
-    for (int i = 0; i < c.ndim; ++i) { c.xold[(int64_t)i * W + w] = c.xnew[(int64_t)i * W + w]; }
+    cb_record(c, L, V);
+    for (int i = 0; i < c.ndim; ++i) { V.xo[i] = V.xn[i]; }
 }
 
 // --------------------------------------------------------------------------
 // observables (ObservableFunctionInterface::observableFunction of each kind)
 // --------------------------------------------------------------------------
-__device__ inline void obs_eval(const Chain &c, const ObsDev &o, int64_t w)
+__device__ __forceinline__ void obs_eval(const Chain &c, const ObsDev &o, const Views &V)
 {
-    const int64_t W = c.W;
-    const double *x = c.xold;
-    double *out = c.obsval + (int64_t)o.voff * W;
+    const MciVec &x = V.xo;
+    const MciVec out = rows_from(V.ov, o.voff);
     switch (o.kind) {
     case MCI_OBS_X2:
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; out[(int64_t)i * W + w] = v * v; }
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; out[i] = v * v; }
         break;
     case MCI_OBS_X2_SUM: {
         double s = 0.0;
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; s = s + v * v; }
-        out[w] = s / o.p0;
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; s = s + v * v; }
+        out[0] = s / o.p0;
         break;
     }
     case MCI_OBS_X:
-        for (int i = 0; i < c.ndim; ++i) { out[(int64_t)i * W + w] = x[(int64_t)i * W + w]; }
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { out[i] = x[i]; }
         break;
     case MCI_OBS_X_SUM: {
         double s = 0.0;
-        for (int i = 0; i < c.ndim; ++i) { s = s + x[(int64_t)i * W + w]; }
-        out[w] = s;
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { s = s + x[i]; }
+        out[0] = s;
         break;
     }
     case MCI_OBS_CONST:
-        out[w] = o.p0;
+        out[0] = o.p0;
         break;
     case MCI_OBS_EXP_X2: {
         double s = 0.0;
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; s = s + v * v; }
-        out[w] = exp(-(s / o.p0));
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; s = s + v * v; }
+        out[0] = exp(-(s / o.p0));
         break;
     }
     case MCI_OBS_INDICATOR:
-        out[w] = (x[(int64_t)(int)o.p0 * W + w] > 0.0) ? 1.0 : 0.0;
+        out[0] = (x[(int)o.p0] > 0.0) ? 1.0 : 0.0;
         break;
     case MCI_OBS_GAUSS_X2: {
         double s = 0.0;
-        for (int i = 0; i < c.ndim; ++i) { const double v = x[(int64_t)i * W + w]; s = s + v * v; }
-        out[w] = exp(-s) * s * o.p0;
+#pragma unroll 4
+        for (int i = 0; i < c.ndim; ++i) { const double v = x[i]; s = s + v * v; }
+        out[0] = exp(-s) * s * o.p0;
         break;
     }
     case MCI_OBS_PDF_LOG: { // the committed proto values of sampling function p0
         const PdfDev &p = c.pdf[(int)o.p0];
-        const double *pv = c.pold + (int64_t)p.off * W + w;
-        if (p.kind == MCI_PDF_GMM_ISO) { out[w] = pv[(int64_t)p.K * W]; }
+        const MciVec pv = rows_from(V.po, p.off);
+        if (p.kind == MCI_PDF_GMM_ISO) { out[0] = pv[p.K]; }
 #ifdef MCI_RTC_USER
-        else if (p.kind == MCI_PDF_DEVICE) { out[w] = log(mci_user_pdf_sampling(p.uid, p.nproto, MciVec{const_cast<double *>(pv), W}, p.a)); }
+        else if (p.kind == MCI_PDF_DEVICE) { out[0] = log(mci_user_pdf_sampling(p.uid, p.nproto, pv, p.a)); }
 #endif
         else {
             double s = 0.0;
-            for (int j = 0; j < p.nproto; ++j) { s = s + pv[(int64_t)j * W]; }
-            out[w] = -s;
+            for (int j = 0; j < p.nproto; ++j) { s = s + pv[j]; }
+            out[0] = -s;
         }
         break;
     }
     case MCI_OBS_PDF_PROTO: {
         const PdfDev &p = c.pdf[(int)o.p0];
-        for (int j = 0; j < o.nobs; ++j) { out[(int64_t)j * W + w] = c.pold[(int64_t)(p.off + j) * W + w]; }
+        for (int j = 0; j < o.nobs; ++j) { out[j] = V.po[p.off + j]; }
         break;
     }
     case MCI_OBS_DEP_SQUARE: { // the last values of an earlier observable (evaluated before this one)
-        const double *v = c.obsval + (int64_t)c.obs[(int)o.p0].voff * W;
-        for (int j = 0; j < o.nobs; ++j) { const double y = v[(int64_t)j * W + w]; out[(int64_t)j * W + w] = y * y; }
+        const MciVec v = rows_from(V.ov, c.obs[(int)o.p0].voff);
+        for (int j = 0; j < o.nobs; ++j) { const double y = v[j]; out[j] = y * y; }
         break;
     }
 #ifdef MCI_RTC_USER
     case MCI_OBS_DEVICE: // the caller's observableFunction (built at run time with the functor's source)
-        mci_user_observable(o.uid, c.ndim, MciVec{const_cast<double *>(x) + w, W}, o.par, MciVec{out + w, W});
+        mci_user_observable(o.uid, c.ndim, x, o.par, out);
         break;
 #endif
     }
@@ -823,27 +949,55 @@ __device__ inline void obs_eval(const Chain &c, const ObsDev &o, int64_t w)
 // storage of Simple/Block/FullAccumulator).  Observable values are a function of the
 // current position, so they are re-evaluated exactly when the position changed since the
 // last evaluation (the reference's _nchanged bookkeeping) — the stored numbers are equal.
-__device__ inline void accumulate(const Chain &c, const Lane &L, int64_t s, uint32_t &dirty)
+// SUMS: the running block sums stay in the wave's columns (Views::sums) and a block's mean is written
+// when it ends (the sum times the accumulator's factor, as finalize_accu forms it); else they are
+// added to the data in HBM.
+template <bool SUMS>
+__device__ __forceinline__ void accumulate(const Chain &c, const Lane &L, const Views &V, int64_t s, uint32_t &dirty)
 {
     const int64_t W = c.W, w = L.w;
     if (L.accepted) { dirty = 0xffffffffu; }
     for (int i = 0; i < c.nobs; ++i) {
         const ObsDev &o = c.obs[i];
-        if (s % o.nskip != 0) { continue; }
+        if (SUMS) {
+            int &skip = V.cnt[i * V.cs];
+            const int n = skip;
+            skip = n + 1 == o.nskip ? 0 : n + 1;
+            if (n != 0) { continue; }
+        }
+        else if (s % o.nskip != 0) { continue; }
         if (dirty & (1u << i)) {
-            obs_eval(c, o, w);
+            obs_eval(c, o, V);
             dirty &= ~(1u << i);
         }
-        const int64_t a = s / o.nskip;
-        const double *v = c.obsval + (int64_t)o.voff * W;
+        const MciVec v = rows_from(V.ov, o.voff);
         if (o.acc == ACC_FULL) {
-            for (int j = 0; j < o.nobs; ++j) { o.data[(a * o.nobs + j) * W + w] = v[(int64_t)j * W + w]; }
+            const int64_t a = o.nskip == 1 ? s : s / o.nskip;
+            for (int j = 0; j < o.nobs; ++j) { o.data[(a * o.nobs + j) * W + w] = v[j]; }
+        }
+        else if (SUMS) {
+            const MciVec t = rows_from(V.sums, o.voff);
+#pragma unroll 4
+            for (int j = 0; j < o.nobs; ++j) { t[j] = t[j] + v[j]; }
+            if (o.acc == ACC_BLOCK) {
+                int &filled = V.cnt[(c.nobs + i) * V.cs];
+                const int m = filled + 1;
+                filled = m == o.blocksize ? 0 : m;
+                if (m == o.blocksize) {
+                    const int64_t b = (s / o.nskip) / o.blocksize;
+                    const double normf = 1. / o.blocksize;
+                    for (int j = 0; j < o.nobs; ++j) {
+                        o.data[(b * o.nobs + j) * W + w] = t[j] * normf;
+                        t[j] = 0.0;
+                    }
+                }
+            }
         }
         else {
-            const int64_t b = (o.acc == ACC_BLOCK) ? a / o.blocksize : 0;
+            const int64_t b = (o.acc == ACC_BLOCK) ? (s / o.nskip) / o.blocksize : 0;
             for (int j = 0; j < o.nobs; ++j) {
                 double &d = o.data[(b * o.nobs + j) * W + w];
-                d = d + v[(int64_t)j * W + w];
+                d = d + v[j];
             }
         }
     }
@@ -881,13 +1035,22 @@ __device__ inline void load_lane(const Chain &c, Lane &L, int64_t w)
     L.w = w;
     L.mtp = (c.rng == MCI_RNG_MT19937_64) ? c.mtp[w] : 0;
     L.t = (c.rng == MCI_RNG_PHILOX) ? c.ctr[w] : 0;
+    L.m0 = L.m1 = L.mm = 0;
+    if (c.rng == MCI_RNG_MT19937_64) {
+        L.m0 = c.mt[(int64_t)L.mtp * c.W + w];
+        mt_ahead(c, L);
+    }
     L.k = 0;
     L.kx = 0;
+    L.b0t = L.bkt = ~(uint64_t)0;  // no block yet (a pair's counter stays below 2^63)
+    L.bkn = 0;
+    for (int i = 0; i < 4; ++i) { L.b0[i] = L.bk[i] = 0u; }
     L.nchanged = c.ndim;
     L.cfirst = 0;
     L.accepted = true;
     L.acc = 0;
     L.rej = 0;
+    L.st0 = c.steps[w];
     L.sf = 0;
     L.sv[0] = L.sv[1] = 0.0;
     if (c.nsf != nullptr) {

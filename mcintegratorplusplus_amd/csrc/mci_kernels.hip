@@ -1086,7 +1086,7 @@ __global__ void k_decorr_compare(double *oa, double *oe, const double *na, const
 }
 
 // MCI::moveX (MCIntegrator.cpp:606-612)
-__global__ void k_move_x(Chain c)
+__global__ __launch_bounds__(64) void k_move_x(Chain c)
 {
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= c.W) { return; }
@@ -1095,7 +1095,15 @@ __global__ void k_move_x(Chain c)
     const int64_t W = c.W;
     for (int i = 0; i < c.ndim; ++i) { c.xnew[(int64_t)i * W + w] = c.xold[(int64_t)i * W + w]; }
     step_begin(L);
-    trial_move(c, L);
+    Views V;
+    V.xo = column(c.xold, W, w);
+    V.xn = column(c.xnew, W, w);
+    V.po = column(c.pold, W, w);
+    V.pn = column(c.pnew, W, w);
+    V.ov = V.sums = V.xo;
+    V.cnt = nullptr;
+    V.cs = 0;
+    trial_move(c, L, V);
     step_end(c, L);
     for (int j = 0; j < c.ndim; ++j) {
         double x = c.xnew[(int64_t)j * W + w];
@@ -1173,14 +1181,26 @@ hipError_t launch_mt_align(uint64_t *mt, int32_t *mtp, int64_t W, hipStream_t s)
 
 hipError_t launch_sample(const Chain &c, int64_t nsteps, int acc, const uint8_t *active, hipStream_t s, const CalibCtrl *skip)
 {
-    hipLaunchKernelGGL(k_sample, grid1(c.W, 64), dim3(64), 0, s, c, nsteps, acc, active, skip);
+    const StateLds st = state_lds_of(c, acc != 0);
+    const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
+    if (st.in_lds) { hipLaunchKernelGGL(k_sample<true>, g, b, st.bytes, s, c, nsteps, acc, active, skip); }
+    else { hipLaunchKernelGGL(k_sample<false>, g, b, 0, s, c, nsteps, acc, active, skip); }
     return hipGetLastError();
 }
 
 hipError_t launch_calibrate_indep(const Chain &c, int nfind, double target, int64_t min_stat, const double *dimSizes, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_calibrate_indep, grid1(c.W, 64), dim3(64), 0, s, c, nfind, target, min_stat, dimSizes);
+    const StateLds st = state_lds_of(c, false);
+    const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
+    if (st.in_lds) { hipLaunchKernelGGL(k_calibrate_indep<true>, g, b, st.bytes, s, c, nfind, target, min_stat, dimSizes); }
+    else { hipLaunchKernelGGL(k_calibrate_indep<false>, g, b, 0, s, c, nfind, target, min_stat, dimSizes); }
     return hipGetLastError();
+}
+
+StateLds state_lds_of(const Chain &c, bool observables)
+{
+    const size_t n = state_lds(c, observables ? chain_nobsdim(c) : 0);
+    return n <= STATE_LDS_MAX ? StateLds{n, 1} : StateLds{0, 0};
 }
 
 hipError_t launch_scale_steps(const Chain &c, const CalibCtrl *ctrl, const double *dimSizes, hipStream_t s)

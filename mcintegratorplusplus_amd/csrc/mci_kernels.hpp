@@ -54,6 +54,13 @@ hipError_t launch_walker_columns(const Chain &c, const Chain &dense, const int32
                                  hipStream_t s);
 // every walker's mt19937_64 state rotated to next index 0 (the same generator)
 hipError_t launch_mt_align(uint64_t *mt, int32_t *mtp, int64_t W, hipStream_t s);
+// dynamic LDS of a generic step kernel's launch and whether the walkers' state goes there
+struct StateLds
+{
+    size_t bytes;
+    int in_lds;
+};
+StateLds state_lds_of(const Chain &c, bool observables);
 hipError_t launch_sample(const Chain &c, int64_t nsteps, int acc, const uint8_t *active, hipStream_t s,
                          const CalibCtrl *skip = nullptr);
 hipError_t launch_calibrate_indep(const Chain &c, int nfind, double target, int64_t min_stat, const double *dimSizes, hipStream_t s);

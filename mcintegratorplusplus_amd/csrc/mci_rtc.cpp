@@ -32,11 +32,11 @@ struct Loaded
 };
 std::map<std::pair<std::string, int>, Loaded> g_cache;
 
-const char *kSample = "mcid::k_sample", *kCalib = "mcid::k_calibrate_indep";
+// the walkers' state in HBM, in LDS
+const char *const kNames[4] = {"mcid::k_sample<false>", "mcid::k_sample<true>", "mcid::k_calibrate_indep<false>", "mcid::k_calibrate_indep<true>"};
 
-// compiles text; on success code holds the code object and the kernels' lowered names
-int compile(const std::string &text, const std::string &arch, std::vector<char> &code, std::string &nsample, std::string &ncalib,
-            std::string &log)
+// compiles text; on success code holds the code object and names the kernels' lowered names
+int compile(const std::string &text, const std::string &arch, std::vector<char> &code, std::string (&names)[4], std::string &log)
 {
     hiprtcProgram p;
     if (hiprtcCreateProgram(&p, text.c_str(), "mci_device_functors.hip", rtc_nheaders, rtc_header_texts, rtc_header_names) !=
@@ -44,8 +44,7 @@ int compile(const std::string &text, const std::string &arch, std::vector<char> 
         log = "hiprtcCreateProgram failed";
         return MCI_E_DEVICE;
     }
-    hiprtcAddNameExpression(p, kSample);
-    hiprtcAddNameExpression(p, kCalib);
+    for (const char *n : kNames) { hiprtcAddNameExpression(p, n); }
     // the library's own flags: no contraction (bit-exact FP64 chains), correctly rounded FP32
     // divide and sqrt, no packed FP32 instructions
     const std::string off = "--offload-arch=" + arch;
@@ -67,13 +66,15 @@ int compile(const std::string &text, const std::string &arch, std::vector<char> 
     hiprtcGetCodeSize(p, &cs);
     code.resize(cs);
     hiprtcGetCode(p, code.data());
-    const char *ls1 = nullptr, *ls2 = nullptr;
-    hiprtcGetLoweredName(p, kSample, &ls1);
-    hiprtcGetLoweredName(p, kCalib, &ls2);
-    nsample = ls1 ? ls1 : "";
-    ncalib = ls2 ? ls2 : "";
+    bool all = cs > 0;
+    for (int i = 0; i < 4; ++i) {
+        const char *l = nullptr;
+        hiprtcGetLoweredName(p, kNames[i], &l);
+        names[i] = l ? l : "";
+        all = all && !names[i].empty();
+    }
     hiprtcDestroyProgram(&p);
-    return (cs > 0 && !nsample.empty() && !ncalib.empty()) ? MCI_OK : MCI_E_DEVICE;
+    return all ? MCI_OK : MCI_E_DEVICE;
 }
 
 void dispatch(std::string &t, const char *sig, const char *call, const char *ret, const std::vector<RtcFunctor> &f, const char *suffix)
@@ -162,8 +163,8 @@ bool rtc_program(const std::vector<RtcFunctor> &pdfs, const std::vector<RtcFunct
 int rtc_check(const std::string &text, const char *arch, std::string &log)
 {
     std::vector<char> code;
-    std::string a, b;
-    return compile(text, arch ? arch : "gfx950", code, a, b, log);
+    std::string names[4];
+    return compile(text, arch ? arch : "gfx950", code, names, log);
 }
 
 int rtc_get(const std::string &text, RtcKernels &out, std::string &log)
@@ -183,18 +184,20 @@ int rtc_get(const std::string &text, RtcKernels &out, std::string &log)
     const size_t colon = arch.find(':');
     if (colon != std::string::npos) { arch.resize(colon); }
     std::vector<char> code;
-    std::string ns, nc;
-    const int st = compile(text, arch, code, ns, nc, log);
+    std::string names[4];
+    const int st = compile(text, arch, code, names, log);
     if (st != MCI_OK) { return st; }
     Loaded L;
     if (hipModuleLoadData(&L.mod, code.data()) != hipSuccess) {
         log = "hipModuleLoadData failed";
         return MCI_E_DEVICE;
     }
-    if (hipModuleGetFunction(&L.k.sample, L.mod, ns.c_str()) != hipSuccess ||
-        hipModuleGetFunction(&L.k.calibrate, L.mod, nc.c_str()) != hipSuccess) {
-        log = "hipModuleGetFunction failed";
-        return MCI_E_DEVICE;
+    hipFunction_t *const f[4] = {&L.k.sample[0], &L.k.sample[1], &L.k.calibrate[0], &L.k.calibrate[1]};
+    for (int i = 0; i < 4; ++i) {
+        if (hipModuleGetFunction(f[i], L.mod, names[i].c_str()) != hipSuccess) {
+            log = "hipModuleGetFunction failed";
+            return MCI_E_DEVICE;
+        }
     }
     g_cache.emplace(key, L);
     out = L.k;
@@ -205,17 +208,19 @@ hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps
                              const CalibCtrl *skip)
 {
     Chain cc = c;
+    const StateLds st = state_lds_of(c, acc != 0);
     void *args[] = {&cc, &nsteps, &acc, &active, &skip};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
-    return hipModuleLaunchKernel(k.sample, grid, 1, 1, 64, 1, 1, 0, s, args, nullptr);
+    return hipModuleLaunchKernel(k.sample[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
 }
 
 hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int nfind, double target, int64_t min_stat,
                                       const double *dimSizes, hipStream_t s)
 {
     Chain cc = c;
+    const StateLds st = state_lds_of(c, false);
     void *args[] = {&cc, &nfind, &target, &min_stat, &dimSizes};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
-    return hipModuleLaunchKernel(k.calibrate, grid, 1, 1, 64, 1, 1, 0, s, args, nullptr);
+    return hipModuleLaunchKernel(k.calibrate[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
 }
 } // namespace mcid

@@ -15,10 +15,10 @@ struct RtcFunctor
     std::string name, source;
 };
 
-// the generic step kernels of one module (loaded on one device)
+// the generic step kernels of one module (loaded on one device): the walkers' state in HBM [0], in LDS [1]
 struct RtcKernels
 {
-    hipFunction_t sample = nullptr, calibrate = nullptr;
+    hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
 };
 
 // true when name is a C identifier

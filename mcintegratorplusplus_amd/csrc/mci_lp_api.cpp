@@ -7,6 +7,7 @@
 #include "mci_kernels.hpp"
 #include "mci_lp.hpp"
 #include "mci_mlp.hpp"
+#include "mci_mlp_step.hpp"
 
 #include <algorithm>
 #include <cfloat>
@@ -66,6 +67,13 @@ struct mci_mlp
     DBuf<bf16_t> Xb, H1b, H2b, dOb, dZ2b, dZ1b;
     DBuf<float> X, Y, Z1, Z2, OUT, dO, dH2, dH1, loss;
     DBuf<float> ws; // split-reduction partials of the weight gradients
+    // networks whose sample tile fits a compute unit train through mci_mlp_step.hip (else gemm by gemm)
+    bool tiled = false;
+    mcim::StepNet step{};
+    mcim::StepWork work{};
+    int64_t step_cap = 0;
+    DBuf<bf16_t> copies, tiles;
+    DBuf<float> tile_bias;
     int adam_t = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -115,6 +123,60 @@ mci_status mlp_upload_params(mci_mlp *n, const std::vector<float> &pad)
     HIPCHK(hipMemset(n->m.p, 0, pad.size() * sizeof(float)));
     HIPCHK(hipMemset(n->v.p, 0, pad.size() * sizeof(float)));
     n->adam_t = 0;
+    if (n->tiled) { HIPCHK(mcim::launch_step_copies(n->step, n->stream)); }
+    return MCI_OK;
+}
+
+// the BF16 copies of the weights that the tiled training path reads, their padding cleared
+mci_status mlp_step_setup(mci_mlp *n)
+{
+    n->tiled = mcim::step_lds(n->d, n->H, n->Op) <= mcim::STEP_LDS_MAX;
+    if (!n->tiled) { return MCI_OK; }
+    mcim::StepNet &N = n->step;
+    N.d = n->d;
+    N.H = n->H;
+    N.K = n->K;
+    N.Op = n->Op;
+    N.dp = round_up(n->d, 32);
+    N.Hp = round_up(n->H, 32);
+    N.oW1 = n->oW1;
+    N.ob1 = n->ob1;
+    N.oW2 = n->oW2;
+    N.ob2 = n->ob2;
+    N.oW3 = n->oW3;
+    N.ob3 = n->ob3;
+    N.npad = n->npad;
+    N.p = n->p.p;
+    const size_t w1 = (size_t)N.Hp * N.dp, w2 = (size_t)N.Hp * N.Hp, w3 = (size_t)N.Hp * N.Op;
+    HIPCHK(n->copies.ensure(w1 + 2 * w2 + 2 * w3));
+    N.W1t = n->copies.p;
+    N.W2t = N.W1t + w1;
+    N.W2 = N.W2t + w2;
+    N.W3t = N.W2 + w2;
+    N.W3 = N.W3t + w3;
+    HIPCHK(hipMemsetAsync(n->copies.p, 0, n->copies.n * sizeof(bf16_t), n->stream));
+    return MCI_OK;
+}
+
+// workspace of a gradient over ns samples (tiled path)
+mci_status mlp_step_reserve(mci_mlp *n, int64_t ns)
+{
+    HIPCHK(n->loss.ensure((size_t)ns));
+    if (ns <= n->step_cap) { return MCI_OK; }
+    const mcim::StepNet &N = n->step;
+    const size_t rows = (size_t)((ns + mcim::STEP_NS - 1) / mcim::STEP_NS * mcim::STEP_NS);
+    HIPCHK(n->tiles.ensure(rows * (size_t)(N.dp + 4 * N.Hp + N.Op)));
+    HIPCHK(n->tile_bias.ensure(rows / mcim::STEP_NS * (size_t)(N.Op + 2 * N.Hp)));
+    HIPCHK(n->ws.ensure((size_t)mcim::step_splits(N, ns) * (size_t)n->npad));
+    mcim::StepWork &w = n->work;
+    w.X = n->tiles.p;
+    w.H1 = w.X + rows * N.dp;
+    w.H2 = w.H1 + rows * N.Hp;
+    w.dZ2 = w.H2 + rows * N.Hp;
+    w.dZ1 = w.dZ2 + rows * N.Hp;
+    w.dO = w.dZ1 + rows * N.Hp;
+    w.bias = n->tile_bias.p;
+    n->step_cap = ns;
     return MCI_OK;
 }
 
@@ -181,12 +243,26 @@ mci_status mlp_fwd_bwd(mci_mlp *n, int64_t ns)
     return MCI_OK;
 }
 
-mci_status mlp_adam(mci_mlp *n, float lr)
+// the update with the gradient of the last minibatch (ns samples)
+mci_status mlp_adam(mci_mlp *n, int64_t ns, float lr)
 {
     ++n->adam_t;
     const float b1 = 0.9f, b2 = 0.999f;
     const float bc1 = 1.0f - std::pow(b1, (float)n->adam_t), bc2 = 1.0f - std::pow(b2, (float)n->adam_t);
+    if (n->tiled) {
+        HIPCHK(mcim::launch_step_adam(n->step, ns, n->work, n->g.p, n->p.p, n->m.p, n->v.p, n->pb.p, lr, b1, b2, 1e-8f, bc1, bc2, n->stream));
+        return MCI_OK;
+    }
     HIPCHK(mcim::launch_adam(n->p.p, n->m.p, n->v.p, n->g.p, n->pb.p, n->npad, lr, b1, b2, 1e-8f, bc1, bc2, n->stream));
+    return MCI_OK;
+}
+
+// the minibatch's gradient as split sums (tiled path); loss per sample in n->loss
+mci_status mlp_step_grad(mci_mlp *n, const mcim::StepBatch &B)
+{
+    n->work.loss = n->loss.p;
+    n->work.ws = n->ws.p;
+    HIPCHK(mcim::launch_step_grad(n->step, B, n->work, n->stream));
     return MCI_OK;
 }
 
@@ -221,6 +297,10 @@ mci_status mlp_make(int d, int H, int K, uint64_t seed, hipStream_t stream, mci_
         n->g.ensure(n->npad) != hipSuccess || n->pb.ensure(n->npad) != hipSuccess) {
         delete n;
         return fail(MCI_E_DEVICE, "allocation failed");
+    }
+    if (const mci_status st = mlp_step_setup(n); st != MCI_OK) {
+        delete n;
+        return st;
     }
     // Glorot-uniform weights (output layer scaled by 0.1), zero biases
     std::vector<float> flat((size_t)n->np, 0.f);
@@ -850,10 +930,23 @@ mci_status mci_mlp_loss_grad(mci_mlp *m, int64_t n, const float *ctx, const floa
 {
     CHECKM(m);
     if (n < 1 || !ctx || !y) { return fail(MCI_E_INVALID_ARGUMENT, "bad arguments"); }
-    TRY(mlp_reserve(m, n));
+    if (m->tiled) {
+        TRY(mlp_step_reserve(m, n));
+        HIPCHK(m->X.ensure((size_t)m->d * n));
+        HIPCHK(m->Y.ensure((size_t)m->d * n));
+    }
+    else { TRY(mlp_reserve(m, n)); }
     TRY(upload_transposed(m->X.p, ctx, n, m->d));
     TRY(upload_transposed(m->Y.p, y, n, m->d));
-    TRY(mlp_fwd_bwd(m, n));
+    if (m->tiled) {
+        mcim::StepBatch B{};
+        B.n = n;
+        B.X = m->X.p;
+        B.Y = m->Y.p;
+        TRY(mlp_step_grad(m, B));
+        HIPCHK(mcim::launch_step_sum(m->step, n, m->work, m->g.p, m->stream));
+    }
+    else { TRY(mlp_fwd_bwd(m, n)); }
     std::vector<float> l((size_t)n), gp((size_t)m->npad);
     HIPCHK(hipMemcpyAsync(l.data(), m->loss.p, sizeof(float) * n, hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipMemcpyAsync(gp.data(), m->g.p, sizeof(float) * m->npad, hipMemcpyDeviceToHost, m->stream));
@@ -1062,7 +1155,7 @@ mci_status mci_lp_train(mci_lp *lp, int iters, int batch, double lr, double *los
     if (iters < 1 || batch < 64 || batch > (1 << 20) || !(lr > 0.)) { return fail(MCI_E_INVALID_ARGUMENT, "bad training settings"); }
     TRY(net_ready(lp));
     mci_mlp *n = lp->net;
-    TRY(mlp_reserve(n, batch));
+    TRY(n->tiled ? mlp_step_reserve(n, batch) : mlp_reserve(n, batch));
     if (lp->fixed_input) {
         HIPCHK(lp->dctx0.ensure((size_t)lp->d));
         HIPCHK(hipMemcpy(lp->dctx0.p, lp->ctx0.data(), sizeof(float) * (size_t)lp->d, hipMemcpyHostToDevice));
@@ -1079,11 +1172,17 @@ mci_status mci_lp_train(mci_lp *lp, int iters, int batch, double lr, double *los
         return MCI_OK;
     };
     for (int it = 0; it < iters; ++it) {
-        HIPCHK(mcil::launch_lp_pairs(lp->snap.p, lp->nsnap, lp->d, lp->W, batch, lp->train_iter++, k0, k1, (float)lp->same_frac,
-                                     lp->fixed_input ? lp->dctx0.p : nullptr, n->X.p, n->Y.p, n->stream));
-        TRY(mlp_fwd_bwd(n, batch));
+        const float *ctx = lp->fixed_input ? lp->dctx0.p : nullptr;
+        if (n->tiled) {
+            TRY(mlp_step_grad(n, {batch, nullptr, nullptr, lp->snap.p, ctx, lp->nsnap, lp->W, lp->train_iter++, k0, k1, (float)lp->same_frac}));
+        }
+        else {
+            HIPCHK(mcil::launch_lp_pairs(lp->snap.p, lp->nsnap, lp->d, lp->W, batch, lp->train_iter++, k0, k1, (float)lp->same_frac, ctx,
+                                         n->X.p, n->Y.p, n->stream));
+            TRY(mlp_fwd_bwd(n, batch));
+        }
         if (it == 0) { TRY(mean_loss(lp->loss_first)); }
-        TRY(mlp_adam(n, (float)lr));
+        TRY(mlp_adam(n, batch, (float)lr));
     }
     TRY(mean_loss(lp->loss_last)); // loss of the last minibatch (before its update)
     lp->timings[3] = ms_since(t0);

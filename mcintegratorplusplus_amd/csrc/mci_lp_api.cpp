@@ -154,6 +154,7 @@ mci_status mlp_step_setup(mci_mlp *n)
     N.W2 = N.W2t + w2;
     N.W3t = N.W2 + w2;
     N.W3 = N.W3t + w3;
+    N.lines = (int)(n->copies.n * sizeof(bf16_t) / 128);
     HIPCHK(hipMemsetAsync(n->copies.p, 0, n->copies.n * sizeof(bf16_t), n->stream));
     return MCI_OK;
 }

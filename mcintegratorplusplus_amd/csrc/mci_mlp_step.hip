@@ -2,7 +2,7 @@
 //
 // k_step_tile: one workgroup of 16 waves takes 16 samples through the whole network and back.  The
 // samples' activations stay in LDS (pre-activations in FP32, the products' operands in BF16), the
-// weights come from the L2: at the learned proposal's size (d 32, H 128, 576 outputs) 375 KB per
+// weights come from the L2 in operand order: at the learned proposal's size (d 32, H 128, 576 outputs) 375 KB per
 // workgroup, 96 MB for the 256 workgroups of 4096 samples.  Every product is
 // v_mfma_f32_16x16x32_bf16 with the features as rows and the samples as columns: lane l supplies row or
 // column l % 16 and terms 8 (l / 16) .. + 7 of the reduction, accumulator element i of lane l is
@@ -19,10 +19,12 @@
 // reads.
 //
 // What bounds it: latency.  4096 samples are one workgroup per compute unit, and a layer is one or two
-// round trips to the L2 and a barrier.  Measured at d 32, H 128, K 8 and 4096 samples: 35.6 + 8.3 + 5.1 us
-// an iteration (tile, weight gradients, Adam), 49 us with the launches; as separate products, row sums and
-// elementwise passes (about 25 launches, 50 MB of activations through memory) 276 us.  Tiles past the LDS
-// of a compute unit (d > 80 at H 128, K 8; H > 512 at d 32) still train that way.
+// round trips to the L2 and a barrier.  Measured at d 32, H 128, K 8 and 4096 samples: 24.7 + 8.3 + 5.1 us
+// an iteration (tile, weight gradients, Adam), 42 us with the launches; as separate products, row sums and
+// elementwise passes (about 25 launches, 50 MB of activations through memory) 276 us.  With row-major
+// weights (half lines per request), no warming of the L2, 64-bit remainders in the pairs and one wave per
+// tile of the backward products the tile took 35.6 us.  Tiles past the LDS of a compute unit (d > 75 at
+// H 128, K 8; H > 512 at d 32) train by separate products.
 #include "mci_mlp_step.hpp"
 
 namespace mcim
@@ -62,27 +64,37 @@ __device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, ui
     o[0] = c0; o[1] = c1; o[2] = c2; o[3] = c3;
 }
 
-// C[16 ft .. + 15][sample] for the wave's feature tiles ft: Wt [16 ntiles][kp], xs [NS][kp + PAD] in
-// LDS, kp a multiple of 32.  Eight loads of a row are in flight at once (the last group's surplus ones
-// repeat the last term's address and are not used).
+// C[16 ft .. + 15][sample] for the wave's feature tiles ft: Wt [16 ntiles][kp] in operand order, xs
+// [NS][kp + PAD] in LDS, kp a multiple of 32.  Eight loads are in flight at once (the last group's surplus
+// ones repeat the last term's address and are not used).  Where the tiles leave half of the waves idle and
+// `half` is given, waves ft and ft + 8 take half of the reduction each and add up there.
 template <class F>
-__device__ __forceinline__ void layer(const bf16_t *__restrict__ Wt, int ntiles, int kp, const bf16_t *xs, F epilogue)
+__device__ __forceinline__ void layer(const bf16_t *__restrict__ Wt, int ntiles, int kp, const bf16_t *xs, float *half, F epilogue)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nk = kp / 32;
     const bf16_t *b = xs + (lane & 15) * (kp + PAD) + 8 * (lane >> 4);
-    for (int ft = wave; ft < ntiles; ft += NWAVE) {
-        const bf16_t *a = Wt + (int64_t)(ft * 16 + (lane & 15)) * kp + 8 * (lane >> 4);
-        f32x4 acc = {};
-        for (int k = 0; k < nk; k += 8) {
+    const bool two = half && ntiles <= NWAVE / 2;
+    const int kb = two && wave >= NWAVE / 2 ? nk / 2 : 0, ke = two && wave < NWAVE / 2 ? nk / 2 : nk;
+    f32x4 acc = {};
+    for (int ft = two ? wave & (NWAVE / 2 - 1) : wave; ft < ntiles; ft += NWAVE) {
+        const bf16_t *a = Wt + (int64_t)ft * nk * 512 + lane * 8;
+        acc = {};
+        for (int k = kb; k < ke; k += 8) {
             bf16x8 av[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) { av[q] = load8(a + 32 * min(k + q, nk - 1)); }
+            for (int q = 0; q < 8; ++q) { av[q] = load8(a + 512 * min(k + q, nk - 1)); }
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                if (k + q < nk) { acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q], load8(b + 32 * (k + q)), acc, 0, 0, 0); }
+                if (k + q < ke) { acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q], load8(b + 32 * (k + q)), acc, 0, 0, 0); }
             }
         }
-        epilogue(ft * 16 + 4 * (lane >> 4), lane & 15, acc);
+        if (!two) { epilogue(ft * 16 + 4 * (lane >> 4), lane & 15, acc); }
+    }
+    if (two) { // (the same for the whole workgroup)
+        f32x4 *h = reinterpret_cast<f32x4 *>(half) + (wave & (NWAVE / 2 - 1)) * 64 + lane;
+        if (wave >= NWAVE / 2) { *h = acc; }
+        __syncthreads();
+        if (wave < ntiles) { epilogue(wave * 16 + 4 * (lane >> 4), lane & 15, acc + *h); }
     }
 }
 
@@ -96,7 +108,7 @@ __device__ __forceinline__ float sum16(float v) // over the 16 samples of a lane
 
 struct Lds
 {
-    float *z1, *z2, *out, *y, *part;
+    float *z1, *z2, *out, *y, *part, *half;
     bf16_t *x, *h1, *h2, *dout;
 };
 
@@ -115,6 +127,7 @@ __host__ __device__ inline size_t lds_layout(int d, int dp, int Hp, int Op, char
     L.out = (float *)take(sizeof(float) * Op * NS);
     L.y = (float *)take(sizeof(float) * d * NS);
     L.part = (float *)take(sizeof(float) * 2 * 8 * NS);
+    L.half = (float *)take(Hp <= 8 * NWAVE ? sizeof(f32x4) * 64 * (NWAVE / 2) : 0);
     L.x = (bf16_t *)take(sizeof(bf16_t) * NS * (dp + PAD));
     L.h1 = (bf16_t *)take(sizeof(bf16_t) * NS * (Hp + PAD));
     L.h2 = (bf16_t *)take(sizeof(bf16_t) * NS * (Hp + PAD));
@@ -135,7 +148,11 @@ __global__ __launch_bounds__(TPB) void k_step_tile(StepNet N, StepBatch B, StepW
     const bool ok = r < B.n;
     float *bias = w.bias + tile * (Op + 2 * Hp);
 
-    // the samples
+    // the samples; meanwhile an XCD's workgroups bring the weights, which the last update left in other
+    // XCDs' caches and in memory, into its L2, a slice each (blocks go round the eight XCDs)
+    const int slices = max(1, min(32, (int)(gridDim.x / 8))), line = (int)(blockIdx.x / 8) % slices + slices * tid;
+    uint32_t warm = 0;
+    if (line < N.lines) { warm = *reinterpret_cast<const uint32_t *>(N.W1t + (int64_t)line * 64); }
     {
         int64_t at = r, bt = r, sa = B.n, sb = B.n;
         const float *a = B.X, *b = B.Y;
@@ -144,9 +161,10 @@ __global__ __launch_bounds__(TPB) void k_step_tile(StepNet N, StepBatch B, StepW
             philox(0x30000000u, (uint32_t)r, (uint32_t)B.iter, (uint32_t)(B.iter >> 32), B.k0, B.k1, o);
             const int s1 = (int)(o[0] % (uint32_t)B.nsnap);
             int s2 = (int)(o[2] % (uint32_t)B.nsnap);
-            at = (int64_t)(o[1] % (uint64_t)B.W);
+            const uint32_t W = (uint32_t)B.W; // <= 2^30
+            at = (int64_t)(o[1] % W);
             const bool same = (float)(o[3] >> 24) * 0x1p-8f < B.same_frac;
-            bt = same ? at : (int64_t)((o[3] & 0xffffffu) % (uint64_t)B.W);
+            bt = same ? at : (int64_t)((o[3] & 0xffffffu) % W);
             if (same && B.nsnap > 1 && s2 == s1) { s2 = (s1 + 1) % B.nsnap; }
             a = B.snap + (int64_t)s1 * d * B.W;
             b = B.snap + (int64_t)s2 * d * B.W;
@@ -165,6 +183,7 @@ __global__ __launch_bounds__(TPB) void k_step_tile(StepNet N, StepBatch B, StepW
             if (j < d) { L.y[j * NS + s] = yv; }
         }
     }
+    asm volatile("" ::"v"(warm));
     __syncthreads();
 
     // forward: z = W h + b, h = silu(z)
@@ -181,11 +200,11 @@ __global__ __launch_bounds__(TPB) void k_step_tile(StepNet N, StepBatch B, StepW
             }
         };
     };
-    layer(N.W1t, Hp / 16, dp, L.x, hidden(L.z1, L.h1, w.H1, N.ob1));
+    layer(N.W1t, Hp / 16, dp, L.x, nullptr, hidden(L.z1, L.h1, w.H1, N.ob1));
     __syncthreads();
-    layer(N.W2t, Hp / 16, Hp, L.h1, hidden(L.z2, L.h2, w.H2, N.ob2));
+    layer(N.W2t, Hp / 16, Hp, L.h1, nullptr, hidden(L.z2, L.h2, w.H2, N.ob2));
     __syncthreads();
-    layer(N.W3t, Op / 16, Hp, L.h2, [&](int f, int c, f32x4 acc) {
+    layer(N.W3t, Op / 16, Hp, L.h2, nullptr, [&](int f, int c, f32x4 acc) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) { L.out[(f + i) * NS + c] = acc[i] + N.p[N.ob3 + f + i]; }
     });
@@ -282,9 +301,9 @@ __global__ __launch_bounds__(TPB) void k_step_tile(StepNet N, StepBatch B, StepW
             }
         };
     };
-    layer(N.W3, Hp / 16, Op, L.dout, back(L.z2, L.h2, w.dZ2, bias + Op));
+    layer(N.W3, Hp / 16, Op, L.dout, L.half, back(L.z2, L.h2, w.dZ2, bias + Op));
     __syncthreads();
-    layer(N.W2, Hp / 16, Hp, L.h2, back(L.z1, nullptr, w.dZ1, bias + Op + Hp));
+    layer(N.W2, Hp / 16, Hp, L.h2, nullptr, back(L.z1, nullptr, w.dZ1, bias + Op + Hp));
 }
 
 // one weight matrix: A, B as [tile][rows][16]; its gradient [na][nb] at off, row stride nb
@@ -359,18 +378,18 @@ __device__ __forceinline__ void put_copies(const StepNet &N, int64_t i, bf16_t v
     if (i >= N.oW3) {
         if (i >= N.ob3) { return; }
         const int e = (int)(i - N.oW3), h = e / Op, o = e % Op;
-        N.W3[e] = v;
-        N.W3t[(int64_t)o * N.Hp + h] = v;
+        N.W3[step_operand(h, o, Op)] = v;
+        N.W3t[step_operand(o, h, N.Hp)] = v;
     }
     else if (i >= N.oW2) {
         if (i >= N.ob2) { return; }
         const int e = (int)(i - N.oW2), k = e / H, f = e % H;
-        N.W2[k * N.Hp + f] = v;
-        N.W2t[f * N.Hp + k] = v;
+        N.W2[step_operand(k, f, N.Hp)] = v;
+        N.W2t[step_operand(f, k, N.Hp)] = v;
     }
     else if (i < N.ob1) {
         const int e = (int)i, k = e / H, f = e % H;
-        N.W1t[f * N.dp + k] = v;
+        N.W1t[step_operand(f, k, N.dp)] = v;
     }
 }
 

@@ -16,12 +16,20 @@ struct StepNet
     int d, H, K, Op, dp, Hp;
     int64_t oW1, ob1, oW2, ob2, oW3, ob3, npad;
     const float *p;
-    bf16_t *W1t;  // [Hp][dp]  the matrix instruction takes eight consecutive terms of the reduction
-    bf16_t *W2t;  // [Hp][Hp]  from a lane: forward reads the transposes,
-    bf16_t *W3t;  // [Op][Hp]
-    bf16_t *W2;   // [Hp][Hp]  backward the matrices themselves
-    bf16_t *W3;   // [Hp][Op]
+    // BF16 copies in the matrix instruction's operand order (step_operand): forward reads the transposes
+    // W1t [Hp][dp], W2t [Hp][Hp], W3t [Op][Hp], backward the matrices W2 [Hp][Hp], W3 [Hp][Op]; one
+    // array of `lines` 128-byte lines from W1t on
+    bf16_t *W1t, *W2t, *W3t, *W2, *W3;
+    int lines;
 };
+
+// where element (row, k) of a matrix with kp columns lies in operand order: blocks of 16 rows x 32 terms,
+// in a block the eight terms that lane row % 16 + 16 (k % 32 / 8) supplies -- a wave's load is one
+// contiguous KB
+__host__ __device__ inline int64_t step_operand(int row, int k, int kp)
+{
+    return ((int64_t)(row / 16 * (kp / 32) + k / 32) * 64 + row % 16 + 16 * (k % 32 / 8)) * 8 + k % 8;
+}
 
 // a minibatch: either X, Y [d][n] given, or (snap not null) pairs drawn from the snapshots
 // [nsnap][d][W]: context from one, target from another one (the context's walker with probability
@@ -49,8 +57,8 @@ struct StepWork
 
 // LDS of the tile kernel; the path serves every network whose tile fits a compute unit, since it is the
 // faster one up to that edge: an iteration, tiles against separate products (us), d 8 H 16 K 2 1024
-// samples 21 / 105, d 32 H 128 K 8 1024 samples 45 / 198, 65536 samples 631 / 2363, and at the edge
-// d 32 H 512 K 8 4096 samples 123 / 520, d 8 H 640 K 8 124 / 502
+// samples 20 / 105, d 32 H 128 K 8 1024 samples 32 / 198, 65536 samples 464 / 2363, and at the edge
+// d 32 H 512 K 8 4096 samples 84 / 520, d 8 H 640 K 8 80 / 502
 size_t step_lds(int d, int H, int Op);
 constexpr size_t STEP_LDS_MAX = 160 * 1024;
 // splits of the sample range in the weight gradients' products

@@ -1051,7 +1051,8 @@ __device__ __forceinline__ uint32_t bf16_bits(float v)
 // FAST32_REFRESH steps that never cross a block end; every chunk end closes all dwells and
 // recomputes |x|^2 from the position.  With X2 the per-coordinate state is 12 bytes in three
 // [coordinate][lane] arrays: x_i, the block sum of x_i^2, and (BF16 compensation, step of the last
-// change in the chunk) -- 48 KiB at d = 64, so three workgroups share a CU.
+// change in the chunk) -- 48 KiB at d = 64 for 64 walkers, so three workgroups share a CU (lanes32: four
+// of fewer walkers).
 // the running sums of one walker in k_fast32 (chunk steps jr, je: when the current |x|^2 and exp
 // values were set)
 struct Run32
@@ -1115,7 +1116,7 @@ __device__ __forceinline__ void step32(const FastArgs &A, float *xs, float *Ss, 
 }
 
 // Steps t and t + 1 (t even) of k_fast32 at chunk steps q, q + 1, as pair64 does for the FP64 chain
-template <int FL>
+template <int FL, bool NARROW>
 __device__ __forceinline__ void pair32(const FastArgs &A, float *xs, float *Ss, uint32_t *CJ, const float *as, Run32 &R,
                                        const uint32_t (&c)[6], uint32_t (&n)[6], uint64_t t, int q, uint32_t wid, float step,
                                        float inv_ediv, int lane)
@@ -1140,7 +1141,8 @@ __device__ __forceinline__ void pair32(const FastArgs &A, float *xs, float *Ss, 
         wA = c[4];
         wB = c[5];
     }
-    const int sA = vA * WAVE + lane, sB = vB * WAVE + lane;
+    const int LN = NARROW ? A.lanes : WAVE;
+    const int sA = vA * LN + lane, sB = vB * LN + lane;
     float xA = xs[sA], xB = xs[sB], SA = 0.f, SB = 0.f;
     uint32_t jA = 0u, jB = 0u;
     if (HX2) { SA = Ss[sA]; jA = CJ[sA]; SB = Ss[sB]; jB = CJ[sB]; }
@@ -1154,26 +1156,27 @@ __device__ __forceinline__ void pair32(const FastArgs &A, float *xs, float *Ss, 
     step32<FL>(A, xs, Ss, CJ, as, R, vB, sB, xB, SB, jB, uB, wB, q + 1, step, inv_ediv);
 }
 
-template <int FL>
+template <int FL, bool NARROW>
 __global__ __launch_bounds__(WAVE) void k_fast32(FastArgs A)
 {
     constexpr bool ACC = (FL & 7) != 0, HX2 = (FL & F_X2) != 0, HSUM = (FL & F_SUM) != 0, HEXP = (FL & F_EXP) != 0;
     extern __shared__ float lds32[];
     const int d = A.ndim;
     const int lane = threadIdx.x;
-    const int64_t w = (int64_t)blockIdx.x * WAVE + lane;
-    const bool live = w < A.W && (!A.wcount || w < *A.wcount);
+    const int LN = NARROW ? A.lanes : WAVE;
+    const int64_t w = (int64_t)blockIdx.x * LN + lane;
+    const bool live = (!NARROW || lane < LN) && w < A.W && (!A.wcount || w < *A.wcount);
     float *xs = lds32;                                                // [d][64] x_i
-    float *Ss = lds32 + d * WAVE;                                     // X2: [d][64] block sums of x_i^2
-    uint32_t *CJ = reinterpret_cast<uint32_t *>(lds32 + 2 * d * WAVE); // X2: [d][64] BF16 compensation << 16 | last change
-    float *as = lds32 + (HX2 ? 3 : 1) * d * WAVE;                     // [d]
+    float *Ss = lds32 + d * LN;                                     // X2: [d][64] block sums of x_i^2
+    uint32_t *CJ = reinterpret_cast<uint32_t *>(lds32 + 2 * d * LN); // X2: [d][64] BF16 compensation << 16 | last change
+    float *as = lds32 + (HX2 ? 3 : 1) * d * LN;                     // [d]
     for (int i = lane; i < d; i += WAVE) { as[i] = (float)A.a[i]; }
     float r = 0.f, rc = 0.f;                                          // |x|^2, Kahan-compensated
     if (live) {
         for (int i = 0; i < d; ++i) {
             const float v = (float)A.x64[(int64_t)i * A.W + w];
-            xs[i * WAVE + lane] = v;
-            if (HX2) { Ss[i * WAVE + lane] = 0.f; CJ[i * WAVE + lane] = 0u; }
+            xs[i * LN + lane] = v;
+            if (HX2) { Ss[i * LN + lane] = 0.f; CJ[i * LN + lane] = 0u; }
             kahan(r, rc, v * v);
         }
     }
@@ -1216,7 +1219,7 @@ __global__ __launch_bounds__(WAVE) void k_fast32(FastArgs A)
                 wp = pick(odd, p[5], p[4]);
                 ub = ws >> 8;
             }
-            const int slot = v * WAVE + lane;
+            const int slot = v * LN + lane;
             float xo = xs[slot], So = 0.f;
             uint32_t cj = 0u;
             if (HX2) { So = Ss[slot]; cj = CJ[slot]; }
@@ -1232,8 +1235,8 @@ __global__ __launch_bounds__(WAVE) void k_fast32(FastArgs A)
         if (uni) {
             if (((uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)t) & 1u) != 0u && q < len) { single(q); ++q; }
             for (; q + 4 <= len; q += 4) {
-                pair32<FL>(A, xs, Ss, CJ, as, R, p, nx, t, q, wid, step, inv_ediv, lane);
-                pair32<FL>(A, xs, Ss, CJ, as, R, nx, p, t + 2, q + 2, wid, step, inv_ediv, lane);
+                pair32<FL, NARROW>(A, xs, Ss, CJ, as, R, p, nx, t, q, wid, step, inv_ediv, lane);
+                pair32<FL, NARROW>(A, xs, Ss, CJ, as, R, nx, p, t + 2, q + 2, wid, step, inv_ediv, lane);
                 t += 4;
             }
         }
@@ -1249,20 +1252,20 @@ __global__ __launch_bounds__(WAVE) void k_fast32(FastArgs A)
             const double norm = 1. / B;
             float rx = 0.f, rxc = 0.f;
             for (int i = 0; i < d; ++i) {
-                const float v2 = xs[i * WAVE + lane];
+                const float v2 = xs[i * LN + lane];
                 if (HX2) {
-                    float Si = Ss[i * WAVE + lane];
-                    const uint32_t c2 = CJ[i * WAVE + lane];
+                    float Si = Ss[i * LN + lane];
+                    const uint32_t c2 = CJ[i * LN + lane];
                     float Ci = __uint_as_float(c2 & 0xFFFF0000u);
                     kahan_prod(Si, Ci, v2 * v2, (float)(len - (int)(c2 & 0xFFFFu)));
                     if (bend) {
                         A.d_x2[(b * d + i) * A.W + w] = ((double)Si - (double)Ci) * norm;
-                        Ss[i * WAVE + lane] = 0.f;
-                        CJ[i * WAVE + lane] = 0u;
+                        Ss[i * LN + lane] = 0.f;
+                        CJ[i * LN + lane] = 0u;
                     }
                     else {
-                        Ss[i * WAVE + lane] = Si;
-                        CJ[i * WAVE + lane] = bf16_bits(Ci) << 16;
+                        Ss[i * LN + lane] = Si;
+                        CJ[i * LN + lane] = bf16_bits(Ci) << 16;
                     }
                 }
                 kahan(rx, rxc, v2 * v2);
@@ -1282,16 +1285,33 @@ __global__ __launch_bounds__(WAVE) void k_fast32(FastArgs A)
             if (HEXP) { R.e = mcif::bexp(-R.r * inv_ediv); }
         }
     }
-    for (int i = 0; i < d; ++i) { A.x64[(int64_t)i * A.W + w] = (double)xs[i * WAVE + lane]; }
+    for (int i = 0; i < d; ++i) { A.x64[(int64_t)i * A.W + w] = (double)xs[i * LN + lane]; }
     A.ctr[w] = t;
     A.acc[w] = nacc;
     A.rej[w] = A.nsteps - nacc;
 }
 
-size_t lds_bytes(int prec, int ndim, bool x2)
+size_t lds_bytes(int prec, int ndim, bool x2, int lanes = WAVE)
 {
     if (prec == MCI_PREC_FP64) { return sizeof(double) * ((size_t)(x2 ? 2 : 1) * ndim * WAVE + ndim) + sizeof(float) * ndim; }
-    return sizeof(float) * ((size_t)(x2 ? 3 : 1) * ndim * WAVE + ndim);
+    return sizeof(float) * ((size_t)(x2 ? 3 : 1) * ndim * lanes + ndim);
+}
+
+// Walkers of a wave in k_fast32.  A wave alone on its SIMD takes the same time whatever lanes it fills, so
+// where the walkers' LDS keeps fewer than four waves of 64 on a compute unit (X2, d > 53), the most walkers
+// that leave room for four, one a SIMD, save whole rounds of workgroups.  The price is bank conflicts: in
+// rows of 64 a lane has its bank to itself, in narrower ones a step costs about a seventh more, so the
+// narrow wave is taken where the rounds saved are worth that.  Sampling 2,560 steps, ms, 64 walkers a wave /
+// narrow: d 64 (53 walkers) 50,000 walkers 1.23 / 0.64 (2 rounds / 1), 262,144 3.74 / 3.51 (6 / 5); d 56, 262,144 4.33 / 3.83 (6 / 5).
+int lanes32(int ndim, bool x2, int64_t W)
+{
+    constexpr int64_t CU_LDS = 160 * 1024, CUS = 256, SIMDS = 4;
+    const int64_t full = CU_LDS / (int64_t)lds_bytes(MCI_PREC_FP32, ndim, x2);
+    if (full >= SIMDS || full < 1) { return WAVE; }
+    const int64_t one = (int64_t)lds_bytes(MCI_PREC_FP32, ndim, x2, 1), per = (int64_t)lds_bytes(MCI_PREC_FP32, ndim, x2, 2) - one;
+    const int64_t lanes = (CU_LDS / SIMDS - (one - per)) / per;
+    auto rounds = [&](int64_t waves, int64_t l) { return (W + CUS * waves * l - 1) / (CUS * waves * l); };
+    return 8 * rounds(SIMDS, lanes) < 7 * rounds(full, WAVE) ? (int)lanes : WAVE;
 }
 
 // the one-lane all-coordinate kernels: k_fast64_allr holds up to ALL_DM coordinates in registers (no
@@ -1320,7 +1340,10 @@ template <int FL>
 void launch_fl(int prec, dim3 grid, size_t sh, hipStream_t s, const FastArgs &A)
 {
     if (prec == MCI_PREC_FP64) { hipLaunchKernelGGL(k_fast64<FL>, grid, dim3(WAVE), sh, s, A); }
-    else if constexpr ((FL & (F_FULL | F_MT)) == 0) { hipLaunchKernelGGL(k_fast32<FL>, grid, dim3(WAVE), sh, s, A); }
+    else if constexpr ((FL & (F_FULL | F_MT)) == 0) {
+        if (A.lanes < WAVE) { hipLaunchKernelGGL((k_fast32<FL, true>), grid, dim3(WAVE), sh, s, A); }
+        else { hipLaunchKernelGGL((k_fast32<FL, false>), grid, dim3(WAVE), sh, s, A); }
+    }
 }
 
 // All-coordinate launches that no group of lanes takes (group_shape): native streams with up to 16
@@ -1419,6 +1442,7 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     A.ubits = A.ibits > 0 ? (uint32_t)A.ibits : 0u;
     A.umask = 0xFFFFFFFFu >> A.ubits;
     A.uexp = (float)(32 - (int)A.ubits);
+    A.lanes = WAVE;
     A.blocksize = 1;
     A.nblocks = 0;
     A.d_x2 = A.d_x2sum = A.d_exp = nullptr;
@@ -1437,8 +1461,8 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     }
     if (!A.a && c.movetype != MCI_MOVE_ALL) { return MCI_E_INVALID_ARGUMENT; } // single-coordinate moves: explicit weights
     if (prec != MCI_PREC_FP64 && A.blocksize > INT32_MAX) { return MCI_E_INVALID_ARGUMENT; }
-    const dim3 grid((unsigned)((c.W + WAVE - 1) / WAVE));
     if (c.movetype == MCI_MOVE_ALL) {
+        const dim3 grid((unsigned)((c.W + WAVE - 1) / WAVE));
         if (prec != MCI_PREC_FP64 || (mt && (!c.mt || !c.mtp))) { return MCI_E_INVALID_ARGUMENT; }
         if (mt) { fl |= F_MT; }
         const size_t sha = lds_bytes_all(c.ndim, (fl & F_X2) != 0 && !(fl & F_FULL), mt);
@@ -1482,7 +1506,6 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         }
         return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
     }
-    const size_t sh = lds_bytes(prec, c.ndim, (fl & F_X2) != 0 && !(fl & F_FULL));
     if (mt) {
         if (prec != MCI_PREC_FP64 || (c.nvecs & (c.nvecs - 1)) != 0 || !c.mt || !c.mtp) { return MCI_E_INVALID_ARGUMENT; }
         fl |= F_MT;
@@ -1493,6 +1516,10 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         }
     }
     if (A.ibits >= 0) { fl |= F_P2; }
+    const bool recs = (fl & F_X2) != 0 && !(fl & F_FULL);
+    if (prec != MCI_PREC_FP64) { A.lanes = lanes32(c.ndim, recs, c.W); }
+    const size_t sh = lds_bytes(prec, c.ndim, recs, A.lanes);
+    const dim3 grid((unsigned)((c.W + A.lanes - 1) / A.lanes));
     switch (fl) {
     case 0: launch_fl<0>(prec, grid, sh, s, A); break;
     case 1: launch_fl<1>(prec, grid, sh, s, A); break;

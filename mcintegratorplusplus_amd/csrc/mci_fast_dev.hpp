@@ -17,6 +17,7 @@ struct FastArgs
 {
     int64_t W;
     int ndim;
+    int lanes;             // walkers of a wave (k_fast32)
     int64_t nsteps;
     uint32_t key0, key1;
     uint64_t *ctr;         // [W]

@@ -163,3 +163,24 @@ def test_fp32_precision_form_full_size():
     print("FP32 vs FP64 (chains coupled through the same words): max |diff|/err",
           np.max(np.abs(a32 - a64) / e64), "max rel", np.max(np.abs(a32 - a64) / np.abs(a64)), flush=True)
     assert np.all(np.abs(a32 - a64) < 0.25 * e64)
+
+
+@pytest.mark.parametrize("d", [54, 60, 64, 80])
+def test_fp32_narrow_waves_run_the_same_chains(d):
+    """with X2 and d > 53, walker counts past one round of wide waves run fewer walkers a wave; a walker's
+    chain is the same in both (independent walkers: the first W of W + 1 are those of W)"""
+    W = 49152 if d <= 71 else 32768  # three / two waves of 64 on each of 256 compute units
+    print("narrow waves", d, W, flush=True)
+    out = []
+    for n in (W, W + 1):
+        c = chain_setup("mci", fp32_cfg(d, [(OBS_X2, [], 32, 1, 1, ESTIM_UNCORR), (OBS_X2_SUM, [], 32, 1, 1, ESTIM_UNCORR)], ndecorr=3),
+                        nwalkers=n)
+        c.setRng(RNG_PHILOX)
+        c.setCoupling(COUPLING_INDEPENDENT)
+        c.setPrecision(PREC_FP32)
+        c.integrate(67 // 32 * 32, False, True)
+        out.append([np.asarray(v) for v in (*c.walkerResults(), c.getX(), *c.walkerAcceptance())])
+    for k, (a, b) in enumerate(zip(*out)):
+        axis = [i for i, m in enumerate(b.shape) if m == W + 1]
+        assert len(axis) == 1, (k, b.shape)
+        assert np.array_equal(a, np.take(b, np.arange(W), axis=axis[0])), k

@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "lib")
 LIB = os.path.join(OUT, "libmci_amd.so")
-SOURCES = ["mci_kernels.hip", "mci_fast.hip", "mci_fast_group.hip", "mci_batch.hip", "mci_mlp.hip", "mci_mlp_step.hip", "mci_lp.hip", "mci_noalloc.hip", "mci_em.hip", "mci_api.cpp",
+SOURCES = ["mci_kernels.hip", "mci_fast.hip", "mci_fast_group.hip", "mci_fast_duo.hip", "mci_batch.hip", "mci_mlp.hip", "mci_mlp_step.hip", "mci_lp.hip", "mci_noalloc.hip", "mci_em.hip", "mci_api.cpp",
            "mci_batch_api.cpp", "mci_lp_api.cpp", "mci_rtc.cpp"]
 ROOT = os.path.dirname(HERE)
 # headers the run-time build of the step kernels with the caller's device functors needs, under the

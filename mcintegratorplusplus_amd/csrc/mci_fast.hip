@@ -23,7 +23,11 @@
 // acceptance uniform on a 2^-24 grid, block sums as Kahan-compensated FP32 pairs, flushed to
 // FP64 for the FP64 estimators.  Every FP32 operation is correctly rounded and exp is the
 // library's own bexp (mci_f32math.hpp), so the CPU oracle reproduces the chain bit for bit.
+//
+// Other forms of the same chains: a walker on a group of lanes (mci_fast_group.hip: all-coordinate moves
+// and the reference streams), a producer wave beside the chain's (mci_fast_duo.hip: few walkers).
 #include "mci_fast_dev.hpp"
+#include "mci_fast_duo.hpp"
 #include "mci_fast_group.hpp"
 
 #include <type_traits>
@@ -32,27 +36,6 @@ namespace mcid
 {
 namespace
 {
-// Lemire index on [0, range) from word w0 (SRRDVecMove.hpp:78 through uniform_int_distribution), for
-// a range whose index the shared word does not hold: low = (w0 * range) mod 2^32 < thr = 2^32 mod
-// range rejects and draws from the extra-word stream of step t.  thr is computed on the host; a wave
-// vote skips the rare path.
-__device__ __forceinline__ int draw_lemire(uint32_t w0, uint32_t range, uint32_t thr, uint32_t wid, uint64_t t, uint32_t k0, uint32_t k1)
-{
-    uint64_t prod = (uint64_t)w0 * range;
-    if (__builtin_expect(__any((uint32_t)prod < thr), 0)) {
-        uint32_t low = (uint32_t)prod;
-        uint32_t kx = 0;
-        while (low < thr) {
-            const uint32_t k = 0x80000000u + (kx++);
-            uint32_t o[4];
-            philox(k >> 2, wid, (uint32_t)t, (uint32_t)(t >> 32), k0, k1, o[0], o[1], o[2], o[3]);
-            prod = (uint64_t)o[k & 3u] * range;
-            low = (uint32_t)prod;
-        }
-    }
-    return (int)(prod >> 32);
-}
-
 // FP64 chain.  One wave runs alone on its SIMD at the benchmark size (65,536 walkers =
 // 1,024 waves), so a step costs about 4 cycles per instruction of any kind and 16 per
 // v_mad_u64_u32 (quarter rate; a Philox call holds 20 of them).  The step is written to issue few
@@ -1516,6 +1499,10 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         }
     }
     if (A.ibits >= 0) { fl |= F_P2; }
+    if (prec == MCI_PREC_FP64 && (fl & (F_FULL | F_MT)) == 0 && duo_launch(c.ndim, (fl & F_P2) != 0, (fl & 7) != 0, A.blocksize, c.W)) {
+        if (!launch_duo(fl, A, s)) { return MCI_E_INVALID_ARGUMENT; }
+        return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
+    }
     const bool recs = (fl & F_X2) != 0 && !(fl & F_FULL);
     if (prec != MCI_PREC_FP64) { A.lanes = lanes32(c.ndim, recs, c.W); }
     const size_t sh = lds_bytes(prec, c.ndim, recs, A.lanes);

@@ -72,6 +72,27 @@ __device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, ui
 // can otherwise become a select of their addresses, which puts the array in scratch memory
 __device__ __forceinline__ uint32_t pick(bool on, uint32_t a, uint32_t b) { return b ^ ((a ^ b) & (0u - (uint32_t)on)); }
 
+// Lemire index on [0, range) from word w0 (SRRDVecMove.hpp:78 through uniform_int_distribution), for
+// a range whose index the shared word does not hold: low = (w0 * range) mod 2^32 < thr = 2^32 mod
+// range rejects and draws from the extra-word stream of step t.  thr is computed on the host; a wave
+// vote skips the rare path.
+__device__ __forceinline__ int draw_lemire(uint32_t w0, uint32_t range, uint32_t thr, uint32_t wid, uint64_t t, uint32_t k0, uint32_t k1)
+{
+    uint64_t prod = (uint64_t)w0 * range;
+    if (__builtin_expect(__any((uint32_t)prod < thr), 0)) {
+        uint32_t low = (uint32_t)prod;
+        uint32_t kx = 0;
+        while (low < thr) {
+            const uint32_t k = 0x80000000u + (kx++);
+            uint32_t o[4];
+            philox(k >> 2, wid, (uint32_t)t, (uint32_t)(t >> 32), k0, k1, o[0], o[1], o[2], o[3]);
+            prod = (uint64_t)o[k & 3u] * range;
+            low = (uint32_t)prod;
+        }
+    }
+    return (int)(prod >> 32);
+}
+
 // observable set of one launch (template flags: no per-step branches on them)
 // F_P2: the index is the shared word's top bits (a power-of-two range); F_FULL: Full accumulators (every
 // step's values stored)

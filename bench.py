@@ -188,8 +188,7 @@ def run_reference_streams():
     """The benchmark workload on the reference's random streams (one mt19937_64 per walker, the
     library's default, which reproduces the reference's chains bit for bit), on the specialised
     kernel and, for comparison, on the generic one: whole integrate and sampling kernel.  The
-    reference-stream kernel's traffic is the walkers' generator states: three outputs per step,
-    each reading two state words and writing one (24 B)."""
+    walkers' generator states stay in registers during a launch (read and written once)."""
     from mcintegratorplusplus_amd import MCI, constants as K
     sig = sigmas()
     exact = np.concatenate([sig ** 2, [np.sum(sig ** 2)]])
@@ -216,7 +215,6 @@ def run_reference_streams():
         out[name] = {"integrate_ms": ms, "walker_steps_per_s": W * NMC / (ms / 1000), "sampling_kernel_ms": kt[2],
                      "max_abs_z": float(np.max(np.abs(z)))}
         if name == "specialised":
-            out[name]["generator_state_gbps"] = 3 * 24 * W * NMC / (kt[2] / 1000) / 1e9
             out[name]["avg"] = avg
     out["speedup_specialised_vs_generic"] = out["generic"]["integrate_ms"] / out["specialised"]["integrate_ms"]
     out["specialised"].pop("avg")
@@ -227,8 +225,8 @@ def run_all_coordinate_moves():
     """The benchmark's target, observables and walkers with the reference's default move (every
     coordinate at once, one step size, SRRDAllMove) instead of the single-coordinate move, on both
     random-stream modes, on the specialised all-coordinate kernel and, for comparison, on the
-    generic one: whole integrate and sampling kernel.  A step reads and writes the walker's 16
-    coordinates in LDS; the native streams' Philox blocks (nine per step at d = 16) bound it."""
+    generic one: whole integrate and sampling kernel.  The walker's 16 coordinates are
+    in registers; the native streams' Philox blocks (nine per pair of steps at d = 16) bound it."""
     from mcintegratorplusplus_amd import MCI, constants as K
     sig = sigmas()
     exact = np.concatenate([sig ** 2, [np.sum(sig ** 2)]])
@@ -258,7 +256,7 @@ def run_all_coordinate_moves():
                        "max_abs_z": float(np.max(np.abs(z))), "acceptance": float(m.getAcceptanceRate())}
         r["speedup_specialised_vs_generic"] = r["generic"]["integrate_ms"] / r["specialised"]["integrate_ms"]
         out[rname] = r
-    # beyond the register width: d = 64 (the walker in LDS), native streams, the specialised kernel
+    # d = 64 (the walker on a group of lanes), native streams, the specialised kernel
     d64 = 64
     s64 = np.linspace(0.5, 2.0, d64)
     m = MCI(d64, W)

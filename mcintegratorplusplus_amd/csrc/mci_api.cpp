@@ -352,7 +352,7 @@ mci_status ensure_rtc(mci_ctx *c)
     const RtcFunctor mv{c->mv_name, c->mv_src};
     std::string text, msg;
     if (!rtc_program(fp, fo, dmove ? &mv : nullptr, text, msg)) { return fail(MCI_E_INVALID_ARGUMENT, "%s", msg.c_str()); }
-    if (text == c->rtc_text && c->rtc.sample[0]) { return MCI_OK; }
+    if (text == c->rtc_text && c->rtc.text) { return MCI_OK; }
     RtcKernels k;
     std::string log;
     const int st = rtc_get(text, k, log);
@@ -366,7 +366,7 @@ hipError_t sample_launch(const mci_ctx *c, const Chain &ch, int64_t nsteps, int 
                          const CalibCtrl *skip = nullptr)
 {
     c->mt_diverged = true;
-    if (c->rtc.sample[0]) { return rtc_launch_sample(c->rtc, ch, nsteps, acc, active, s, skip); }
+    if (c->rtc.text) { return rtc_launch_sample(c->rtc, ch, nsteps, acc, active, s, skip); }
     return launch_sample(ch, nsteps, acc, active, s, skip);
 }
 
@@ -374,7 +374,7 @@ hipError_t calibrate_indep_launch(const mci_ctx *c, const Chain &ch, int nfind, 
                                   hipStream_t s)
 {
     c->mt_diverged = true;
-    if (c->rtc.calibrate[0]) { return rtc_launch_calibrate_indep(c->rtc, ch, nfind, target, min_stat, dimSizes, s); }
+    if (c->rtc.text) { return rtc_launch_calibrate_indep(c->rtc, ch, nfind, target, min_stat, dimSizes, s); }
     return launch_calibrate_indep(ch, nfind, target, min_stat, dimSizes, s);
 }
 

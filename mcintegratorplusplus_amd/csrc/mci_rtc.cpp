@@ -27,16 +27,17 @@ namespace
 std::mutex g_mu;
 struct Loaded
 {
-    hipModule_t mod = nullptr;
+    hipModule_t mod[2] = {nullptr, nullptr};
     RtcKernels k;
 };
 std::map<std::pair<std::string, int>, Loaded> g_cache;
 
 // the walkers' state in HBM, in LDS
-const char *const kNames[4] = {"mcid::k_sample<false>", "mcid::k_sample<true>", "mcid::k_calibrate_indep<false>", "mcid::k_calibrate_indep<true>"};
+const char *const kNames[2][2] = {{"mcid::k_sample<false>", "mcid::k_calibrate_indep<false>"},
+                                  {"mcid::k_sample<true>", "mcid::k_calibrate_indep<true>"}};
 
-// compiles text; on success code holds the code object and names the kernels' lowered names
-int compile(const std::string &text, const std::string &arch, std::vector<char> &code, std::string (&names)[4], std::string &log)
+// compiles text's kernels of one kind; on success code holds the code object and names their lowered names
+int compile(const std::string &text, const std::string &arch, int lds, std::vector<char> &code, std::string (&names)[2], std::string &log)
 {
     hiprtcProgram p;
     if (hiprtcCreateProgram(&p, text.c_str(), "mci_device_functors.hip", rtc_nheaders, rtc_header_texts, rtc_header_names) !=
@@ -44,7 +45,7 @@ int compile(const std::string &text, const std::string &arch, std::vector<char> 
         log = "hiprtcCreateProgram failed";
         return MCI_E_DEVICE;
     }
-    for (const char *n : kNames) { hiprtcAddNameExpression(p, n); }
+    for (const char *n : kNames[lds]) { hiprtcAddNameExpression(p, n); }
     // the library's own flags: no contraction (bit-exact FP64 chains), correctly rounded FP32
     // divide and sqrt, no packed FP32 instructions
     const std::string off = "--offload-arch=" + arch;
@@ -67,9 +68,9 @@ int compile(const std::string &text, const std::string &arch, std::vector<char> 
     code.resize(cs);
     hiprtcGetCode(p, code.data());
     bool all = cs > 0;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2; ++i) {
         const char *l = nullptr;
-        hiprtcGetLoweredName(p, kNames[i], &l);
+        hiprtcGetLoweredName(p, kNames[lds][i], &l);
         names[i] = l ? l : "";
         all = all && !names[i].empty();
     }
@@ -163,44 +164,72 @@ bool rtc_program(const std::vector<RtcFunctor> &pdfs, const std::vector<RtcFunct
 int rtc_check(const std::string &text, const char *arch, std::string &log)
 {
     std::vector<char> code;
-    std::string names[4];
-    return compile(text, arch ? arch : "gfx950", code, names, log);
+    std::string names[2];
+    return compile(text, arch ? arch : "gfx950", 1, code, names, log);
 }
+
+namespace
+{
+// the kernels of one kind of L's program, compiled and loaded on the current device (g_mu held)
+int load(const std::string &text, int lds, Loaded &L, std::string &log)
+{
+    int dev = 0;
+    hipDeviceProp_t prop;
+    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) { return MCI_E_DEVICE; }
+    std::string arch = prop.gcnArchName;
+    const size_t colon = arch.find(':');
+    if (colon != std::string::npos) { arch.resize(colon); }
+    std::vector<char> code;
+    std::string names[2];
+    const int st = compile(text, arch, lds, code, names, log);
+    if (st != MCI_OK) { return st; }
+    if (hipModuleLoadData(&L.mod[lds], code.data()) != hipSuccess) {
+        log = "hipModuleLoadData failed";
+        return MCI_E_DEVICE;
+    }
+    hipFunction_t fs = nullptr, fc = nullptr;
+    if (hipModuleGetFunction(&fs, L.mod[lds], names[0].c_str()) != hipSuccess ||
+        hipModuleGetFunction(&fc, L.mod[lds], names[1].c_str()) != hipSuccess) {
+        log = "hipModuleGetFunction failed";
+        return MCI_E_DEVICE;
+    }
+    L.k.sample[lds] = fs;
+    L.k.calibrate[lds] = fc;
+    return MCI_OK;
+}
+
+// k's kernels of the kind a launch takes
+hipError_t need(const RtcKernels &k, int lds)
+{
+    if (k.sample[lds]) { return hipSuccess; }
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) { return hipErrorInvalidDevice; }
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_cache.find(std::make_pair(*k.text, dev));
+    if (it == g_cache.end()) { return hipErrorInvalidDevice; }
+    std::string log;
+    if (!it->second.k.sample[lds] && load(*k.text, lds, it->second, log) != MCI_OK) { return hipErrorInvalidKernelFile; }
+    k.sample[lds] = it->second.k.sample[lds];
+    k.calibrate[lds] = it->second.k.calibrate[lds];
+    return hipSuccess;
+}
+} // namespace
 
 int rtc_get(const std::string &text, RtcKernels &out, std::string &log)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { return MCI_E_DEVICE; }
     std::lock_guard<std::mutex> lk(g_mu);
-    auto key = std::make_pair(text, dev);
+    const auto key = std::make_pair(text, dev);
     auto it = g_cache.find(key);
-    if (it != g_cache.end()) {
-        out = it->second.k;
-        return MCI_OK;
+    if (it == g_cache.end()) {
+        Loaded L;
+        const int st = load(text, 1, L, log);
+        if (st != MCI_OK) { return st; }
+        it = g_cache.emplace(key, L).first;
+        it->second.k.text = &it->first.first;
     }
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) { return MCI_E_DEVICE; }
-    std::string arch = prop.gcnArchName;
-    const size_t colon = arch.find(':');
-    if (colon != std::string::npos) { arch.resize(colon); }
-    std::vector<char> code;
-    std::string names[4];
-    const int st = compile(text, arch, code, names, log);
-    if (st != MCI_OK) { return st; }
-    Loaded L;
-    if (hipModuleLoadData(&L.mod, code.data()) != hipSuccess) {
-        log = "hipModuleLoadData failed";
-        return MCI_E_DEVICE;
-    }
-    hipFunction_t *const f[4] = {&L.k.sample[0], &L.k.sample[1], &L.k.calibrate[0], &L.k.calibrate[1]};
-    for (int i = 0; i < 4; ++i) {
-        if (hipModuleGetFunction(f[i], L.mod, names[i].c_str()) != hipSuccess) {
-            log = "hipModuleGetFunction failed";
-            return MCI_E_DEVICE;
-        }
-    }
-    g_cache.emplace(key, L);
-    out = L.k;
+    out = it->second.k;
     return MCI_OK;
 }
 
@@ -209,6 +238,7 @@ hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, acc != 0);
+    if (const hipError_t e = need(k, st.in_lds)) { return e; }
     void *args[] = {&cc, &nsteps, &acc, &active, &skip};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
     return hipModuleLaunchKernel(k.sample[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
@@ -219,6 +249,7 @@ hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int n
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, false);
+    if (const hipError_t e = need(k, st.in_lds)) { return e; }
     void *args[] = {&cc, &nfind, &target, &min_stat, &dimSizes};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
     return hipModuleLaunchKernel(k.calibrate[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);

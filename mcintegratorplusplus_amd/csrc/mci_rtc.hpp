@@ -15,10 +15,12 @@ struct RtcFunctor
     std::string name, source;
 };
 
-// the generic step kernels of one module (loaded on one device): the walkers' state in HBM [0], in LDS [1]
+// the generic step kernels of one program (loaded on one device): the walkers' state in HBM [0], in LDS
+// [1].  The second kind is built with the program, the first (walkers too wide for LDS) by its first launch.
 struct RtcKernels
 {
-    hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
+    const std::string *text = nullptr; // the program (kept with the loaded modules)
+    mutable hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
 };
 
 // true when name is a C identifier

@@ -1,0 +1,37 @@
+"""The generic step kernels with the walkers' state in LDS (up to 80 KiB a wave: 6 d rows of 512 bytes here while
+sampling, 4 d while calibrating) and in HBM, for the catalogue and for device functors, against the specialised
+kernel: bit for bit the same at the last width in LDS, the first in HBM, where only calibration stays in LDS, and
+beyond."""
+import numpy as np
+import pytest
+
+import device_functors as DF
+from mcitest import COUPLING_INDEPENDENT, ESTIM_MJ, KERNELS_GENERIC, OBS_X2, PDF_GAUSS_DIAG, RNG_MT, Chain
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [26, 27, 35, 60])
+def test_state_in_lds_and_in_hbm(d):
+    print("state memory", d, flush=True)
+    a = 0.5 / np.random.default_rng(d).uniform(0.5, 2.0, d) ** 2
+    out = []
+    for name in ("specialised", "catalogue", "device"):
+        c = Chain("mci", d, 70)
+        c.setSeed(99)
+        c.setRng(RNG_MT)
+        c.setCoupling(COUPLING_INDEPENDENT)
+        c.setNdecorrelationSteps(20)
+        if name != "specialised":
+            c.setKernelPath(KERNELS_GENERIC)
+        if name == "device":
+            c.addSamplingFunctionDevice("diag", DF.DIAG, d, a)
+            c.addObservableDevice("xsq", DF.X2, d, (), 4, 1, True, ESTIM_MJ)
+        else:
+            c.addSamplingFunction(PDF_GAUSS_DIAG, a)
+            c.addObservable(OBS_X2, (), 4, 1, True, ESTIM_MJ)
+        first = c.integrate(4 * 32)
+        out.append((*first, *c.integrate(4 * 16, False, False), c.getX(), c.getWalkerSteps(), *c.walkerAcceptance(), *c.walkerResults()))
+    for other in out[1:]:
+        for k, (f, g) in enumerate(zip(out[0], other)):
+            assert np.array_equal(f, g), k

@@ -129,12 +129,10 @@ __device__ __forceinline__ double mt_symmetric(U64 w)
 // The generators of a wave's walkers in their groups' registers (groups of four lanes): element 4 i + g is
 // register i of lane g, so that elements 156 apart share a lane.
 constexpr int MT_NR = MT_N / 4;              // registers
-constexpr int MT_SEG = 6;                    // parts in which a round of the elements is made
-constexpr int MT_RS = MT_NR / MT_SEG;        // registers and
-constexpr int MT_CH = MT_N / MT_SEG;         // elements of a part
+constexpr int MT_RS = MT_NR / MT_SEG;        // registers of a part
 constexpr int MT_RP = WAVE / 4 + 2;          // an LDS row: one output of each walker, padded so that a walker's
                                              // lanes reading rows some way apart use different banks
-static_assert(MT_NR % MT_SEG == 0 && MT_N == 2 * MT_M && MT_M % 4 == 0, "");
+static_assert(MT_NR % MT_SEG == 0 && MT_N == MT_SEG * MT_CH && MT_N == 2 * MT_M && MT_M % 4 == 0, "");
 
 // the state rotated so that its next index is 0 (the same generator)
 __device__ __forceinline__ void mt_load(const FastArgs &A, int64_t w, int g, U64 (&m)[MT_NR])
@@ -189,47 +187,30 @@ __device__ __forceinline__ void mt_store(const FastArgs &A, int64_t w, int g, co
     }
 }
 
-// Runs nsteps steps of `per` outputs each: step(row) takes them from consecutive rows (MT_RP apart) from
-// `row`.  A part's outputs go to rows LEFT .. LEFT + MT_CH - 1, after the up to per - 1 that are left over,
-// which move to the rows before LEFT, so that a step's outputs are always consecutive.
+// Runs nsteps steps of `per` outputs each in the order of mt_parts (mci_fast_plan.hpp): step(row) takes them
+// from consecutive rows (MT_RP apart) from `row`.
 template <int LEFT, class F>
 __device__ __forceinline__ void mt_run(const FastArgs &A, int64_t w, int g, uint64_t *mine, int per, F step)
 {
     U64 m[MT_NR];
     mt_load(A, w, g, m);
-    int kc = LEFT, avail = 0, kt = 0;  // row of the next output, outputs waiting, next element
-    for (int64_t done = 0; done < A.nsteps;) {
-        const int64_t stretch = A.nsteps - done < FAST_MAX_CHUNK ? A.nsteps - done : FAST_MAX_CHUNK;
-        int left = (int)stretch;
-        done += stretch;
-        while (left > 0) {
-#pragma unroll
-            for (int q = 0; q < MT_SEG; ++q) {
-                if (left > 0) {
-                    if constexpr (LEFT == 4) {
-                        if (g < avail) { mine[(LEFT - avail + g) * MT_RP] = mine[(kc + g) * MT_RP]; }
-                    }
-                    else {
-                        for (int r = g; r < avail; r += 4) { mine[(LEFT - avail + r) * MT_RP] = mine[(kc + r) * MT_RP]; }
-                    }
-                    kc = LEFT - avail;
-                    mt_part(m, q, g, mine + LEFT * MT_RP);
-                    wave_order();
-                    avail += MT_CH;
-                    kt = (q + 1) * MT_CH;
-                    while (avail >= per && left > 0) {
-                        const uint64_t *row = mine + kc * MT_RP;
-                        kc += per;
-                        avail -= per;
-                        --left;
-                        step(row);
-                    }
-                    wave_order();
-                }
+    const MtEnd end = mt_parts<LEFT>(
+        A.nsteps, per,
+        [&](int from, int to, int n) {
+            wave_order();
+            if constexpr (LEFT == 4) {
+                if (g < n) { mine[(to + g) * MT_RP] = mine[(from + g) * MT_RP]; }
             }
-        }
-    }
-    mt_store(A, w, g, m, kt, avail);
+            else {
+                for (int r = g; r < n; r += 4) { mine[(to + r) * MT_RP] = mine[(from + r) * MT_RP]; }
+            }
+        },
+        [&](int q) {
+            mt_part(m, q, g, mine + LEFT * MT_RP);
+            wave_order();
+        },
+        [&](int row) { step(mine + row * MT_RP); });
+    mt_store(A, w, g, m, end.next, end.over);
 }
 
 // q / div, the division (a dozen FP64 instructions) left out where it changes nothing: by 1, the default
@@ -563,13 +544,11 @@ __global__ __launch_bounds__(WAVE, S <= 4 ? 2 : 1) void k_fast64_vec4(FastArgs A
     double e = 0.0, Sr = 0.0, Se = 0.0;
     if (HEXP) { e = exp(-(ordered(q2) / A.exp_div)); }
     int64_t nacc = 0, inblk = 0;
-    int na = 0;  // accepted steps of the block or, without sums, of the run so far (below 2^31 by the flush)
     char *rx = reinterpret_cast<char *>(A.d_x2), *rs = reinterpret_cast<char *>(A.d_x2sum), *re = reinterpret_cast<char *>(A.d_exp);
     const int64_t w8 = W * 8, rowx = w8 * d;
     const uint32_t off = (uint32_t)w * 8u;
     auto put = [](char *row, uint32_t o, double v) { *reinterpret_cast<double *>(row + o) = v; };
     const uint32_t ibits = (uint32_t)A.ibits, vshift = (uint32_t)A.vshift;
-    int flush = 1 << 30;
     mt_run<4>(A, w, g, st + wl, 3, [&](const uint64_t *row) {
         const U64 oi = halves(row[0]), op = halves(row[MT_RP]), uw = halves(row[2 * MT_RP]);
         const uint32_t v = __builtin_amdgcn_ubfe(apart(oi.hi), vshift, ibits);
@@ -596,17 +575,12 @@ __global__ __launch_bounds__(WAVE, S <= 4 ? 2 : 1) void k_fast64_vec4(FastArgs A
             }
         }
         acc = acc && own;
-        na += acc ? 1 : 0;
+        nacc += acc ? 1 : 0;
         const int to = acc ? slot : -1;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             x[s] = to == s ? xn : x[s];
             q2[s] = to == s ? xn2 : q2[s];
-        }
-        if (--flush == 0) {
-            nacc += na;
-            na = 0;
-            flush = 1 << 30;
         }
         if (!(ACC || FULL)) { return; }
         double q = 0.0;
@@ -663,7 +637,6 @@ __global__ __launch_bounds__(WAVE, S <= 4 ? 2 : 1) void k_fast64_vec4(FastArgs A
             inblk = 0;
         }
     });
-    nacc += na;
     // the walker's accepted steps: the sum over its lanes
     auto plus = [&](auto ctrl) {
         constexpr int C = decltype(ctrl)::value;

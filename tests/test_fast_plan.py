@@ -108,3 +108,86 @@ def test_shared_index_bits_match_the_oracle(tmp_path):
         assert lib.orc_shared_index_bits(c.ctx) == rows[d][1], d
         c.setTrialMoveMultistep(2, 0, 1, 1, None)
         assert lib.orc_shared_index_bits(c.ctx) == -1
+
+
+PARTS = r"""
+#include "mci_fast_plan.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+// a run of n steps on a buffer whose rows hold the running number of the output they were given
+template <int LEFT> const char *run(int64_t n, int per)
+{
+    std::vector<int64_t> row(LEFT + mcid::MT_CH, -1);
+    int64_t made = 0, taken = 0;
+    const char *bad = nullptr;
+    auto in = [&](int r) { if (r < 0 || r >= (int)row.size()) { bad = "row out of range"; } return bad == nullptr; };
+    const mcid::MtEnd end = mcid::mt_parts<LEFT>(
+        n, per,
+        [&](int from, int to, int k) {
+            if (k > LEFT) { bad = "more left over than the rows before a part"; return; }
+            for (int r = 0; r < k; ++r) {
+                if (in(from + r) && in(to + r)) { row[to + r] = row[from + r]; }
+            }
+        },
+        [&](int q) {
+            if (q != (made / mcid::MT_CH) % mcid::MT_SEG) { bad = "part out of order"; }
+            for (int j = 0; j < mcid::MT_CH; ++j) { row[LEFT + j] = made++; }
+        },
+        [&](int r) {
+            for (int j = 0; j < per; ++j) {
+                if (in(r + j) && row[r + j] != taken + j) { bad = "not the next output"; }
+            }
+            taken += per;
+        });
+    if (taken != n * per) { return "steps"; }
+    if (end.over != made - taken || end.over < 0 || end.over >= per + mcid::MT_CH) { return "outputs left over"; }
+    if (n > 0 && end.next != (made - 1) % 312 + 1) { return "next element"; }
+    return bad ? bad : "ok";
+}
+int main(int argc, char **argv)
+{
+    if (argc > 1) { // a long run: only the count of its steps and the parts' order
+        int64_t steps = 0, parts = 0, wrong = 0;
+        const mcid::MtEnd end = mcid::mt_parts<4>(std::atoll(argv[1]), 3, [](int, int, int) {},
+                                                  [&](int q) { wrong += q != parts++ % mcid::MT_SEG; }, [&](int) { ++steps; });
+        std::printf("%lld %lld %lld %d\n", (long long)steps, (long long)parts, (long long)wrong, end.over);
+        return 0;
+    }
+#define SHAPE(S) for (int d = 1; d <= 4 * S; ++d) { for (int64_t n : N) { report(run<4 * S>(n, d + 1), d + 1, n); } }
+    std::vector<int64_t> N;
+    for (int64_t n = 0; n <= 700; ++n) { N.push_back(n); }
+    N.push_back(20011);
+    int fails = 0;
+    auto report = [&](const char *r, int per, int64_t n) {
+        if (r[0] != 'o' || r[1] != 'k') { if (fails++ < 10) { std::printf("%d outputs a step, %lld steps: %s\n", per, (long long)n, r); } }
+    };
+    SHAPE(1) SHAPE(2) SHAPE(3) SHAPE(4) SHAPE(6) SHAPE(8) SHAPE(12) SHAPE(16)
+    for (int64_t n : N) { report(run<4>(n, 3), 3, n); }
+    std::printf("%d failures\n", fails);
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def parts(tmp_path_factory):
+    d = tmp_path_factory.mktemp("parts")
+    (d / "parts.cpp").write_text(PARTS)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-I", CSRC, str(d / "parts.cpp"), "-o", str(d / "parts")], check=True)
+    return lambda *a: subprocess.run([str(d / "parts"), *map(str, a)], capture_output=True, text=True, check=True).stdout
+
+
+def test_generator_parts_follow_each_other_in_order(parts):
+    """The lane-group kernels' order of making and taking a reference-stream generator's outputs
+    (mt_parts): for every number of outputs a step takes in every form, and runs that end at every place
+    of a part and of several rounds, each step takes the next outputs, parts are made in their order,
+    every row lies in the buffer, and the end says which outputs were made and not taken."""
+    assert parts() == "0 failures\n"
+
+
+def test_generator_parts_in_a_run_past_32_bits(parts):
+    """... and a run of more than 2^32 steps is one run: it neither stops short nor starts a part anew."""
+    n = 2 ** 32 + 3
+    made = -(-3 * n // 52)
+    assert parts(n) == f"{n} {made} 0 {52 * made - 3 * n}\n"

@@ -55,3 +55,30 @@ def check(rng, d, W, veclen, blocksize, obs):
         out[path] = (*first, *second, c.getX(), c.getWalkerSteps(), *c.walkerAcceptance(), *c.walkerResults(), *data)
     for k, (f, g) in enumerate(zip(out["groups"], out["generic"])):
         assert np.array_equal(f, g), k
+
+
+# (outputs a step, coordinates, moves) and run lengths that end just before, at and after a part (52 outputs), a
+# round (312) and two: the outputs left over go back to the state through element 0 and beyond
+ENDS = [(3, 16, 1, (17, 18, 34, 35, 103, 104, 105, 208, 209)), (4, 3, 0, (12, 13, 14, 77, 78, 79, 156)),
+        (13, 12, 0, (3, 4, 5, 23, 24, 25, 48)), (52, 51, 0, (1, 2, 5, 6, 7)), (65, 64, 0, (1, 2, 4, 5, 24, 25))]
+
+
+@pytest.mark.parametrize("per,d,veclen,runs", ENDS)
+def test_runs_that_end_at_the_edges_of_the_generator_parts(per, d, veclen, runs):
+    """each run continues the streams of the one before, so a state put back wrongly shows in the next"""
+    cfg = dict(ndim=d, seed=9 + d, ndecorr=0, nfind=0, move=(0, veclen, 1, None),
+               pdfs=[(PDF_GAUSS_DIAG, 0.5 / np.random.default_rng(d).uniform(0.5, 2.0, d) ** 2)], obs=[(OBS_X2, [], 0, 1, 0, ESTIM_NOOP)])
+    out = {}
+    for path in ("groups", "generic"):
+        c = chain_setup("mci", cfg, nwalkers=21)
+        c.setRng(RNG_MT)
+        c.setCoupling(1)
+        c.setMRT2Step(0.7)
+        if path == "generic":
+            c.setKernelPath(KERNELS_GENERIC)
+        out[path] = []
+        for n in runs:
+            print("generator parts", per, d, path, n, flush=True)
+            out[path] += [*c.integrate(n, False, False), c.getX(), *c.walkerAcceptance()]
+    for k, (f, g) in enumerate(zip(out["groups"], out["generic"])):
+        assert np.array_equal(f, g), k

@@ -112,9 +112,10 @@ __global__ __launch_bounds__(2 * WAVE) void k_fast64_duo(FastArgs A)
         }
         if (A.pend->done) { return; }
     }
+    const bool live = listed && (!A.active || A.active[w]);
+    if (__builtin_amdgcn_ballot_w64(live) == 0) { return; } // no walker here (the same 64 in both waves)
     // (lanes without a walker run along on a state of their own and store nothing: every wave reaches
     // every barrier)
-    const bool live = listed && (!A.active || A.active[w]);
     Draw *ring = reinterpret_cast<Draw *>(lds) + lane;  // [2][CH][64]
     double *state = lds + 2 * CH * WAVE * 2;
     double *as = state + (REC ? 2 : 1) * d * WAVE;

@@ -6,7 +6,7 @@ both sides of the rule, odd counters, and launches that continue the streams."""
 import numpy as np
 import pytest
 
-from mcitest import (ESTIM_NOOP, ESTIM_UNCORR, KERNELS_GENERIC, OBS_EXP_X2, OBS_X2, OBS_X2_SUM, PDF_GAUSS_DIAG, RNG_PHILOX, chain_setup)
+from mcitest import (COUPLING_INDEPENDENT, ESTIM_NOOP, ESTIM_UNCORR, KERNELS_GENERIC, OBS_EXP_X2, OBS_X2, OBS_X2_SUM, PDF_GAUSS_DIAG, RNG_PHILOX, chain_setup, dptr)
 
 pytestmark = pytest.mark.gpu
 SETS = [[OBS_X2], [OBS_X2_SUM], [OBS_X2, OBS_X2_SUM], [OBS_EXP_X2], [OBS_X2, OBS_X2_SUM, OBS_EXP_X2]]
@@ -42,3 +42,27 @@ def test_two_waves_run_the_generic_chain(d, W, block):
     # its coordinate's largest x^2 in the block: 2^-53 times their number times that, far below 1e-12 here
     for f, g in zip(out["waves"][1], out["generic"][1]):
         assert np.allclose(f, g, rtol=1e-10, atol=1e-12)
+
+
+def test_groups_without_a_walker_left_end_at_once():
+    """Independent calibration enqueues as many iterations as the last one took; those after the last walker has
+    left its loop hold no walker and take no steps.  64 iterations from a step far too small (doubled about 50
+    times, then five more), then from the step that they found (five to a dozen hold a walker): the rest of an
+    idle iteration (its compaction and bookkeeping) is about a tenth of one with walkers, so the whole is below
+    half; with idle iterations that run, the two take the same time."""
+    d, W = 128, 70
+    cfg = dict(ndim=d, seed=5, ndecorr=0, nfind=-64, move=(0, 1, 1, None), pdfs=[(PDF_GAUSS_DIAG, np.full(d, 0.5))],
+               obs=[(OBS_X2, [], 0, 1, 0, ESTIM_NOOP)])
+    c = chain_setup("mci", cfg, nwalkers=W)
+    c.setRng(RNG_PHILOX)
+    c.setCoupling(COUPLING_INDEPENDENT)
+    took = []
+    for small in (True, True, False):  # the first loads the kernels and finds the number of iterations
+        print("calibration from", "a small step" if small else "the step found", flush=True)
+        if small:
+            c.setMRT2Step(1e-15)
+        c.integrate(0, True, False)
+        t = np.zeros(5)
+        c.call("get_timings", dptr(t), 5)
+        took.append(t[0])
+    assert took[2] < 0.5 * took[1], took

@@ -45,6 +45,10 @@ struct DBuf
         if (p) { (void)hipFree(p); p = nullptr; n = 0; }
         hipError_t e = hipMalloc((void **)&p, std::max<size_t>(m, 1) * sizeof(T));
         if (e == hipSuccess) { n = m; }
+        else {
+            p = nullptr;
+            (void)hipGetLastError(); // reported by the return: not again by the next launch's check
+        }
         return e;
     }
 };

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import device_functors as DF
-from mcitest import COUPLING_INDEPENDENT, ESTIM_MJ, KERNELS_GENERIC, OBS_X2, PDF_GAUSS_DIAG, RNG_MT, Chain
+from mcitest import COUPLING_INDEPENDENT, ESTIM_MJ, ESTIM_NOOP, KERNELS_GENERIC, OBS_X2, PDF_GAUSS_DIAG, RNG_MT, Chain
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,20 @@ def test_state_in_lds_and_in_hbm(d):
     for other in out[1:]:
         for k, (f, g) in enumerate(zip(out[0], other)):
             assert np.array_equal(f, g), k
+
+
+def test_a_run_too_large_for_the_card_is_an_error_once():
+    """traces of 348 GB are refused, and the calls after that are not"""
+    d, W = 16, 1024
+    c = Chain("mci", d, W)
+    c.setSeed(99)
+    c.setRng(RNG_MT)
+    c.setNdecorrelationSteps(20)
+    c.addSamplingFunction(PDF_GAUSS_DIAG, np.full(d, 0.5))
+    c.addObservable(OBS_X2, (), 1, 1, False, ESTIM_NOOP)
+    print("traces of 348 GB", flush=True)
+    with pytest.raises(RuntimeError):
+        c.integrate(2_660_000, False, False)
+    print("and of a few steps", flush=True)
+    avg, _ = c.integrate(8, False, False)
+    assert np.all(np.isfinite(avg))

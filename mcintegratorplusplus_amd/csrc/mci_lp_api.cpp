@@ -164,6 +164,7 @@ mci_status mlp_step_reserve(mci_mlp *n, int64_t ns)
 {
     HIPCHK(n->loss.ensure((size_t)ns));
     if (ns <= n->step_cap) { return MCI_OK; }
+    n->step_cap = 0; // until every buffer has grown: one that cannot loses what it held
     const mcim::StepNet &N = n->step;
     const size_t rows = (size_t)((ns + mcim::STEP_NS - 1) / mcim::STEP_NS * mcim::STEP_NS);
     HIPCHK(n->tiles.ensure(rows * (size_t)(N.dp + 4 * N.Hp + N.Op)));
@@ -184,6 +185,7 @@ mci_status mlp_step_reserve(mci_mlp *n, int64_t ns)
 mci_status mlp_reserve(mci_mlp *n, int64_t cap)
 {
     if (cap <= n->cap) { return MCI_OK; }
+    n->cap = 0; // as in mlp_step_reserve
     const int d = n->d, H = n->H, Op = n->Op;
     HIPCHK(n->X.ensure((size_t)d * cap));
     HIPCHK(n->Y.ensure((size_t)d * cap));

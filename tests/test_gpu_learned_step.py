@@ -73,3 +73,21 @@ def test_training_leaves_the_copies_of_its_parameters():
     x = rng.normal(0.0, 2.0, (40, d)).astype(np.float32)
     a, b = net.lossGrad(x, x[::-1].copy()), other.lossGrad(x, x[::-1].copy())
     assert a[0] == b[0] and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("d,H,K,n", [
+    (1, 800, 1, 48_000_000),   # sample tiles: 6.6 KB of workspace a sample, 316 GB
+    (1, 1024, 1, 80_000_000),  # the products one by one: 4 KB a sample of the first layer's outputs, 328 GB
+])
+def test_a_minibatch_too_large_leaves_the_network_usable(d, H, K, n):
+    """a workspace that cannot grow is an error, and later minibatches do not use what it held before"""
+    from mcintegratorplusplus_amd.learned import Network
+    print("workspace", d, H, K, n, flush=True)
+    net = Network(d, H, K, seed=3)
+    x = np.random.default_rng(1).normal(0.0, 2.0, (64, d)).astype(np.float32)
+    loss, g = net.lossGrad(x, x[::-1].copy())
+    big = np.zeros((n, d), np.float32)
+    with pytest.raises(RuntimeError):
+        net.lossGrad(big, big)
+    l2, g2 = net.lossGrad(x, x[::-1].copy())
+    assert l2 == loss and np.array_equal(g, g2)

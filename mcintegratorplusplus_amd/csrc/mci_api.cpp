@@ -332,8 +332,23 @@ int obs_uid(const mci_ctx *c, size_t i)
     return c->obs[i].kind == MCI_OBS_DEVICE ? u : 0;
 }
 
+// the kinds of step kernels an integrate launches (bits of rtc_get): calibration and fixed decorrelation
+// without observables, sampling with all of them; the equilibration's are in between
+int rtc_kinds(const mci_ctx *c)
+{
+    Chain ch;
+    std::memset(&ch, 0, sizeof ch);
+    ch.ndim = c->ndim;
+    ch.nproto = nproto_total(c);
+    int kinds = 1 << state_lds_of(ch, false).in_lds;
+    ch.nobs = (int)c->obs.size();
+    for (int i = 0; i < ch.nobs; ++i) { ch.obs[i].nobs = c->obs[(size_t)i].nobs; }
+    kinds |= 1 << state_lds_of(ch, true).in_lds;
+    return kinds;
+}
+
 // the step kernels for the context's device functors: built (or taken from the process's cache)
-// when the set of functors changed; none: the library's own kernels
+// when the set of functors, or the width of the state, changed; none: the library's own kernels
 mci_status ensure_rtc(mci_ctx *c)
 {
     std::vector<RtcFunctor> fp, fo;
@@ -352,10 +367,11 @@ mci_status ensure_rtc(mci_ctx *c)
     const RtcFunctor mv{c->mv_name, c->mv_src};
     std::string text, msg;
     if (!rtc_program(fp, fo, dmove ? &mv : nullptr, text, msg)) { return fail(MCI_E_INVALID_ARGUMENT, "%s", msg.c_str()); }
-    if (text == c->rtc_text && c->rtc.text) { return MCI_OK; }
+    const int kinds = rtc_kinds(c);
+    if (text == c->rtc_text && c->rtc.has(kinds)) { return MCI_OK; }
     RtcKernels k;
     std::string log;
-    const int st = rtc_get(text, k, log);
+    const int st = rtc_get(text, kinds, k, log);
     if (st != MCI_OK) { return fail(st, "building the device functors failed:\n%s", log.c_str()); }
     c->rtc = k;
     c->rtc_text = text;
@@ -366,7 +382,7 @@ hipError_t sample_launch(const mci_ctx *c, const Chain &ch, int64_t nsteps, int 
                          const CalibCtrl *skip = nullptr)
 {
     c->mt_diverged = true;
-    if (c->rtc.text) { return rtc_launch_sample(c->rtc, ch, nsteps, acc, active, s, skip); }
+    if (c->rtc.any()) { return rtc_launch_sample(c->rtc, ch, nsteps, acc, active, s, skip); }
     return launch_sample(ch, nsteps, acc, active, s, skip);
 }
 
@@ -374,7 +390,7 @@ hipError_t calibrate_indep_launch(const mci_ctx *c, const Chain &ch, int nfind, 
                                   hipStream_t s)
 {
     c->mt_diverged = true;
-    if (c->rtc.text) { return rtc_launch_calibrate_indep(c->rtc, ch, nfind, target, min_stat, dimSizes, s); }
+    if (c->rtc.any()) { return rtc_launch_calibrate_indep(c->rtc, ch, nfind, target, min_stat, dimSizes, s); }
     return launch_calibrate_indep(ch, nfind, target, min_stat, dimSizes, s);
 }
 

@@ -197,39 +197,20 @@ int load(const std::string &text, int lds, Loaded &L, std::string &log)
     L.k.calibrate[lds] = fc;
     return MCI_OK;
 }
-
-// k's kernels of the kind a launch takes
-hipError_t need(const RtcKernels &k, int lds)
-{
-    if (k.sample[lds]) { return hipSuccess; }
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) { return hipErrorInvalidDevice; }
-    std::lock_guard<std::mutex> lk(g_mu);
-    auto it = g_cache.find(std::make_pair(*k.text, dev));
-    if (it == g_cache.end()) { return hipErrorInvalidDevice; }
-    std::string log;
-    if (!it->second.k.sample[lds] && load(*k.text, lds, it->second, log) != MCI_OK) { return hipErrorInvalidKernelFile; }
-    k.sample[lds] = it->second.k.sample[lds];
-    k.calibrate[lds] = it->second.k.calibrate[lds];
-    return hipSuccess;
-}
 } // namespace
 
-int rtc_get(const std::string &text, RtcKernels &out, std::string &log)
+int rtc_get(const std::string &text, int kinds, RtcKernels &out, std::string &log)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { return MCI_E_DEVICE; }
     std::lock_guard<std::mutex> lk(g_mu);
-    const auto key = std::make_pair(text, dev);
-    auto it = g_cache.find(key);
-    if (it == g_cache.end()) {
-        Loaded L;
-        const int st = load(text, 1, L, log);
+    Loaded &L = g_cache[std::make_pair(text, dev)];
+    for (int lds = 0; lds < 2; ++lds) {
+        if (!(kinds & (1 << lds)) || L.k.sample[lds]) { continue; }
+        const int st = load(text, lds, L, log);
         if (st != MCI_OK) { return st; }
-        it = g_cache.emplace(key, L).first;
-        it->second.k.text = &it->first.first;
     }
-    out = it->second.k;
+    out = L.k;
     return MCI_OK;
 }
 
@@ -238,7 +219,7 @@ hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, acc != 0);
-    if (const hipError_t e = need(k, st.in_lds)) { return e; }
+    if (!k.sample[st.in_lds]) { return hipErrorInvalidDeviceFunction; }
     void *args[] = {&cc, &nsteps, &acc, &active, &skip};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
     return hipModuleLaunchKernel(k.sample[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
@@ -249,7 +230,7 @@ hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int n
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, false);
-    if (const hipError_t e = need(k, st.in_lds)) { return e; }
+    if (!k.calibrate[st.in_lds]) { return hipErrorInvalidDeviceFunction; }
     void *args[] = {&cc, &nfind, &target, &min_stat, &dimSizes};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
     return hipModuleLaunchKernel(k.calibrate[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);

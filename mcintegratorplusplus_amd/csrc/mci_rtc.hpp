@@ -16,11 +16,12 @@ struct RtcFunctor
 };
 
 // the generic step kernels of one program (loaded on one device): the walkers' state in HBM [0], in LDS
-// [1].  The second kind is built with the program, the first (walkers too wide for LDS) by its first launch.
+// [1] (state_lds_of).  Each kind is a build of its own: a program is built in the kinds its chain takes.
 struct RtcKernels
 {
-    const std::string *text = nullptr; // the program (kept with the loaded modules)
-    mutable hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
+    hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
+    bool any() const { return sample[0] || sample[1]; }
+    bool has(int kinds) const { return (!(kinds & 1) || sample[0]) && (!(kinds & 2) || sample[1]); }
 };
 
 // true when name is a C identifier
@@ -31,10 +32,12 @@ bool rtc_valid_name(const std::string &name);
 // move: the caller's trial move (or null)
 bool rtc_program(const std::vector<RtcFunctor> &pdfs, const std::vector<RtcFunctor> &obs, const RtcFunctor *move, std::string &text,
                  std::string &msg);
-// compiles text for arch (e.g. "gfx950") without loading it; log: the compiler's messages
+// compiles text for arch (e.g. "gfx950") without loading it; log: the compiler's messages.  One kind: the
+// functors are the same text in both.
 int rtc_check(const std::string &text, const char *arch, std::string &log);
-// the kernels of text on the current device: compiled and loaded once per text and device
-int rtc_get(const std::string &text, RtcKernels &out, std::string &log);
+// the kernels of text on the current device, those of the given kinds (bit 0: HBM, bit 1: LDS) among
+// them: compiled and loaded once per text, device and kind
+int rtc_get(const std::string &text, int kinds, RtcKernels &out, std::string &log);
 hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps, int acc, const uint8_t *active, hipStream_t s,
                              const CalibCtrl *skip);
 hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int nfind, double target, int64_t min_stat,

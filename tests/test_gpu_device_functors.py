@@ -8,6 +8,8 @@ mci_add_observable_device): the generic kernels compiled at run time with the fu
 - restatements of the catalogue's diagonal Gaussian and x_i^2 give the catalogue's chains bit for
   bit on many walkers, both random modes and both couplings;
 - a functor that does not compile fails integrate with the compiler's message."""
+import time
+
 import numpy as np
 import pytest
 
@@ -103,3 +105,22 @@ __device__ double always_updated_acceptance(int ndim, int nproto, MciVec xnew, M
         c.integrate(16 * 16, False, False)
         rates[veclen] = c.acceptance()[2]
     assert rates[1] == 1.0 and rates[0] < 0.9, rates
+
+
+@pytest.mark.parametrize("d", [26, 35, 60])
+def test_all_kernels_are_built_ahead(d):
+    """buildDeviceFunctors builds every kernel the integrates launch, whatever the width of the state (in LDS, in
+    LDS while calibrating, in HBM): an integrate of a few steps after it takes a small part of a build's time"""
+    name = f"ahead{time.time_ns()}"  # (the compiler keeps what it has built on disk)
+    c = Chain("mci", d, 70)
+    c.setSeed(3)
+    c.setCoupling(COUPLING_SHARED)
+    c.setNdecorrelationSteps(20)
+    c.addSamplingFunctionDevice(name, DF.DIAG.replace("diag_", name + "_"), d, np.full(d, 0.5))
+    c.addObservableDevice("xsq", DF.X2, d, (), 4, 1, True, ESTIM_MJ)
+    t = [time.perf_counter()]
+    for step in (lambda: c.call("build_device_functors"), lambda: c.integrate(4 * 32)):
+        step()
+        t.append(time.perf_counter())
+        print("built ahead", d, t[-1] - t[-2], flush=True)
+    assert t[2] - t[1] < 0.3 * (t[1] - t[0])

@@ -130,13 +130,20 @@ __device__ __forceinline__ MciVec rows_from(const MciVec &v, int i) { return Mci
 // --------------------------------------------------------------------------
 // random streams
 // --------------------------------------------------------------------------
-struct Lane
+// what draws take and leave of a walker's stream
+struct Draws
 {
     int64_t w;
     int32_t mtp;       // MT: next index
     uint64_t m0, m1, mm; // MT: elements mtp, mtp + 1, mtp + 156 (mod 312)
     uint64_t t;        // Philox: step counter
     uint32_t k, kx;    // Philox: word index within the step, extra-word index
+    double sv[2];      // saved normals of the move's distribution (nsv)
+    int sf;            // their availability bits (nsf)
+};
+
+struct Lane : Draws
+{
     uint32_t b0[4], bk[4];  // Philox: block 0 of step pair b0t, block bkn of step pair bkt
     uint64_t b0t, bkt;
     uint32_t bkn;
@@ -145,8 +152,6 @@ struct Lane
     bool accepted;
     int64_t acc, rej;
     double st0;        // the step size of type 0
-    double sv[2];      // saved normals of the move's distribution (nsv)
-    int sf;            // their availability bits (nsf)
 };
 
 // mt19937_64 with the twist done lazily, one element per output: element k of a round
@@ -172,7 +177,7 @@ __device__ __forceinline__ uint64_t mt_temper(uint64_t z)
 // the elements the next output is made from (Lane::m0, m1, mm), read an output ahead: their latency would
 // otherwise be part of every draw
 template <class C>
-__device__ __forceinline__ void mt_ahead(const C &c, Lane &L)
+__device__ __forceinline__ void mt_ahead(const C &c, Draws &L)
 {
     const int64_t W = c.W;
     const int k = L.mtp;
@@ -183,7 +188,7 @@ __device__ __forceinline__ void mt_ahead(const C &c, Lane &L)
 }
 
 template <class C>
-__device__ __forceinline__ uint64_t mt_next(const C &c, Lane &L)
+__device__ __forceinline__ uint64_t mt_next(const C &c, Draws &L)
 {
     const int64_t W = c.W;
     const int k = L.mtp;
@@ -221,7 +226,7 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 // rejections (block 0x20000000 + kx / 4, word kx mod 4) and the acceptance uniform's low word
 // (block 0x30000000, word 0).
 template <class C>
-__device__ __forceinline__ uint32_t ph_block_word(const C &c, const Lane &L, uint32_t blk, uint64_t ct, uint32_t word)
+__device__ __forceinline__ uint32_t ph_block_word(const C &c, const Draws &L, uint32_t blk, uint64_t ct, uint32_t word)
 {
     uint32_t o[4];
     philox4x32_10(blk, (uint32_t)L.w, (uint32_t)ct, (uint32_t)(ct >> 32), c.key0, c.key1, o);
@@ -255,6 +260,15 @@ __device__ __forceinline__ uint32_t ph_word(const C &c, Lane &L, uint32_t k)
     return (L.t & 1u) ? b : a;
 }
 
+// the same word, its block drawn for it alone (the draws of srrd_run_other: with rejections, lanes need other
+// blocks at other times, and a block kept for its second word saved less than the branch on it cost: a call with
+// 256 Student steps 28.2 ms instead of 24.7)
+template <class C>
+__device__ __forceinline__ uint32_t ph_word(const C &c, Draws &L, uint32_t k)
+{
+    return ph_block_word(c, L, k >> 1, L.t >> 1, 2u * (uint32_t)(L.t & 1u) + (k & 1u));
+}
+
 __device__ __forceinline__ void step_begin(Lane &L) { L.k = 1; L.kx = 0; }
 __device__ __forceinline__ void step_end(const Chain &c, Lane &L) { if (c.rng == MCI_RNG_PHILOX) { ++L.t; } }
 
@@ -267,8 +281,8 @@ __device__ __forceinline__ double canonical53(uint64_t w)
 }
 
 // symmetric uniform on (-1,1) (TrialMoveInterface.hpp:120-124): (u*(b-a)) + a
-template <class C>
-__device__ __forceinline__ double draw_sym(const C &c, Lane &L)
+template <class C, class S>
+__device__ __forceinline__ double draw_sym(const C &c, S &L)
 {
     if (c.rng == MCI_RNG_MT19937_64) {
         const double u = canonical53(mt_next(c, L));
@@ -279,8 +293,8 @@ __device__ __forceinline__ double draw_sym(const C &c, Lane &L)
 }
 
 // uniform on [0,1) (MCIntegrator.cpp:343 acceptance draw; :365 random moves)
-template <class C>
-__device__ __forceinline__ double draw_unit(const C &c, Lane &L)
+template <class C, class S>
+__device__ __forceinline__ double draw_unit(const C &c, S &L)
 {
     if (c.rng == MCI_RNG_MT19937_64) {
         const double u = canonical53(mt_next(c, L));
@@ -350,8 +364,8 @@ __device__ __forceinline__ int draw_index(const Chain &c, Lane &L, int n)
 // the value (SymmetrizedPRRD, TrialMoveInterface.hpp:80-98).  With the reference stream the
 // draws are the reference's up to the last place of the device's log, tan, pow and exp.
 // --------------------------------------------------------------------------
-template <class C>
-__device__ inline double nd_draw(const C &c, Lane &L, int s)
+template <class C, class S>
+__device__ inline double nd_draw(const C &c, S &L, int s)
 {
     double ret;
     if (L.sf & (1 << s)) {
@@ -373,8 +387,8 @@ __device__ inline double nd_draw(const C &c, Lane &L, int s)
     return ret * 1.0 + 0.0;
 }
 
-template <class C>
-__device__ inline double gamma_draw(const C &c, Lane &L, int s, double alpha, double beta)
+template <class C, class S>
+__device__ inline double gamma_draw(const C &c, S &L, int s, double alpha, double beta)
 {
     const double malpha = alpha < 1.0 ? alpha + 1.0 : alpha;
     const double a1 = malpha - 1.0 / 3.0;
@@ -402,9 +416,8 @@ struct Streams
     int64_t W;
 };
 
-// the distributions other than the uniform one, in a function of their own: inlined at every draw they
-// made the step kernels larger than the instruction cache
-__device__ __noinline__ double srrd_draw_other(const Streams c, Lane &L)
+// the distributions other than the uniform one
+__device__ __forceinline__ double srrd_draw_other(const Streams &c, Draws &L)
 {
     double val;
     switch (c.srrd) {
@@ -434,13 +447,26 @@ __device__ __noinline__ double srrd_draw_other(const Streams c, Lane &L)
     return ((draw_unit(c, L) - 0.0) < 0.5 * (1.0 - 0.0)) ? val : -val;
 }
 
-__device__ __forceinline__ double srrd_draw(const Chain &c, Lane &L)
+// x_i + st r_i for the n coordinates x, r of these distributions.  A function of its own, since inlined at
+// every move it made the step kernels larger than the instruction cache; one call for a run of coordinates,
+// since a call carries the walker's stream through memory and back (a call for every draw took more time
+// than the draws: Student moves in four dimensions, 512 steps of 16,384 walkers, 34.7 ms, 13.3 here).
+__device__ __noinline__ void srrd_run_other(const Streams c, Draws &L, const MciVec x, int n, double st)
 {
-    if (c.srrd == MCI_SRRD_UNIFORM) { return draw_sym(c, L); }
-    Lane other = L;  // a copy, so that L itself stays in registers
-    const double v = srrd_draw_other(Streams{c.rng, c.srrd, c.key0, c.key1, c.mt, c.W}, other);
-    L = other;
-    return v;
+    Draws l = L;  // in registers while it draws
+    for (int i = 0; i < n; ++i) { x[i] = x[i] + st * srrd_draw_other(c, l); }
+    L = l;
+}
+
+__device__ __forceinline__ void srrd_run(const Chain &c, Lane &L, const MciVec &x, int n, double st)
+{
+    if (c.srrd == MCI_SRRD_UNIFORM) {
+        for (int i = 0; i < n; ++i) { x[i] = x[i] + st * draw_sym(c, L); }
+        return;
+    }
+    Draws other = L;  // a copy, so that L itself stays in registers
+    srrd_run_other(Streams{c.rng, c.srrd, c.key0, c.key1, c.mt, c.W}, other, x, n, st);
+    static_cast<Draws &>(L) = other;
 }
 
 // --------------------------------------------------------------------------
@@ -636,11 +662,8 @@ __device__ __forceinline__ double srrd_move(const Chain &c, Lane &L, const MciVe
         int xidx = 0;
         for (int t = 0; t < c.ntypes; ++t) {
             const double st = t == 0 ? L.st0 : c.steps[(int64_t)t * W + w];
-            while (xidx < c.typeEnds[t]) {
-                double &v = xn[xidx];
-                v = v + st * srrd_draw(c, L);
-                ++xidx;
-            }
+            srrd_run(c, L, rows_from(xn, xidx), c.typeEnds[t] - xidx, st);
+            xidx = c.typeEnds[t];
         }
         L.nchanged = c.ndim;
         L.cfirst = 0;
@@ -657,10 +680,7 @@ __device__ __forceinline__ double srrd_move(const Chain &c, Lane &L, const MciVe
     }
     double st = L.st0;
     if (t > 0) { st = c.steps[(int64_t)t * W + w]; }
-    for (int i = 0; i < c.veclen; ++i) {
-        double &v = xn[xidx + i];
-        v = v + st * srrd_draw(c, L);
-    }
+    srrd_run(c, L, rows_from(xn, xidx), c.veclen, st);
     L.nchanged = c.veclen;
     L.cfirst = xidx;
     return 1.;

@@ -12,7 +12,7 @@ import pytest
 
 import golden_io as G
 from mcitest import (COUPLING_INDEPENDENT, COUPLING_SHARED, ESTIM_CORR, ESTIM_FC, ESTIM_MJ, ESTIM_NOOP, ESTIM_UNCORR, KERNELS_AUTO, KERNELS_GENERIC,
-                     OBS_EXP_X2, OBS_X, OBS_X2, OBS_X2_SUM, PDF_GAUSS_DIAG, PREC_FP32, RNG_MT, RNG_PHILOX, Chain,
+                     OBS_EXP_X2, OBS_X, OBS_X2, OBS_X2_SUM, PDF_EXP_DIAG, PDF_GAUSS_DIAG, PREC_FP32, RNG_MT, RNG_PHILOX, Chain,
                      chain_setup, estimate)
 
 pytestmark = pytest.mark.gpu
@@ -768,3 +768,24 @@ def test_specialised_moves_after_generator_positions_diverge(veclen, d):
     f, g = out["fast"], out["generic"]
     for k in range(len(f)):
         assert np.array_equal(f[k], g[k]), k
+
+
+def test_moves_of_other_distributions_cost_their_draws():
+    """The draws of Student moves (a normal and a gamma with rejections each) run in registers: a call takes at
+    most fifteen times what it takes with uniform moves (nine are measured; twenty-three with the walker's stream
+    carried through memory for every draw)."""
+    import time
+    d, took = 4, []
+    for srrd in (0, 2):
+        c = chain_setup("mci", dict(ndim=d, seed=3, ndecorr=200, move=(srrd, 0, 1, None), pdfs=[(PDF_EXP_DIAG, np.full(d, 1.0))],
+                                    obs=[(OBS_X2, [], 16, 1, 0, ESTIM_MJ)]), nwalkers=16384)
+        c.setRng(RNG_PHILOX)
+        c.setCoupling(1)
+        t = []
+        for _ in range(4):
+            print("moves of distribution", srrd, flush=True)
+            t0 = time.perf_counter()
+            c.integrate(512)
+            t.append(time.perf_counter() - t0)
+        took.append(min(t[1:]))
+    assert took[1] < 15 * took[0], took

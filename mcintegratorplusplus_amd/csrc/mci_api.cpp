@@ -339,11 +339,12 @@ int rtc_kinds(const mci_ctx *c)
     Chain ch;
     std::memset(&ch, 0, sizeof ch);
     ch.ndim = c->ndim;
+    ch.W = c->W;
     ch.nproto = nproto_total(c);
-    int kinds = 1 << state_lds_of(ch, false).in_lds;
+    int kinds = 1 << state_lds_of(ch, false).kind;
     ch.nobs = (int)c->obs.size();
     for (int i = 0; i < ch.nobs; ++i) { ch.obs[i].nobs = c->obs[(size_t)i].nobs; }
-    kinds |= 1 << state_lds_of(ch, true).in_lds;
+    kinds |= 1 << state_lds_of(ch, true).kind;
     return kinds;
 }
 

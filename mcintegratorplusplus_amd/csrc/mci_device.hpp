@@ -748,6 +748,28 @@ __device__ inline double lm_move(const Chain &c, Lane &L, const Views &V)
     return exp(lm_logq(c, V.xo) - lm_logq(c, V.xn));
 }
 
+// elements [first, first + n) after a step: the new ones to the old where it was accepted, else the old ones
+// back.  LDSV: both are read and both written, without a branch or a choice of addresses; in HBM the traffic
+// counts and only one is (39 dimensions, 262,144 walkers on the reference streams, 128 steps of exp(-|x|): 90.6
+// ms with both written, 81.1 so).
+template <bool LDSV>
+__device__ __forceinline__ void commit(const MciVec &o, const MciVec &n, int first, int count, bool acc)
+{
+    if constexpr (LDSV) {
+#pragma unroll 4
+        for (int j = first; j < first + count; ++j) {
+            const double vo = o[j], vn = n[j];
+            const double v = acc ? vn : vo;
+            o[j] = v;
+            n[j] = v;
+        }
+    }
+    else {
+        const MciVec from{acc ? n.p : o.p, o.s}, to{acc ? o.p : n.p, o.s};
+        for (int j = first; j < first + count; ++j) { to[j] = from[j]; }
+    }
+}
+
 // MultiStepMove::trialMove (MultiStepMove.cpp:6-47): ms_nsteps Metropolis steps of the contained
 // move under the move's own sampling functions (none: every step accepted), from xold; xnew ends at
 // the last position, xold is restored, every coordinate counts as changed, and the factor
@@ -783,16 +805,8 @@ __device__ __forceinline__ double trial_move(const Chain &c, Lane &L, const View
         double pdfAcc = 1.;
         for (int p = 0; p < c.ms_npdf; ++p) { pdfAcc *= pdf_compute_acceptance(c, c.ms_pdf[p], L, V.xo, V.xn, mo, mn); }
         const bool acc = (draw_unit(c, L) <= pdfAcc * moveAcc);
-        for (int i = 0; i < c.ms_nproto; ++i) {
-            const double v = acc ? mn[i] : mo[i];
-            mo[i] = v;
-            mn[i] = v;
-        }
-        for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
-            const double v = acc ? V.xn[j] : V.xo[j];
-            V.xo[j] = v;
-            V.xn[j] = v;
-        }
+        commit<false>(mo, mn, 0, c.ms_nproto, acc);
+        commit<false>(V.xo, V.xn, L.cfirst, L.nchanged, acc);
     }
     double newPDF = 1.;
     for (int p = 0; p < c.ms_npdf; ++p) { newPDF *= pdf_value(c.ms_pdf[p], mo); }
@@ -826,6 +840,7 @@ __device__ __forceinline__ void init_sampling(const Chain &c, Lane &L, const Vie
 }
 
 // MCI::doStepMRT2 (MCIntegrator.cpp:326-360)
+template <bool LDSV>
 __device__ __forceinline__ void step_mrt2(const Chain &c, Lane &L, const Views &V)
 {
     step_begin(L);
@@ -840,21 +855,8 @@ __device__ __forceinline__ void step_mrt2(const Chain &c, Lane &L, const Views &
     cb_record(c, L, V);
     step_end(c, L);
     // commit or roll back the coordinates and proto values that can differ
-    const bool acc = L.accepted;
-#pragma unroll 4
-    for (int j = L.cfirst; j < L.cfirst + L.nchanged; ++j) {
-        const double o = V.xo[j], n = V.xn[j];
-        const double v = acc ? n : o;
-        V.xo[j] = v;
-        V.xn[j] = v;
-    }
-#pragma unroll 4
-    for (int i = 0; i < c.nproto; ++i) {
-        const double o = V.po[i], n = V.pn[i];
-        const double v = acc ? n : o;
-        V.po[i] = v;
-        V.pn[i] = v;
-    }
+    commit<LDSV>(V.xo, V.xn, L.cfirst, L.nchanged, L.accepted);
+    commit<LDSV>(V.po, V.pn, 0, c.nproto, L.accepted);
 #ifdef MCI_RTC_USER
     if (c.movetype == MCI_MOVE_DEVICE) { // the trial move's newToOld / oldToNew
         const int64_t W = c.W, w = L.w;

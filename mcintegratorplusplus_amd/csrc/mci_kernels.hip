@@ -1183,8 +1183,11 @@ hipError_t launch_sample(const Chain &c, int64_t nsteps, int acc, const uint8_t 
 {
     const StateLds st = state_lds_of(c, acc != 0);
     const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
-    if (st.in_lds) { hipLaunchKernelGGL(k_sample<true>, g, b, st.bytes, s, c, nsteps, acc, active, skip); }
-    else { hipLaunchKernelGGL(k_sample<false>, g, b, 0, s, c, nsteps, acc, active, skip); }
+    switch (st.kind) {
+    case STATE_LDS: hipLaunchKernelGGL(k_sample<STATE_LDS>, g, b, st.bytes, s, c, nsteps, acc, active, skip); break;
+    case STATE_HBM_TWO: hipLaunchKernelGGL(k_sample<STATE_HBM_TWO>, g, b, 0, s, c, nsteps, acc, active, skip); break;
+    default: hipLaunchKernelGGL(k_sample<STATE_HBM>, g, b, 0, s, c, nsteps, acc, active, skip);
+    }
     return hipGetLastError();
 }
 
@@ -1192,15 +1195,19 @@ hipError_t launch_calibrate_indep(const Chain &c, int nfind, double target, int6
 {
     const StateLds st = state_lds_of(c, false);
     const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
-    if (st.in_lds) { hipLaunchKernelGGL(k_calibrate_indep<true>, g, b, st.bytes, s, c, nfind, target, min_stat, dimSizes); }
-    else { hipLaunchKernelGGL(k_calibrate_indep<false>, g, b, 0, s, c, nfind, target, min_stat, dimSizes); }
+    switch (st.kind) {
+    case STATE_LDS: hipLaunchKernelGGL(k_calibrate_indep<STATE_LDS>, g, b, st.bytes, s, c, nfind, target, min_stat, dimSizes); break;
+    case STATE_HBM_TWO: hipLaunchKernelGGL(k_calibrate_indep<STATE_HBM_TWO>, g, b, 0, s, c, nfind, target, min_stat, dimSizes); break;
+    default: hipLaunchKernelGGL(k_calibrate_indep<STATE_HBM>, g, b, 0, s, c, nfind, target, min_stat, dimSizes);
+    }
     return hipGetLastError();
 }
 
 StateLds state_lds_of(const Chain &c, bool observables)
 {
     const size_t n = state_lds(c, observables ? chain_nobsdim(c) : 0);
-    return n <= STATE_LDS_MAX ? StateLds{n, 1} : StateLds{0, 0};
+    if (n <= STATE_LDS_MAX) { return StateLds{n, STATE_LDS}; }
+    return StateLds{0, c.W > STATE_TWO ? STATE_HBM_TWO : STATE_HBM};
 }
 
 hipError_t launch_scale_steps(const Chain &c, const CalibCtrl *ctrl, const double *dimSizes, hipStream_t s)

@@ -45,6 +45,10 @@ struct EstimJob
     const double *sum = nullptr;
 };
 
+// where a generic step kernel keeps the walkers' state: HBM, the wave's LDS, or HBM with the registers for
+// two waves a SIMD
+enum StateKind { STATE_HBM, STATE_LDS, STATE_HBM_TWO, STATE_KINDS };
+
 #ifndef MCI_RTC_USER // the host's launch interface (not part of the run-time build of the step kernels)
 hipError_t launch_seed_mt(uint64_t *mt, int32_t *mtp, const uint64_t *seeds, int64_t W, hipStream_t s);
 // the walkers with a set flag listed (count starts at 0); their sampling columns moved to / from
@@ -54,11 +58,11 @@ hipError_t launch_walker_columns(const Chain &c, const Chain &dense, const int32
                                  hipStream_t s);
 // every walker's mt19937_64 state rotated to next index 0 (the same generator)
 hipError_t launch_mt_align(uint64_t *mt, int32_t *mtp, int64_t W, hipStream_t s);
-// dynamic LDS of a generic step kernel's launch and whether the walkers' state goes there
+// dynamic LDS of a generic step kernel's launch and which form of the kernel it takes
 struct StateLds
 {
     size_t bytes;
-    int in_lds;
+    int kind;
 };
 StateLds state_lds_of(const Chain &c, bool observables);
 hipError_t launch_sample(const Chain &c, int64_t nsteps, int acc, const uint8_t *active, hipStream_t s,

@@ -27,17 +27,18 @@ namespace
 std::mutex g_mu;
 struct Loaded
 {
-    hipModule_t mod[2] = {nullptr, nullptr};
+    hipModule_t mod[STATE_KINDS] = {};
     RtcKernels k;
 };
 std::map<std::pair<std::string, int>, Loaded> g_cache;
 
-// the walkers' state in HBM, in LDS
-const char *const kNames[2][2] = {{"mcid::k_sample<false>", "mcid::k_calibrate_indep<false>"},
-                                  {"mcid::k_sample<true>", "mcid::k_calibrate_indep<true>"}};
+// by StateKind
+const char *const kNames[STATE_KINDS][2] = {{"mcid::k_sample<0>", "mcid::k_calibrate_indep<0>"},
+                                            {"mcid::k_sample<1>", "mcid::k_calibrate_indep<1>"},
+                                            {"mcid::k_sample<2>", "mcid::k_calibrate_indep<2>"}};
 
 // compiles text's kernels of one kind; on success code holds the code object and names their lowered names
-int compile(const std::string &text, const std::string &arch, int lds, std::vector<char> &code, std::string (&names)[2], std::string &log)
+int compile(const std::string &text, const std::string &arch, int kind, std::vector<char> &code, std::string (&names)[2], std::string &log)
 {
     hiprtcProgram p;
     if (hiprtcCreateProgram(&p, text.c_str(), "mci_device_functors.hip", rtc_nheaders, rtc_header_texts, rtc_header_names) !=
@@ -45,7 +46,7 @@ int compile(const std::string &text, const std::string &arch, int lds, std::vect
         log = "hiprtcCreateProgram failed";
         return MCI_E_DEVICE;
     }
-    for (const char *n : kNames[lds]) { hiprtcAddNameExpression(p, n); }
+    for (const char *n : kNames[kind]) { hiprtcAddNameExpression(p, n); }
     // the library's own flags: no contraction (bit-exact FP64 chains), correctly rounded FP32
     // divide and sqrt, no packed FP32 instructions
     const std::string off = "--offload-arch=" + arch;
@@ -70,7 +71,7 @@ int compile(const std::string &text, const std::string &arch, int lds, std::vect
     bool all = cs > 0;
     for (int i = 0; i < 2; ++i) {
         const char *l = nullptr;
-        hiprtcGetLoweredName(p, kNames[lds][i], &l);
+        hiprtcGetLoweredName(p, kNames[kind][i], &l);
         names[i] = l ? l : "";
         all = all && !names[i].empty();
     }
@@ -165,13 +166,13 @@ int rtc_check(const std::string &text, const char *arch, std::string &log)
 {
     std::vector<char> code;
     std::string names[2];
-    return compile(text, arch ? arch : "gfx950", 1, code, names, log);
+    return compile(text, arch ? arch : "gfx950", STATE_LDS, code, names, log);
 }
 
 namespace
 {
 // the kernels of one kind of L's program, compiled and loaded on the current device (g_mu held)
-int load(const std::string &text, int lds, Loaded &L, std::string &log)
+int load(const std::string &text, int kind, Loaded &L, std::string &log)
 {
     int dev = 0;
     hipDeviceProp_t prop;
@@ -181,20 +182,20 @@ int load(const std::string &text, int lds, Loaded &L, std::string &log)
     if (colon != std::string::npos) { arch.resize(colon); }
     std::vector<char> code;
     std::string names[2];
-    const int st = compile(text, arch, lds, code, names, log);
+    const int st = compile(text, arch, kind, code, names, log);
     if (st != MCI_OK) { return st; }
-    if (hipModuleLoadData(&L.mod[lds], code.data()) != hipSuccess) {
+    if (hipModuleLoadData(&L.mod[kind], code.data()) != hipSuccess) {
         log = "hipModuleLoadData failed";
         return MCI_E_DEVICE;
     }
     hipFunction_t fs = nullptr, fc = nullptr;
-    if (hipModuleGetFunction(&fs, L.mod[lds], names[0].c_str()) != hipSuccess ||
-        hipModuleGetFunction(&fc, L.mod[lds], names[1].c_str()) != hipSuccess) {
+    if (hipModuleGetFunction(&fs, L.mod[kind], names[0].c_str()) != hipSuccess ||
+        hipModuleGetFunction(&fc, L.mod[kind], names[1].c_str()) != hipSuccess) {
         log = "hipModuleGetFunction failed";
         return MCI_E_DEVICE;
     }
-    L.k.sample[lds] = fs;
-    L.k.calibrate[lds] = fc;
+    L.k.sample[kind] = fs;
+    L.k.calibrate[kind] = fc;
     return MCI_OK;
 }
 } // namespace
@@ -205,9 +206,9 @@ int rtc_get(const std::string &text, int kinds, RtcKernels &out, std::string &lo
     if (hipGetDevice(&dev) != hipSuccess) { return MCI_E_DEVICE; }
     std::lock_guard<std::mutex> lk(g_mu);
     Loaded &L = g_cache[std::make_pair(text, dev)];
-    for (int lds = 0; lds < 2; ++lds) {
-        if (!(kinds & (1 << lds)) || L.k.sample[lds]) { continue; }
-        const int st = load(text, lds, L, log);
+    for (int kind = 0; kind < STATE_KINDS; ++kind) {
+        if (!(kinds & (1 << kind)) || L.k.sample[kind]) { continue; }
+        const int st = load(text, kind, L, log);
         if (st != MCI_OK) { return st; }
     }
     out = L.k;
@@ -219,10 +220,10 @@ hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, acc != 0);
-    if (!k.sample[st.in_lds]) { return hipErrorInvalidDeviceFunction; }
+    if (!k.sample[st.kind]) { return hipErrorInvalidDeviceFunction; }
     void *args[] = {&cc, &nsteps, &acc, &active, &skip};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
-    return hipModuleLaunchKernel(k.sample[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
+    return hipModuleLaunchKernel(k.sample[st.kind], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
 }
 
 hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int nfind, double target, int64_t min_stat,
@@ -230,9 +231,9 @@ hipError_t rtc_launch_calibrate_indep(const RtcKernels &k, const Chain &c, int n
 {
     Chain cc = c;
     const StateLds st = state_lds_of(c, false);
-    if (!k.calibrate[st.in_lds]) { return hipErrorInvalidDeviceFunction; }
+    if (!k.calibrate[st.kind]) { return hipErrorInvalidDeviceFunction; }
     void *args[] = {&cc, &nfind, &target, &min_stat, &dimSizes};
     const unsigned grid = (unsigned)((c.W + 63) / 64);
-    return hipModuleLaunchKernel(k.calibrate[st.in_lds], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
+    return hipModuleLaunchKernel(k.calibrate[st.kind], grid, 1, 1, 64, 1, 1, (unsigned)st.bytes, s, args, nullptr);
 }
 } // namespace mcid

@@ -15,13 +15,19 @@ struct RtcFunctor
     std::string name, source;
 };
 
-// the generic step kernels of one program (loaded on one device): the walkers' state in HBM [0], in LDS
-// [1] (state_lds_of).  Each kind is a build of its own: a program is built in the kinds its chain takes.
+// the generic step kernels of one program (loaded on one device), by StateKind.  Each kind is a build of its
+// own: a program is built in the kinds its chain takes.
 struct RtcKernels
 {
-    hipFunction_t sample[2] = {nullptr, nullptr}, calibrate[2] = {nullptr, nullptr};
-    bool any() const { return sample[0] || sample[1]; }
-    bool has(int kinds) const { return (!(kinds & 1) || sample[0]) && (!(kinds & 2) || sample[1]); }
+    hipFunction_t sample[STATE_KINDS] = {}, calibrate[STATE_KINDS] = {};
+    bool any() const { return kinds() != 0; }
+    bool has(int k) const { return (kinds() & k) == k; }
+    int kinds() const
+    {
+        int k = 0;
+        for (int i = 0; i < STATE_KINDS; ++i) { k |= sample[i] ? 1 << i : 0; }
+        return k;
+    }
 };
 
 // true when name is a C identifier
@@ -35,7 +41,7 @@ bool rtc_program(const std::vector<RtcFunctor> &pdfs, const std::vector<RtcFunct
 // compiles text for arch (e.g. "gfx950") without loading it; log: the compiler's messages.  One kind: the
 // functors are the same text in both.
 int rtc_check(const std::string &text, const char *arch, std::string &log);
-// the kernels of text on the current device, those of the given kinds (bit 0: HBM, bit 1: LDS) among
+// the kernels of text on the current device, those of the given kinds (bits 1 << StateKind) among
 // them: compiled and loaded once per text, device and kind
 int rtc_get(const std::string &text, int kinds, RtcKernels &out, std::string &log);
 hipError_t rtc_launch_sample(const RtcKernels &k, const Chain &c, int64_t nsteps, int acc, const uint8_t *active, hipStream_t s,

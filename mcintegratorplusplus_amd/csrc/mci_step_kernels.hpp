@@ -21,6 +21,12 @@ namespace mcid
 // latency is not hidden).
 constexpr int STATE_WAVE = 64;
 constexpr size_t STATE_LDS_MAX = 80 * 1024;  // two waves a CU: beyond that the columns stay in HBM
+// Waves a SIMD that a kind's registers leave room for.  In HBM a step waits for its accesses, so waves in
+// flight count where there are more than one a SIMD (STATE_TWO walkers); the registers that the second one
+// needs spill, which costs up to an eighth with fewer.  A call with 128 steps in 39 / 60 dimensions, one wave /
+// two, ms: exp(-|x|), single-coordinate moves, 262,144 walkers 66.0 / 54.6, 65,536 29.2 / 32.8 (d 60).
+constexpr int64_t STATE_TWO = 65536;
+inline __host__ __device__ constexpr int state_waves(int kind) { return kind == STATE_HBM_TWO ? 2 : 1; }
 inline __host__ __device__ int state_rows(const Chain &c, int nobsdim) { return 2 * c.ndim + 2 * c.nproto + 2 * nobsdim; }
 inline __host__ __device__ size_t state_lds(const Chain &c, int nobsdim)
 {
@@ -92,7 +98,7 @@ __device__ __forceinline__ void sample_walker(const Chain &c, int64_t nsteps, in
         else { zero_accu(c, w); }
     }
     for (int64_t s = 0; s < nsteps; ++s) {
-        if (c.npdf > 0) { step_mrt2(c, L, V); }
+        if (c.npdf > 0) { step_mrt2<LDSV>(c, L, V); }
         else { step_random(c, L, V); }
         if (accumulate_obs) {
             accumulate<LDSV>(c, L, V, s, dirty);
@@ -124,16 +130,16 @@ __device__ __forceinline__ void sample_walker(const Chain &c, int64_t nsteps, in
     store_lane(c, L);
 }
 
-template <bool LDSV>
-__global__ __launch_bounds__(STATE_WAVE) void k_sample(Chain c, int64_t nsteps, int accumulate_obs, const uint8_t *active,
-                                                       const CalibCtrl *skip)
+template <int KIND>
+__global__ __launch_bounds__(STATE_WAVE, state_waves(KIND)) void k_sample(Chain c, int64_t nsteps, int accumulate_obs,
+                                                                          const uint8_t *active, const CalibCtrl *skip)
 {
     extern __shared__ double state_sh[];
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= c.W) { return; }
     if (skip && skip->done) { return; }
     if (active && !active[w]) { return; }
-    sample_walker<LDSV>(c, nsteps, accumulate_obs, w, state_sh);
+    sample_walker<KIND == STATE_LDS>(c, nsteps, accumulate_obs, w, state_sh);
 }
 
 // step clamps of findMRT2Step (MCIntegrator.cpp:147-161)
@@ -163,7 +169,7 @@ __device__ __forceinline__ void calibrate_walker(const Chain &c, int nfind, doub
     int cons = 0, counter = 0;
     while ((nfind < 0 && cons < 5) || counter < nfind) {
         init_sampling(c, L, V);
-        for (int64_t s = 0; s < min_stat; ++s) { step_mrt2(c, L, V); }
+        for (int64_t s = 0; s < min_stat; ++s) { step_mrt2<LDSV>(c, L, V); }
         const double rate = (L.acc > 0) ? (double)L.acc / ((double)L.acc + (double)L.rej) : 0.;
         if (fabs(rate - target) < 0.05) { ++cons; }
         else { cons = 0; }
@@ -177,12 +183,13 @@ __device__ __forceinline__ void calibrate_walker(const Chain &c, int nfind, doub
     store_lane(c, L);
 }
 
-template <bool LDSV>
-__global__ __launch_bounds__(STATE_WAVE) void k_calibrate_indep(Chain c, int nfind, double target, int64_t min_stat, const double *dimSizes)
+template <int KIND>
+__global__ __launch_bounds__(STATE_WAVE, state_waves(KIND)) void k_calibrate_indep(Chain c, int nfind, double target, int64_t min_stat,
+                                                                                   const double *dimSizes)
 {
     extern __shared__ double state_sh[];
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= c.W) { return; }
-    calibrate_walker<LDSV>(c, nfind, target, min_stat, dimSizes, w, state_sh);
+    calibrate_walker<KIND == STATE_LDS>(c, nfind, target, min_stat, dimSizes, w, state_sh);
 }
 } // namespace mcid

@@ -52,3 +52,24 @@ def test_a_run_too_large_for_the_card_is_an_error_once():
     print("and of a few steps", flush=True)
     avg, _ = c.integrate(8, False, False)
     assert np.all(np.isfinite(avg))
+
+
+@pytest.mark.parametrize("d,W", [(28, 65536), (28, 65537)])
+def test_many_walkers_in_hbm(d, W):
+    """a state in HBM with up to one wave a SIMD and with more, against the specialised kernel: bit for bit"""
+    print("state in HBM", d, W, flush=True)
+    out = []
+    for generic in (False, True):
+        c = Chain("mci", d, W)
+        c.setSeed(98)
+        c.setRng(RNG_MT)
+        c.setCoupling(COUPLING_INDEPENDENT)
+        c.setNfindMRT2Iterations(1)
+        c.setNdecorrelationSteps(5)
+        if generic:
+            c.setKernelPath(KERNELS_GENERIC)
+        c.addSamplingFunction(PDF_GAUSS_DIAG, np.full(d, 0.5))
+        c.addObservable(OBS_X2, (), 4, 1, True, ESTIM_MJ)
+        out.append((*c.integrate(4 * 4), c.getX(), *c.walkerAcceptance()))
+    for k, (f, g) in enumerate(zip(*out)):
+        assert np.array_equal(f, g), k

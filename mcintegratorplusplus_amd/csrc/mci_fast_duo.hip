@@ -201,6 +201,7 @@ __global__ __launch_bounds__(2 * WAVE) void k_fast64_duo(FastArgs A)
         if (!live) { return; }
         const double norm = 1. / (double)B;
         double rx = 0.0, sS = 0.0;
+#pragma unroll 8
         for (int i = 0; i < d; ++i) {
             double v2;
             if (REC) {

@@ -1493,7 +1493,7 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         if (prec != MCI_PREC_FP64 || (c.nvecs & (c.nvecs - 1)) != 0 || !c.mt || !c.mtp) { return MCI_E_INVALID_ARGUMENT; }
         fl |= F_MT;
         int S = 0;
-        if (group_slots_vec(c.ndim, c.W, S)) {
+        if (group_slots_vec(c.ndim, c.W, S) && ((fl & 7) != 0 || group_vec_plain(c.ndim, c.W, nsteps))) {
             if (!launch_group(fl, true, 4, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
             return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
         }
@@ -1568,10 +1568,11 @@ bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
     return mt && group_slots_vec(ndim, W, S);
 }
 
-bool fast_rotates_mt(int movetype, int ndim, int64_t W)
+bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, bool sums)
 {
     int L, S;
-    return movetype == MCI_MOVE_ALL ? group_shape(true, ndim, W, L, S) : group_slots_vec(ndim, W, S);
+    if (movetype == MCI_MOVE_ALL) { return group_shape(true, ndim, W, L, S); }
+    return group_slots_vec(ndim, W, S) && (sums || group_vec_plain(ndim, W, nsteps));
 }
 
 void fast_release(FastState &fs) { (void)fs; }

@@ -30,8 +30,8 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
                 const int32_t *wmap = nullptr, const int32_t *wcount = nullptr);
 // the launches of these moves also write the sums of Full traces (ObsDev::sum)
 bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W);
-// the launches of these moves start from whatever next indices the walkers' mt19937_64 states stand at (and
-// leave them all at one), so the states need no realignment before them
-bool fast_rotates_mt(int movetype, int ndim, int64_t W);
+// a launch of nsteps steps of these moves (sums: with observables) starts from whatever next indices the
+// walkers' mt19937_64 states stand at (and leaves them all at one), so the states need no realignment before it
+bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, bool sums);
 void fast_release(FastState &fs);
 } // namespace mcid

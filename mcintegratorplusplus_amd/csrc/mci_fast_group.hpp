@@ -72,6 +72,20 @@ inline bool group_slots_vec(int d, int64_t W, int &S)
     return d <= 64 && (d & (d - 1)) == 0 && W * (int64_t)d < (int64_t)1 << 29;
 }
 
+// Whether such a launch of nsteps steps that sums nothing (calibration, decorrelation) runs on groups of
+// lanes.  One lane a walker then has little to do in LDS, and moves 72 bytes of generator state a step at up to
+// 5.4 TB/s; a group reads and writes the whole state once and issues its selects over S slots on four times as
+// many waves.  ms of one launch, one lane / group, 100, 1,000 steps:
+//   16,384 walkers d 16 0.062 / 0.051, 0.54 / 0.26; d 64 0.066 / 0.073, 0.54 / 0.44
+//   32,768 walkers d 16 0.065 / 0.064, 0.57 / 0.35; d 32 0.067 / 0.074, 0.57 / 0.45; d 64 0.071 / 0.132, 0.58 / 0.85
+//   65,536 walkers d 16 0.081 / 0.120, 0.70 / 0.68; d 32 0.083 / 0.137, 0.70 / 0.85; d 64 0.088 / 0.250, 0.70 / 1.65
+inline bool group_vec_plain(int d, int64_t W, int64_t nsteps)
+{
+    if (W <= 16384) { return true; }
+    if (W <= 32768) { return d <= 32; }
+    return d <= 16 && nsteps >= 512;
+}
+
 // one launch of kernel form fl (the F_* flags of mci_fast_dev.hpp, without F_P2; vec: single-coordinate
 // moves); false: there is no such form
 bool launch_group_0(int fl, bool vec, int L, int S, const FastArgs &A, hipStream_t s);

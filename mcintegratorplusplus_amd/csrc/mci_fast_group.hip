@@ -275,7 +275,7 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
     const uint32_t keep = apart(g == 0 ? 0u : 0xFFFFFFFFu);
     // v_0 + v_1 + ... over the walker's coordinates in order, from 0.0 (empty slots hold 0.0): each
     // lane continues from the lane before, L times over, so that the last lane ends with the whole sum
-    auto ordered = [&](const double (&v)[S]) -> double {
+    auto ordered = [&](const double (&v)[S]) __attribute__((always_inline)) -> double {
         double c = 0.0;
 #pragma unroll
         for (int ph = 0; ph < L; ++ph) {
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
 
     // the step's proposal from the slots' random values r
     double p[S], p2[S];
-    auto propose = [&](int s, double r) {
+    auto propose = [&](int s, double r) __attribute__((always_inline)) {
         double v = x[s] + step * r;
         if (!EX) { v = ok[s] ? v : 0.0; }
         xn[s] = v;
@@ -321,7 +321,9 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
     };
     // the decision from the acceptance word uw (native: the shared word; reference streams: the
     // acceptance output) and the observables after the step, as k_fast64_allr takes them
-    auto finish = [&](U64 uw) {
+    // (inlined at each of its calls, whatever its size: a call of its own takes the walker's arrays by address,
+    // and they then live in scratch memory)
+    auto finish = [&](U64 uw) __attribute__((always_inline)) {
         const double Snew = ordered(p);
         double qn = 0.0;
         if (QN) { qn = ordered(p2); }
@@ -421,7 +423,7 @@ __global__ __launch_bounds__(WAVE, (FL & F_MT) && S <= 4 ? 2 : 1) void k_fast64_
         constexpr int NB = S / 2;  // the lane's Philox blocks of a step pair
         auto rnd = [](uint32_t v) { return fma((double)v, 0x1p-31, -(1.0 - 0x1p-32)); };
         uint32_t sw[S];  // the second step's words of a pair
-        auto single = [&]() {
+        auto single = [&]() __attribute__((always_inline)) {
             const uint32_t par = (uint32_t)(t & 1u);
             const uint64_t tp = t >> 1;
             uint32_t uw = 0;
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(WAVE, S <= 4 ? 2 : 1) void k_fast64_vec4(FastArgs A
         offx[s] = (uint32_t)((mine ? c0 + s : 0) * W * 8) + (uint32_t)w * 8u;
     }
     const uint32_t keep = apart(g == 0 ? 0u : 0xFFFFFFFFu);
-    auto ordered = [&](const double (&v)[S]) -> double {  // as in k_fast64_grp
+    auto ordered = [&](const double (&v)[S]) __attribute__((always_inline)) -> double {  // as in k_fast64_grp
         double c = 0.0;
 #pragma unroll
         for (int ph = 0; ph < L; ++ph) {

@@ -124,3 +124,29 @@ def test_launches_without_sums_do_not_pay_for_the_dimensions():
             best = min(best, t[1])
         took.append(best)
     assert took[1] < 1.7 * took[0], took
+
+
+def phase(c, i, calls):
+    """the shortest of some calls' phases (milliseconds)"""
+    best = np.inf
+    for _ in range(calls):
+        c.integrate(256)
+        t = np.zeros(5)
+        c.call("get_timings", dptr(t), 5)
+        best = min(best, t[i])
+    return best
+
+
+def test_a_lane_of_eighteen_slots_keeps_them_in_registers():
+    """three observables of a walker in sixty dimensions cost their sums, at most twice one observable's launch (1.1
+    times is measured; eleven times with the walker's arrays in scratch memory)"""
+    took = []
+    for obs in ([OBS_X2], ALL_OBS):
+        print("slots", obs, flush=True)
+        c = chain_setup("mci", dict(ndim=60, seed=4, ndecorr=20, move=(0, 0, 1, None), pdfs=[(PDF_GAUSS_DIAG, np.full(60, 0.5))],
+                                    obs=[(k, [], 1, 1, 0, ESTIM_MJ) for k in obs]), nwalkers=16384)
+        c.setRng(RNG_PHILOX)
+        c.setCoupling(1)
+        took.append(phase(c, 2, 4))
+    print("took", took, flush=True)
+    assert took[1] < 2 * took[0], took

@@ -770,7 +770,8 @@ __global__ __launch_bounds__(WAVE) void k_fast64_all(FastArgs A)
 // pairs, one Philox block per two words of each of the two steps (the first step keeps words 2 and
 // 3 of every block for the second), so a pair computes ceil((d + 1) / 2) blocks.
 // EX: d == DM exactly (every coordinate guard folds away, the step is straight-line code).
-template <int FL, int DM, bool EX>
+// TS: the traces' sums are kept too (their registers leave one wave a SIMD: fast_sums_traces).
+template <int FL, int DM, bool EX, bool TS>
 __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
 {
     constexpr bool FULL = (FL & F_FULL) != 0;
@@ -847,18 +848,18 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
                 for (int i = 0; i < DM; ++i) {
                     if (i < d) {
                         const double v = x[i] * x[i];
-                        sm[i] = sm[i] + v;
+                        if (TS) { sm[i] = sm[i] + v; }
                         A.d_x2[(s * d + i) * W + w] = v;
                     }
                 }
             }
             if (HSUM) {
                 const double v = q / A.x2sum_div;
-                Sr = Sr + v;
+                if (TS) { Sr = Sr + v; }
                 A.d_x2sum[s * W + w] = v;
             }
             if (HEXP) {
-                Se = Se + e;
+                if (TS) { Se = Se + e; }
                 A.d_exp[s * W + w] = e;
             }
         }
@@ -961,11 +962,11 @@ __global__ __launch_bounds__(WAVE) void k_fast64_allr(FastArgs A)
     for (int i = 0; i < DM; ++i) {
         if (i < d) {
             A.x64[(int64_t)i * W + w] = x[i];
-            if (FULL && HX2 && A.s_x2) { A.s_x2[(int64_t)i * W + w] = sm[i]; }
+            if (TS && HX2 && A.s_x2) { A.s_x2[(int64_t)i * W + w] = sm[i]; }
         }
     }
-    if (FULL && HSUM && A.s_x2sum) { A.s_x2sum[w] = Sr; }
-    if (FULL && HEXP && A.s_exp) { A.s_exp[w] = Se; }
+    if (TS && HSUM && A.s_x2sum) { A.s_x2sum[w] = Sr; }
+    if (TS && HEXP && A.s_exp) { A.s_exp[w] = Se; }
     A.acc[w] = nacc;
     A.rej[w] = A.nsteps - nacc;
 }
@@ -1336,12 +1337,19 @@ template <int FL>
 void launch_all(dim3 grid, size_t sh, hipStream_t s, const FastArgs &A)
 {
     if constexpr ((FL & F_MT) == 0) {
-        if (A.ndim == ALL_DM) {
-            hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, true>), grid, dim3(WAVE), 0, s, A);
-            return;
-        }
-        if (A.ndim < ALL_DM) {
-            hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, false>), grid, dim3(WAVE), 0, s, A);
+        auto go = [&](auto sums) {
+            constexpr bool TS = decltype(sums)::value;
+            if (A.ndim == ALL_DM) { hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, true, TS>), grid, dim3(WAVE), 0, s, A); }
+            else { hipLaunchKernelGGL((k_fast64_allr<FL, ALL_DM, false, TS>), grid, dim3(WAVE), 0, s, A); }
+        };
+        if (A.ndim <= ALL_DM) {
+            if constexpr ((FL & F_FULL) != 0) {
+                if (A.s_x2 || A.s_x2sum || A.s_exp) {
+                    go(std::true_type{});
+                    return;
+                }
+            }
+            go(std::false_type{});
             return;
         }
     }
@@ -1564,7 +1572,12 @@ bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
 {
     int L, S;
     const bool mt = rng == MCI_RNG_MT19937_64;
-    if (movetype == MCI_MOVE_ALL) { return group_shape(mt, ndim, W, L, S) || (!mt && ndim <= ALL_DM); }
+    if (movetype == MCI_MOVE_ALL) {
+        // one lane a walker: up to one wave a SIMD.  Beyond, the waves that its registers cost are worth more than
+        // the pass that the sums save: 262,144 walkers x 256 steps, X2 traces, d = 3, sampling + estimation
+        // 0.56 + 0.86 ms without, 1.03 + 0.54 with; d = 1 0.49 + 0.32 and 0.93 + 0.20
+        return group_shape(mt, ndim, W, L, S) || (!mt && ndim <= ALL_DM && W <= 65536);
+    }
     return mt && group_slots_vec(ndim, W, S);
 }
 

@@ -150,3 +150,18 @@ def test_a_lane_of_eighteen_slots_keeps_them_in_registers():
         took.append(phase(c, 2, 4))
     print("took", took, flush=True)
     assert took[1] < 2 * took[0], took
+
+
+def test_traces_of_more_walkers_than_lanes_keep_two_waves_a_simd():
+    """the sums that MJBlocker's mean would take are not kept where their registers would cost a wave: four waves a
+    SIMD sample in less than 3.2 times one wave's time (2.1 measured; 3.9 with the sums)"""
+    took = []
+    for W in (65536, 262144):
+        print("traces", W, flush=True)
+        c = chain_setup("mci", dict(ndim=1, seed=4, ndecorr=20, move=(0, 0, 1, None), pdfs=[(PDF_GAUSS_DIAG, np.full(1, 0.5))],
+                                    obs=[(OBS_X2, [], 1, 1, 0, ESTIM_MJ)]), nwalkers=W)
+        c.setRng(RNG_PHILOX)
+        c.setCoupling(1)
+        took.append(phase(c, 2, 5))
+    print("took", took, flush=True)
+    assert took[1] < 3.2 * took[0], took

@@ -340,6 +340,8 @@ int rtc_kinds(const mci_ctx *c)
     std::memset(&ch, 0, sizeof ch);
     ch.ndim = c->ndim;
     ch.W = c->W;
+    ch.rng = c->rng;
+    ch.srrd = c->srrd;
     ch.nproto = nproto_total(c);
     int kinds = 1 << state_lds_of(ch, false).kind;
     ch.nobs = (int)c->obs.size();

@@ -1185,6 +1185,7 @@ hipError_t launch_sample(const Chain &c, int64_t nsteps, int acc, const uint8_t 
     const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
     switch (st.kind) {
     case STATE_LDS: hipLaunchKernelGGL(k_sample<STATE_LDS>, g, b, st.bytes, s, c, nsteps, acc, active, skip); break;
+    case STATE_LDS_TWO: hipLaunchKernelGGL(k_sample<STATE_LDS_TWO>, g, b, st.bytes, s, c, nsteps, acc, active, skip); break;
     case STATE_HBM_TWO: hipLaunchKernelGGL(k_sample<STATE_HBM_TWO>, g, b, 0, s, c, nsteps, acc, active, skip); break;
     default: hipLaunchKernelGGL(k_sample<STATE_HBM>, g, b, 0, s, c, nsteps, acc, active, skip);
     }
@@ -1197,6 +1198,7 @@ hipError_t launch_calibrate_indep(const Chain &c, int nfind, double target, int6
     const dim3 g = grid1(c.W, STATE_WAVE), b(STATE_WAVE);
     switch (st.kind) {
     case STATE_LDS: hipLaunchKernelGGL(k_calibrate_indep<STATE_LDS>, g, b, st.bytes, s, c, nfind, target, min_stat, dimSizes); break;
+    case STATE_LDS_TWO: hipLaunchKernelGGL(k_calibrate_indep<STATE_LDS_TWO>, g, b, st.bytes, s, c, nfind, target, min_stat, dimSizes); break;
     case STATE_HBM_TWO: hipLaunchKernelGGL(k_calibrate_indep<STATE_HBM_TWO>, g, b, 0, s, c, nfind, target, min_stat, dimSizes); break;
     default: hipLaunchKernelGGL(k_calibrate_indep<STATE_HBM>, g, b, 0, s, c, nfind, target, min_stat, dimSizes);
     }
@@ -1206,7 +1208,10 @@ hipError_t launch_calibrate_indep(const Chain &c, int nfind, double target, int6
 StateLds state_lds_of(const Chain &c, bool observables)
 {
     const size_t n = state_lds(c, observables ? chain_nobsdim(c) : 0);
-    if (n <= STATE_LDS_MAX) { return StateLds{n, STATE_LDS}; }
+    if (n <= STATE_LDS_MAX) {
+        const bool two = c.W > STATE_TWO && n <= STATE_LDS_TWO_MAX && c.srrd != MCI_SRRD_UNIFORM && c.rng == MCI_RNG_PHILOX;
+        return StateLds{n, two ? STATE_LDS_TWO : STATE_LDS};
+    }
     return StateLds{0, c.W > STATE_TWO ? STATE_HBM_TWO : STATE_HBM};
 }
 

@@ -45,9 +45,9 @@ struct EstimJob
     const double *sum = nullptr;
 };
 
-// where a generic step kernel keeps the walkers' state: HBM, the wave's LDS, or HBM with the registers for
-// two waves a SIMD
-enum StateKind { STATE_HBM, STATE_LDS, STATE_HBM_TWO, STATE_KINDS };
+// where a generic step kernel keeps the walkers' state: HBM or the wave's LDS; and either with the registers
+// for two waves a SIMD
+enum StateKind { STATE_HBM, STATE_LDS, STATE_HBM_TWO, STATE_LDS_TWO, STATE_KINDS };
 
 #ifndef MCI_RTC_USER // the host's launch interface (not part of the run-time build of the step kernels)
 hipError_t launch_seed_mt(uint64_t *mt, int32_t *mtp, const uint64_t *seeds, int64_t W, hipStream_t s);

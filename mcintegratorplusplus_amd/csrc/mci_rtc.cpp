@@ -35,7 +35,8 @@ std::map<std::pair<std::string, int>, Loaded> g_cache;
 // by StateKind
 const char *const kNames[STATE_KINDS][2] = {{"mcid::k_sample<0>", "mcid::k_calibrate_indep<0>"},
                                             {"mcid::k_sample<1>", "mcid::k_calibrate_indep<1>"},
-                                            {"mcid::k_sample<2>", "mcid::k_calibrate_indep<2>"}};
+                                            {"mcid::k_sample<2>", "mcid::k_calibrate_indep<2>"},
+                                            {"mcid::k_sample<3>", "mcid::k_calibrate_indep<3>"}};
 
 // compiles text's kernels of one kind; on success code holds the code object and names their lowered names
 int compile(const std::string &text, const std::string &arch, int kind, std::vector<char> &code, std::string (&names)[2], std::string &log)

@@ -24,9 +24,13 @@ constexpr size_t STATE_LDS_MAX = 80 * 1024;  // two waves a CU: beyond that the 
 // Waves a SIMD that a kind's registers leave room for.  In HBM a step waits for its accesses, so waves in
 // flight count where there are more than one a SIMD (STATE_TWO walkers); the registers that the second one
 // needs spill, which costs up to an eighth with fewer.  A call with 128 steps in 39 / 60 dimensions, one wave /
-// two, ms: exp(-|x|), single-coordinate moves, 262,144 walkers 66.0 / 54.6, 65,536 29.2 / 32.8 (d 60).
+// two, ms: exp(-|x|), single-coordinate moves, 262,144 walkers 66.0 / 54.6, 65,536 29.2 / 32.8 (d 60).  In LDS it
+// pays only for the long draws of the other distributions on the native streams (64 steps, d 4, 262,144 walkers:
+// Student 78.1 / 61.2, gamma 66.1 / 51.6; the reference streams' Student 216 / 225, uniform moves 7.3 / 11.0).
 constexpr int64_t STATE_TWO = 65536;
-inline __host__ __device__ constexpr int state_waves(int kind) { return kind == STATE_HBM_TWO ? 2 : 1; }
+constexpr size_t STATE_LDS_TWO_MAX = 20 * 1024;  // eight waves a CU
+inline __host__ __device__ constexpr int state_waves(int kind) { return kind == STATE_HBM_TWO || kind == STATE_LDS_TWO ? 2 : 1; }
+inline __host__ __device__ constexpr bool state_in_lds(int kind) { return kind == STATE_LDS || kind == STATE_LDS_TWO; }
 inline __host__ __device__ int state_rows(const Chain &c, int nobsdim) { return 2 * c.ndim + 2 * c.nproto + 2 * nobsdim; }
 inline __host__ __device__ size_t state_lds(const Chain &c, int nobsdim)
 {
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(STATE_WAVE, state_waves(KIND)) void k_sample(Chain 
     if (w >= c.W) { return; }
     if (skip && skip->done) { return; }
     if (active && !active[w]) { return; }
-    sample_walker<KIND == STATE_LDS>(c, nsteps, accumulate_obs, w, state_sh);
+    sample_walker<state_in_lds(KIND)>(c, nsteps, accumulate_obs, w, state_sh);
 }
 
 // step clamps of findMRT2Step (MCIntegrator.cpp:147-161)
@@ -190,6 +194,6 @@ __global__ __launch_bounds__(STATE_WAVE, state_waves(KIND)) void k_calibrate_ind
     extern __shared__ double state_sh[];
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= c.W) { return; }
-    calibrate_walker<KIND == STATE_LDS>(c, nfind, target, min_stat, dimSizes, w, state_sh);
+    calibrate_walker<state_in_lds(KIND)>(c, nfind, target, min_stat, dimSizes, w, state_sh);
 }
 } // namespace mcid

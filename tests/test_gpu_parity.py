@@ -789,3 +789,24 @@ def test_moves_of_other_distributions_cost_their_draws():
             t.append(time.perf_counter() - t0)
         took.append(min(t[1:]))
     assert took[1] < 15 * took[0], took
+
+
+def test_long_draws_of_many_walkers_overlap():
+    """gamma moves of four waves a SIMD on the native streams: two run at a time, so that they take less than 3.5 times
+    one wave's call (3.1 measured; 3.9 one after the other)"""
+    import time
+    took = []
+    for W in (65536, 262144):
+        c = chain_setup("mci", dict(ndim=4, seed=3, ndecorr=100, move=(5, 0, 1, None), pdfs=[(PDF_EXP_DIAG, np.full(4, 1.0))],
+                                    obs=[(OBS_X2, [], 16, 1, 0, ESTIM_MJ)]), nwalkers=W)
+        c.setRng(RNG_PHILOX)
+        c.setCoupling(1)
+        t = []
+        for _ in range(4):
+            print("gamma moves", W, flush=True)
+            t0 = time.perf_counter()
+            c.integrate(64)
+            t.append(time.perf_counter() - t0)
+        took.append(min(t[1:]))
+        print("took", took[-1], flush=True)
+    assert took[1] < 3.5 * took[0], took

@@ -397,13 +397,13 @@ hipError_t calibrate_indep_launch(const mci_ctx *c, const Chain &ch, int nfind, 
     return launch_calibrate_indep(ch, nfind, target, min_stat, dimSizes, s);
 }
 
-// Before a specialised launch in which every walker takes nsteps steps (sums: with observables): if the
+// Before a specialised launch in which every walker takes nsteps steps with these observables: if the
 // walkers' generator next indices may differ, and the launch does not see to it itself, rotate each state to next index 0 (the same generator), so that every state access
 // of a wave is one row instead of a gather over 64 rows.
-mci_status mt_align_if_needed(mci_ctx *c, int64_t nsteps, bool sums)
+mci_status mt_align_if_needed(mci_ctx *c, int64_t nsteps, const std::vector<ObsDev> &obs = {})
 {
     if (c->rng != MCI_RNG_MT19937_64 || !c->mt_diverged) { return MCI_OK; }
-    if (!fast_rotates_mt(c->movetype, c->ndim, c->W, nsteps, sums)) { HIPCHK(launch_mt_align(c->mt.p, c->mtp.p, c->W, c->stream)); }
+    if (!fast_rotates_mt(c->movetype, c->ndim, c->W, nsteps, obs.data(), (int)obs.size())) { HIPCHK(launch_mt_align(c->mt.p, c->mtp.p, c->W, c->stream)); }
     c->mt_diverged = false;
     return MCI_OK;
 }
@@ -463,7 +463,7 @@ mci_status find_shared(mci_ctx *c)
     std::memset(&init, 0, sizeof init);
     HIPCHK(hipMemcpyAsync(c->ctrl.p, &init, sizeof init, hipMemcpyHostToDevice, c->stream));
     const bool fast = fast_chain(c);
-    if (fast) { TRY(mt_align_if_needed(c, min_stat, false)); }
+    if (fast) { TRY(mt_align_if_needed(c, min_stat)); }
     const int maxit = std::abs(N);
     // the first batch is as long as the last calibration of this context took (iterations after
     // the exit are no-ops, so the batch length changes the time, never the result)
@@ -563,7 +563,7 @@ mci_status find_indep_fast(mci_ctx *c, int64_t min_stat)
     HIPCHK(hipMemsetAsync(c->cal_cons.p, 0, sizeof(int32_t) * W, c->stream));
     HIPCHK(hipMemsetAsync(c->cal_count.p, 0, sizeof(int32_t) * W, c->stream));
     HIPCHK(hipMemsetAsync(c->cal_any.p, 0, sizeof(int32_t) * maxit, c->stream));
-    TRY(mt_align_if_needed(c, min_stat, false));
+    TRY(mt_align_if_needed(c, min_stat));
     Chain ch = make_chain(c, nullptr), dense;
     TRY(dense_chain(c, ch, dense));
     int batch = (c->calib_indep_hint > 0) ? c->calib_indep_hint : 4;
@@ -668,7 +668,7 @@ mci_status decorrelate_auto(mci_ctx *c)
     // traces in the dense columns, which the estimators map back to the walkers)
     Chain dense;
     if (fast_dec) {
-        TRY(mt_align_if_needed(c, min_nmc, !od.empty()));
+        TRY(mt_align_if_needed(c, min_nmc, od));
         if (!shared) { TRY(dense_chain(c, ch, dense)); }
     }
     bool compacted = false;
@@ -1690,7 +1690,7 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
         }
     }
     // the estimators that need a trace's mean first take its sum from the sampling launch
-    if (fast_main && c->obsfile.empty() && c->wlkfile.empty() && fast_sums_traces(c->movetype, c->rng, c->ndim, W)) {
+    if (fast_main && c->obsfile.empty() && c->wlkfile.empty() && fast_sums_traces(c->movetype, c->rng, c->ndim, W, nmc, od.data(), (int)od.size())) {
         for (size_t i = 0; i < od.size(); ++i) {
             if (od[i].acc != ACC_FULL || !needs_scratch(c->obs[i].estim, od[i].nstore)) { continue; }
             HIPCHK(c->tracesum[i].ensure((size_t)od[i].nobs * W));
@@ -1727,7 +1727,7 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
     if (!c->pdfs.empty() && do_decorr) {
         if (c->ndecorr > 0) {
             if (fast) {
-                TRY(mt_align_if_needed(c, c->ndecorr, false));
+                TRY(mt_align_if_needed(c, c->ndecorr));
                 TRY(fast_sample(c->fast, make_chain(c, nullptr), c->prec, c->ndecorr, nullptr, 0, c->stream));
             }
             else { HIPCHK(sample_launch(c, make_chain(c, nullptr), c->ndecorr, 0, nullptr, c->stream)); }
@@ -1755,7 +1755,7 @@ mci_status integrate_phases(mci_ctx *c, int64_t nmc, double *average, double *er
         ch.rec_fx = c->wlkfreq;
     }
     if (fast_main) {
-        TRY(mt_align_if_needed(c, nmc, !od.empty()));
+        TRY(mt_align_if_needed(c, nmc, od));
         TRY(fast_sample(c->fast, ch, c->prec, nmc, od.data(), (int)od.size(), c->stream));
     }
     else { HIPCHK(sample_launch(c, ch, nmc, 1, nullptr, c->stream)); }

@@ -1501,7 +1501,7 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
         if (prec != MCI_PREC_FP64 || (c.nvecs & (c.nvecs - 1)) != 0 || !c.mt || !c.mtp) { return MCI_E_INVALID_ARGUMENT; }
         fl |= F_MT;
         int S = 0;
-        if (group_slots_vec(c.ndim, c.W, S) && ((fl & 7) != 0 || group_vec_plain(c.ndim, c.W, nsteps))) {
+        if (group_slots_vec(c.ndim, c.W, S) && group_vec(c.ndim, c.W, nsteps, fl & 7)) {
             if (!launch_group(fl, true, 4, S, A, s)) { return MCI_E_INVALID_ARGUMENT; }
             return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
         }
@@ -1568,7 +1568,15 @@ int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const O
     return hipGetLastError() == hipSuccess ? MCI_OK : MCI_E_DEVICE;
 }
 
-bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
+// the F_* bits of a launch's observables
+static int fast_obs_bits(const ObsDev *obs, int nobs)
+{
+    int b = 0;
+    for (int i = 0; i < nobs; ++i) { b |= obs[i].kind == MCI_OBS_X2 ? F_X2 : obs[i].kind == MCI_OBS_X2_SUM ? F_SUM : F_EXP; }
+    return b;
+}
+
+bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W, int64_t nsteps, const ObsDev *obs, int nobs)
 {
     int L, S;
     const bool mt = rng == MCI_RNG_MT19937_64;
@@ -1578,14 +1586,14 @@ bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W)
         // 0.56 + 0.86 ms without, 1.03 + 0.54 with; d = 1 0.49 + 0.32 and 0.93 + 0.20
         return group_shape(mt, ndim, W, L, S) || (!mt && ndim <= ALL_DM && W <= 65536);
     }
-    return mt && group_slots_vec(ndim, W, S);
+    return mt && group_slots_vec(ndim, W, S) && group_vec(ndim, W, nsteps, fast_obs_bits(obs, nobs));
 }
 
-bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, bool sums)
+bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, const ObsDev *obs, int nobs)
 {
     int L, S;
     if (movetype == MCI_MOVE_ALL) { return group_shape(true, ndim, W, L, S); }
-    return group_slots_vec(ndim, W, S) && (sums || group_vec_plain(ndim, W, nsteps));
+    return group_slots_vec(ndim, W, S) && group_vec(ndim, W, nsteps, fast_obs_bits(obs, nobs));
 }
 
 void fast_release(FastState &fs) { (void)fs; }

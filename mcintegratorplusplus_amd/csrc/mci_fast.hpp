@@ -28,10 +28,10 @@ struct CalibCtrl;
 int fast_sample(FastState &fs, const Chain &c, int prec, int64_t nsteps, const ObsDev *obs, int nobs, hipStream_t s,
                 const CalibCtrl *pend = nullptr, const double *dimsizes = nullptr, const uint8_t *active = nullptr,
                 const int32_t *wmap = nullptr, const int32_t *wcount = nullptr);
-// the launches of these moves also write the sums of Full traces (ObsDev::sum)
-bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W);
-// a launch of nsteps steps of these moves (sums: with observables) starts from whatever next indices the
+// a launch of nsteps steps of these moves also writes the sums of its Full traces (ObsDev::sum)
+bool fast_sums_traces(int movetype, int rng, int ndim, int64_t W, int64_t nsteps, const ObsDev *obs, int nobs);
+// a launch of nsteps steps of these moves with these observables starts from whatever next indices the
 // walkers' mt19937_64 states stand at (and leaves them all at one), so the states need no realignment before it
-bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, bool sums);
+bool fast_rotates_mt(int movetype, int ndim, int64_t W, int64_t nsteps, const ObsDev *obs, int nobs);
 void fast_release(FastState &fs);
 } // namespace mcid

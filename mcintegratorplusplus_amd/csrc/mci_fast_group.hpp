@@ -72,18 +72,26 @@ inline bool group_slots_vec(int d, int64_t W, int &S)
     return d <= 64 && (d & (d - 1)) == 0 && W * (int64_t)d < (int64_t)1 << 29;
 }
 
-// Whether such a launch of nsteps steps that sums nothing (calibration, decorrelation) runs on groups of
-// lanes.  One lane a walker then has little to do in LDS, and moves 72 bytes of generator state a step at up to
-// 5.4 TB/s; a group reads and writes the whole state once and issues its selects over S slots on four times as
-// many waves.  ms of one launch, one lane / group, 100, 1,000 steps:
+// Whether such a launch of nsteps steps runs on groups of lanes; obs: the observables it sums or stores (the
+// F_X2, F_SUM and F_EXP bits).  One lane a walker moves 72 bytes of generator state a step at up to 5.4 TB/s, and
+// with x_i^2 a record of LDS for every coordinate; a group reads and writes the whole state once and issues
+// its selects, and the ordered sum of sums and exponentials, on four times as many waves.
+// ms of one launch, one lane / group:
+//  without observables, 100 and 1,000 steps
 //   16,384 walkers d 16 0.062 / 0.051, 0.54 / 0.26; d 64 0.066 / 0.073, 0.54 / 0.44
 //   32,768 walkers d 16 0.065 / 0.064, 0.57 / 0.35; d 32 0.067 / 0.074, 0.57 / 0.45; d 64 0.071 / 0.132, 0.58 / 0.85
 //   65,536 walkers d 16 0.081 / 0.120, 0.70 / 0.68; d 32 0.083 / 0.137, 0.70 / 0.85; d 64 0.088 / 0.250, 0.70 / 1.65
-inline bool group_vec_plain(int d, int64_t W, int64_t nsteps)
+//  with x_i^2, sampling and estimation of traces at 65,536 walkers, 64 and 256 steps, one lane takes 0.7 to 0.9 and
+//   1.0 to 1.4 times a group's time at d 1 to 64
+//  |x|^2 alone, blocks of 16, 65,536 walkers, 1,024 steps: d 1 0.72 / 0.65, d 32 1.01 / 1.75, d 64 1.37 / 2.58;
+//   exp(-|x|^2 / d) alone one lane takes 0.78 to 0.47 times a group's time
+inline bool group_vec(int d, int64_t W, int64_t nsteps, int obs)
 {
+    constexpr int X2 = 1, EXP = 4;
     if (W <= 16384) { return true; }
-    if (W <= 32768) { return d <= 32; }
-    return d <= 16 && nsteps >= 512;
+    if (obs & X2) { return nsteps >= 128; }
+    if (W <= 32768) { return d <= 16 || (d <= 32 && nsteps >= 512); }
+    return nsteps >= 512 && !(obs & EXP) && d <= (obs ? 8 : 16);
 }
 
 // one launch of kernel form fl (the F_* flags of mci_fast_dev.hpp, without F_P2; vec: single-coordinate

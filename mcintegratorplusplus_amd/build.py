@@ -59,10 +59,10 @@ FLAGS = ["-std=c++17", "-O3", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=
          "-fhip-fp32-correctly-rounded-divide-sqrt",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument"]
-# the learned move keeps the last layer's 128 outputs per lane across phases: matrix-core results in
-# ordinary VGPRs, so that they are not held twice (accumulation registers and VGPRs)
 # sources compiled in several parts at once, each with its number in a macro
 PARTS = {"mci_fast_group.hip": ("GROUP_PART", 7)}
+# the learned move keeps the last layer's 128 outputs per lane across phases: matrix-core results in
+# ordinary VGPRs, so that they are not held twice (accumulation registers and VGPRs)
 EXTRA = {"mci_lp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

@@ -37,9 +37,9 @@ namespace mcid
 namespace
 {
 // FP64 chain.  One wave runs alone on its SIMD at the benchmark size (65,536 walkers =
-// 1,024 waves), so a step costs about 4 cycles per instruction of any kind and 16 per
-// v_mad_u64_u32 (quarter rate; a Philox call holds 20 of them).  The step is written to issue few
-// instructions:
+// 1,024 waves): an instruction of any kind takes it about 4 cycles and a v_mad_u64_u32 8 (a Philox call
+// holds 20 of them), about three quarters of a step's 378; the rest is waiting for LDS and for results.  The
+// step is written to issue few instructions:
 //  - steps go in pairs, as the native stream does: one Philox block holds the shared word
 //    (index bits, then the acceptance uniform's top bits) and the proposal word of two
 //    consecutive steps, so a pair body reads both steps' coordinates from LDS at once, computes
